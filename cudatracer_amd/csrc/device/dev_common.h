@@ -66,7 +66,8 @@ struct DevScene {
     int sky_enabled;
     int sky_tex;            // -1: the constant sky colour
     float sky_r, sky_g, sky_b;
-    uint32_t plane_flags;   // kPlaneNegZero | kPlaneNaN | kEmptyEntry | kCompactBad over the quad tree
+    uint32_t root2;         // the binary root's traversal item (item2 in device/traverse.h)
+    uint32_t plane_flags;   // kPlaneNegZero | kPlaneNaN | kCompactBad over the quad tree
 };
 
 // A primitive's shading record (sh_prim), indexed by primitive id: what
@@ -81,7 +82,6 @@ constexpr int kPrimRows = 8;
 // Properties of the quad tree's box planes, found at upload (k_plane_flags).
 constexpr uint32_t kPlaneNegZero = 1u;  // some plane is -0.0
 constexpr uint32_t kPlaneNaN = 2u;      // some plane is NaN
-constexpr uint32_t kEmptyEntry = 4u;    // some empty slot (count 0) has a child other than 0xFFFFFFFF
 constexpr uint32_t kCompactBad = 8u;    // some node's boxes have no compact encoding (not finite, or too large)
 
 // One camera view (plain frame, batch member or served request).

@@ -111,9 +111,10 @@ CT_DEV void extend_impl(const DevScene& sc, const TraceOpts& to, const Queues& q
     TravCount tc{0u, 0u, 0u, 0u};
     trace_persistent<ACCEL, kClosest, false>(
         sc, to.teps, n, 0u, cnt_fetch_ext(q.counters, bounce), st, tc, q.err,
-        [&](uint32_t i, bool) {
-            const float4 o4 = ro[i], d4 = rd[i];
-            return RayIn{xyz(o4), xyz(d4), 1e34f};
+        [&](uint32_t i, bool, f3& o, f3& d, float& t) {
+            o = xyz(ro[i]);
+            d = xyz(rd[i]);
+            t = 1e34f;
         },
         [&](uint32_t i, bool, float t, int prim) {
             if (prim == -2) { t = 1e34f; prim = -1; }
@@ -174,9 +175,11 @@ CT_DEV void trace_impl(const DevScene& sc, const TraceOpts& to, const Queues& q,
     const float4* __restrict__ sd = q.sh_d[sb & 1];
     trace_persistent<ACCEL, kDual, COUNT>(
         sc, to.teps, n, n2, cnt_fetch_ext(q.counters, bounce), st, tc, q.err,
-        [&](uint32_t i, bool any) {
-            const float4 o4 = any ? so[i] : ro[i], d4 = any ? sd[i] : rd[i];
-            return RayIn{xyz(o4), xyz(d4), any ? o4.w : 1e34f};
+        [&](uint32_t i, bool any, f3& o, f3& d, float& t) {
+            o = xyz((any ? so : ro)[i]);
+            d = xyz((any ? sd : rd)[i]);
+            t = 1e34f;
+            if (any) t = so[i].w;
         },
         [&](uint32_t i, bool any, float t, int prim) {
             if (!any) {
@@ -794,9 +797,10 @@ CT_DEV void flags_impl(const DevScene& sc, const TraceOpts& to, const Queues& q,
     TravCount tc{0u, 0u, 0u, 0u};
     trace_persistent<ACCEL, kAny, false>(
         sc, to.teps, n, 0u, cnt_fetch_sh(q.counters, 0), st, tc, q.err,
-        [&](uint32_t i, bool) {
-            const float4 o4 = q.sh_o[0][i], d4 = q.sh_d[0][i];
-            return RayIn{xyz(o4), xyz(d4), o4.w};
+        [&](uint32_t i, bool, f3& o, f3& d, float& t) {
+            o = xyz(q.sh_o[0][i]);
+            d = xyz(q.sh_d[0][i]);
+            t = q.sh_o[0][i].w;
         },
         [&](uint32_t i, bool, float, int prim) { out[i] = prim >= 0 ? 1 : 0; });
 }
@@ -840,11 +844,21 @@ int full_of(const LaunchShape& ls, int tree) {
     return tree == 2 ? ls.full2 : (tree == 4 ? ls.full4 : (tree == kTreeCompact ? ls.fullc : ls.full8));
 }
 
+// Blocks of a ray-level launch of n rays: the full persistent grid, or the
+// blocks that give each wave four rays of a small launch (trace_persistent
+// spreads them four lanes a ray; fewer rays a wave diverge less, but every
+// block costs its dispatch), a multiple of the fetch ranges.
+int ray_grid(const LaunchShape& ls, int tree, uint32_t n) {
+    const uint64_t per_block = 4u * (uint64_t)(ls.block / 64);
+    const uint64_t need = ((n + per_block - 1) / per_block + kFetchRanges - 1) / kFetchRanges * kFetchRanges;
+    return (int)std::min<uint64_t>((uint64_t)full_of(ls, tree), std::max<uint64_t>(need, kFetchRanges));
+}
+
 template <int TREE>
 void extend_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, int sel, int bounce,
-              hipStream_t s) {
+              uint32_t n, hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
-    const dim3 grid(full_of(ls, TREE)), block(ls.block);
+    const dim3 grid(ray_grid(ls, TREE, n)), block(ls.block);
     hipLaunchKernelGGL((k_extend<TREE>), grid, block, lds, s, sc, to, q, sel, bounce, ls.lds_depth);
 }
 template <int TREE>
@@ -861,12 +875,12 @@ void trace_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, con
 }
 
 hipError_t launch_extend(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, int sel,
-                         int bounce, hipStream_t s) {
+                         int bounce, uint32_t n, hipStream_t s) {
     switch (tree_of(to)) {
-        case 2: extend_t<2>(ls, sc, to, q, sel, bounce, s); break;
-        case 4: extend_t<4>(ls, sc, to, q, sel, bounce, s); break;
-        case kTreeCompact: extend_t<kTreeCompact>(ls, sc, to, q, sel, bounce, s); break;
-        default: extend_t<8>(ls, sc, to, q, sel, bounce, s); break;
+        case 2: extend_t<2>(ls, sc, to, q, sel, bounce, n, s); break;
+        case 4: extend_t<4>(ls, sc, to, q, sel, bounce, n, s); break;
+        case kTreeCompact: extend_t<kTreeCompact>(ls, sc, to, q, sel, bounce, n, s); break;
+        default: extend_t<8>(ls, sc, to, q, sel, bounce, n, s); break;
     }
     return hipGetLastError();
 }
@@ -1001,10 +1015,9 @@ CT_DEV bool compact_axis(const float lo[4], const float hi[4], uint32_t valid, f
 }
 
 // Per quad node: the fast node test's layout (the six plane rows, the four
-// stack entries kLeafBit | first triangle record or the child node, a zero
-// row), the compact layout of cnode4_step (same entries, kNoEntry for an
-// empty slot) and the tree's kPlaneNegZero / kPlaneNaN / kEmptyEntry /
-// kCompactBad flags (flags cleared by the caller; one atomic per wave that
+// stack entries kLeafBit | first triangle record, the child node or kNoEntry
+// for an empty slot, a zero row), the compact layout of cnode4_step (same
+// entries) and the tree's kPlaneNegZero / kPlaneNaN / kCompactBad flags (flags cleared by the caller; one atomic per wave that
 // found something).
 __global__ void k_prepare_quad(const float4* __restrict__ nodes4, uint32_t n4, float4* __restrict__ fast,
                                uint4* __restrict__ compact, uint32_t* flags) {
@@ -1028,11 +1041,9 @@ __global__ void k_prepare_quad(const float4* __restrict__ nodes4, uint32_t n4, f
                                    __float_as_uint(ch.w)};
         const uint32_t count[4] = {__float_as_uint(cn.x), __float_as_uint(cn.y), __float_as_uint(cn.z),
                                    __float_as_uint(cn.w)};
-        uint32_t e[4], ce[4], valid = 0u;
+        uint32_t e[4], valid = 0u;
         for (int k = 0; k < 4; ++k) {
-            e[k] = count[k] == 0xFFFFFFFFu ? child[k] : (ctd::kLeafBit | child[k]);
-            if (count[k] == 0u && child[k] != 0xFFFFFFFFu) f |= ctd::kEmptyEntry;
-            ce[k] = count[k] == 0u ? ctd::kNoEntry : e[k];
+            e[k] = count[k] == 0u ? ctd::kNoEntry : (count[k] == 0xFFFFFFFFu ? child[k] : (ctd::kLeafBit | child[k]));
             if (count[k] != 0u) valid |= 1u << k;
         }
         o[6] = make_float4(__uint_as_float(e[0]), __uint_as_float(e[1]), __uint_as_float(e[2]), __uint_as_float(e[3]));
@@ -1046,10 +1057,10 @@ __global__ void k_prepare_quad(const float4* __restrict__ nodes4, uint32_t n4, f
                           kb[0] | (kb[1] << 8) | (kb[2] << 16));
         w[1] = make_uint4(wl[0], wh[0], wl[1], wh[1]);
         w[2] = make_uint4(wl[2], wh[2], 0u, 0u);
-        w[3] = make_uint4(ce[0], ce[1], ce[2], ce[3]);
+        w[3] = make_uint4(e[0], e[1], e[2], e[3]);
     }
     uint32_t w = 0;
-    for (uint32_t bit : {ctd::kPlaneNegZero, ctd::kPlaneNaN, ctd::kEmptyEntry, ctd::kCompactBad})
+    for (uint32_t bit : {ctd::kPlaneNegZero, ctd::kPlaneNaN, ctd::kCompactBad})
         if (__ballot(f & bit)) w |= bit;
     if (__lane_id() == 0 && w) atomicOr(flags, w);
 }
@@ -1070,7 +1081,7 @@ hipError_t launch_shadow_flags(const LaunchShape& ls, const DevScene& sc, const 
                                uint32_t n, uint8_t* out, hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
     const int tree = tree_of(to);
-    const dim3 grid(full_of(ls, tree)), block(ls.block);
+    const dim3 grid(ray_grid(ls, tree, n)), block(ls.block);
     if (tree == 2) hipLaunchKernelGGL(k_shadow_flags<2>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
     else if (tree == 4) hipLaunchKernelGGL(k_shadow_flags<4>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
     else if (tree == kTreeCompact)

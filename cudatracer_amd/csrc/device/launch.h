@@ -38,10 +38,10 @@ hipError_t launch_setup(uint32_t* counters, const ctd::ChunkHdr* hdr, hipStream_
 hipError_t launch_setup_rays(uint32_t* counters, uint32_t* err, uint32_t n, hipStream_t s);
 hipError_t launch_generate(const LaunchShape& ls, const ctd::ViewDesc* views, const ctd::Segment* segs,
                            const ctd::ChunkHdr* hdr, uint32_t max_n, const ctd::Queues& q, hipStream_t s);
-// Closest hit for the rays [0, active[bounce]) of q.ray_o/ray_d[sel] into
+// Closest hit for the n rays [0, active[bounce]) of q.ray_o/ray_d[sel] into
 // q.hit (the ray-level entry points).
 hipError_t launch_extend(const LaunchShape& ls, const ctd::DevScene& sc, const ctd::TraceOpts& to,
-                         const ctd::Queues& q, int sel, int bounce, hipStream_t s);
+                         const ctd::Queues& q, int sel, int bounce, uint32_t n, hipStream_t s);
 // The frame loop's traversal of bounce b: closest hit for the extension rays
 // of bounce b and any hit for the shadow rays of bounce b - 1 in one launch
 // (bounce = max_depth: the last bounce's shadow rays).  wstats (may be null)

@@ -12,16 +12,22 @@
 // every lane performs the reference's sequence of pops, node tests, pushes
 // and triangle tests for its own ray):
 //   - persistent waves claim rays for their idle lanes with one atomic once
-//     three quarters of the wave is idle, from queue ranges of their XCD
-//     (see Fetcher);
-//   - one step per loop iteration and lane: either pop + node test, or one
-//     triangle of the current leaf, so long leaves do not stall node lanes;
+//     kRefillIdle of them are idle, from queue ranges of their XCD (see
+//     Fetcher); neither the claim nor the new rays' loads are waited for on
+//     their own;
+//   - one step per loop iteration and lane, a node test or one triangle of
+//     the current leaf, with one memory round trip for both kinds (trav_step);
+//   - once a wave has at most 16 rays and no more come, each ray gets the four
+//     lanes of a quad (trace_quads);
 //   - the per-lane stack lives in LDS, laid out [depth][thread]; pushes are
 //     branch-free stores at the stack top (a store for a culled child is
 //     overwritten by the next one); entries beyond the LDS depth spill to
-//     the block's global region, laid out the same way.  The builder's depth limit (64) bounds the
-//     stack at 97 entries; the stack bound (Queues::max_stack, 128 by
-//     default) guards user-supplied trees.
+//     the block's global region, laid out the same way.  The builder's depth
+//     limit (64) bounds the stack at 97 entries; the stack bound
+//     (Queues::max_stack, 128 by default) guards user-supplied trees.
+// 1,048,576 rays against 524,287 triangles: 0.641 ms per call with two round
+// trips per step, waited-for claims and one lane a ray throughout, 0.511 ms
+// as it is; the 1080p atrium frame 3.87 and 3.50 ms.
 #pragma once
 
 #include "dev_common.h"
@@ -98,39 +104,62 @@ struct LaneStack {
         // LDS read at a clamped offset (always in bounds), buffer read only
         // for spilled entries
         uint32_t v = lds(top < lds_end ? top : lds_end - 4u);
-        if (top >= lds_end) v = __builtin_amdgcn_raw_buffer_load_b32(spill, top - lds_end, 0, 0);
+        if (top >= lds_end) {
+            v = __builtin_amdgcn_raw_buffer_load_b32(spill, top - lds_end, 0, 0);
+            // waited for here, not at the join: every pop would wait for
+            // whatever memory operations are in flight
+            __asm__ volatile("" : "+v"(v));
+        }
         return v;
     }
-    // Push v0..v3 where k0..k3 (in that order).  Every value is stored at the
-    // next free position; a culled one is overwritten by the next store or
-    // left above the new top.  Branch-free when all four positions are in LDS.
-    CT_DEV void push4(uint32_t v0, bool k0, uint32_t v1, bool k1, uint32_t v2, bool k2, uint32_t v3, bool k3) {
+    // Push v0..v3 where k0..k3 (in that order), all but the last of them: that
+    // one would be popped next, so it stays in `next`.  Every value but v3 is
+    // stored at the next free position; a culled one is overwritten by the
+    // next store or left above the new top.  Branch-free when all positions
+    // are in LDS.  False if there is nothing to push.  The bound counts the
+    // kept entry as if it were stored.
+    CT_DEV bool push4(uint32_t v0, bool k0, uint32_t v1, bool k1, uint32_t v2, bool k2, uint32_t v3, bool k3,
+                      uint32_t& next) {
+        if (!(k0 || k1 || k2 || k3)) return false;
         const uint32_t a0 = top, a1 = a0 + (k0 ? stride4 : 0u), a2 = a1 + (k1 ? stride4 : 0u),
                        a3 = a2 + (k2 ? stride4 : 0u);
-        top = a3 + (k3 ? stride4 : 0u);
-        if (a3 < lds_end) {
+        const uint32_t end = a3 + (k3 ? stride4 : 0u);
+        next = k3 ? v3 : (k2 ? v2 : (k1 ? v1 : v0));
+        top = end - stride4;
+        if (a2 < lds_end) {
             lds(a0) = v0;
             lds(a1) = v1;
             lds(a2) = v2;
-            lds(a3) = v3;
         } else {
             put(a0, v0);
             put(a1, v1);
             put(a2, v2);
-            put(a3, v3);
-            if (top >= max_end + stride4) {  // a position at or beyond max_stack was needed
-                overflow = true;
-                top = max_end + 4u * threadIdx.x;
-            }
+        }
+        // a position at or beyond max_stack was needed
+        if (end >= max_end + stride4) overflow = true;
+        return true;
+    }
+    // Push v0..v3 where k0..k3, all of them.
+    CT_DEV void push4_all(uint32_t v0, bool k0, uint32_t v1, bool k1, uint32_t v2, bool k2, uint32_t v3, bool k3) {
+        const uint32_t a0 = top, a1 = a0 + (k0 ? stride4 : 0u), a2 = a1 + (k1 ? stride4 : 0u),
+                       a3 = a2 + (k2 ? stride4 : 0u);
+        top = a3 + (k3 ? stride4 : 0u);
+        put(a0, v0);
+        put(a1, v1);
+        put(a2, v2);
+        put(a3, v3);
+        if (top >= max_end + stride4) {
+            overflow = true;
+            top = max_end + 4u * threadIdx.x;
         }
     }
 };
 
 // Push the hit children of a quad node, sorted by the tagged tmin (nearest
 // popped first) with the reference's 5-comparator network.
-CT_DEV void push_children(uint32_t hm, float m0, float m1, float m2, float m3, uint32_t e0, uint32_t e1,
-                          uint32_t e2, uint32_t e3, LaneStack& st) {
-    if (hm == 0u) return;
+CT_DEV bool push_children(uint32_t hm, float m0, float m1, float m2, float m3, uint32_t e0, uint32_t e1,
+                          uint32_t e2, uint32_t e3, LaneStack& st, uint32_t& next) {
+    if (hm == 0u) return false;
     float s0 = m0, s1 = m1, s2 = m2, s3 = m3, tmp;
     if (s0 > s1) { tmp = s0; s0 = s1; s1 = tmp; }
     if (s2 > s3) { tmp = s2; s2 = s3; s3 = tmp; }
@@ -139,17 +168,19 @@ CT_DEV void push_children(uint32_t hm, float m0, float m1, float m2, float m3, u
     if (s2 > s3) { tmp = s2; s2 = s3; s3 = tmp; }
     auto entry = [&](uint32_t slot) { return slot == 0 ? e0 : (slot == 1 ? e1 : (slot == 2 ? e2 : e3)); };
     const uint32_t q3 = fbits(s3) & 3u, q2 = fbits(s2) & 3u, q1 = fbits(s1) & 3u, q0 = fbits(s0) & 3u;
-    st.push4(entry(q3), (hm >> q3) & 1u, entry(q2), (hm >> q2) & 1u, entry(q1), (hm >> q1) & 1u, entry(q0),
-             (hm >> q0) & 1u);
+    return st.push4(entry(q3), (hm >> q3) & 1u, entry(q2), (hm >> q2) & 1u, entry(q1), (hm >> q1) & 1u, entry(q0),
+                    (hm >> q0) & 1u, next);
 }
 
-// Quad node test (MBVHNode::intersect): four slabs in the reference's float
+// The entry of an empty slot, and of a culled child in the sort.
+constexpr uint32_t kNoEntry = 0xFFFFFFFFu;
+
+// Quad node test (MBVHNode::intersect) on a node's rows in nodes4f: four slabs in the reference's float
 // order, tmin tagged with the slot, the 5-comparator network, then pushes in
 // the order of traverseMBVH and traverseMBVHShadow (sorted position 3 first).
-CT_DEV void node4_step(const float4* __restrict__ nodes4, uint32_t e, f3 o, f3 inv, float t, LaneStack& st) {
-    const float4* n = nodes4 + 8 * (size_t)e;
+CT_DEV bool node4_step(const float4 (&n)[7], f3 o, f3 inv, float t, LaneStack& st, uint32_t& next) {
     const float4 bminx = n[0], bmaxx = n[1], bminy = n[2], bmaxy = n[3], bminz = n[4], bmaxz = n[5];
-    const float4 ch = n[6], cn = n[7];
+    const float4 ent = n[6];
     float m0, m1, m2, m3, x0, x1, x2, x3;
 #define CT_SLAB(MN, MX, lo, hi)                                                 \
     {                                                                           \
@@ -171,17 +202,13 @@ CT_DEV void node4_step(const float4* __restrict__ nodes4, uint32_t e, f3 o, f3 i
     CT_SLAB(m2, x2, z, 2u)
     CT_SLAB(m3, x3, w, 3u)
 #undef CT_SLAB
-    const int c0 = (int)fbits(cn.x), c1 = (int)fbits(cn.y), c2 = (int)fbits(cn.z), c3 = (int)fbits(cn.w);
-    // hit mask on the tagged values; empty slots (count 0) never pushed
-    const uint32_t hm = ((x0 > 0.0f && m0 <= x0 && m0 < t && c0 != 0) ? 1u : 0u) |
-                        ((x1 > 0.0f && m1 <= x1 && m1 < t && c1 != 0) ? 2u : 0u) |
-                        ((x2 > 0.0f && m2 <= x2 && m2 < t && c2 != 0) ? 4u : 0u) |
-                        ((x3 > 0.0f && m3 <= x3 && m3 < t && c3 != 0) ? 8u : 0u);
-    const uint32_t e0 = c0 == -1 ? fbits(ch.x) : (kLeafBit | fbits(ch.x));
-    const uint32_t e1 = c1 == -1 ? fbits(ch.y) : (kLeafBit | fbits(ch.y));
-    const uint32_t e2 = c2 == -1 ? fbits(ch.z) : (kLeafBit | fbits(ch.z));
-    const uint32_t e3 = c3 == -1 ? fbits(ch.w) : (kLeafBit | fbits(ch.w));
-    push_children(hm, m0, m1, m2, m3, e0, e1, e2, e3, st);
+    const uint32_t e0 = fbits(ent.x), e1 = fbits(ent.y), e2 = fbits(ent.z), e3 = fbits(ent.w);
+    // hit mask on the tagged values; empty slots never pushed
+    const uint32_t hm = ((x0 > 0.0f && m0 <= x0 && m0 < t && e0 != kNoEntry) ? 1u : 0u) |
+                        ((x1 > 0.0f && m1 <= x1 && m1 < t && e1 != kNoEntry) ? 2u : 0u) |
+                        ((x2 > 0.0f && m2 <= x2 && m2 < t && e2 != kNoEntry) ? 4u : 0u) |
+                        ((x3 > 0.0f && m3 <= x3 && m3 < t && e3 != kNoEntry) ? 8u : 0u);
+    return push_children(hm, m0, m1, m2, m3, e0, e1, e2, e3, st, next);
 }
 
 // Fast quad node test: the same tagged entry distances, hit flags and push
@@ -208,24 +235,19 @@ CT_DEV void node4_step(const float4* __restrict__ nodes4, uint32_t e, f3 o, f3 i
 //    swaps: after (0,2) and (1,3), s2 = max(s0, s2) <= max(s1, s3) = s3.  The
 //    entries ride through the first four comparators instead of being looked
 //    up from the sorted keys' slot tags.
-// A culled child in the sort; also the entry of an empty slot, whose child
-// is 0xFFFFFFFF in the builders' trees (kLeafBit | 0xFFFFFFFF), which the
-// upload checks (kEmptyEntry) because the sorted path relies on it.
-constexpr uint32_t kNoEntry = 0xFFFFFFFFu;
-
 CT_DEV bool fast_ray(f3 o, f3 inv, uint32_t plane_flags) {
     constexpr float kMax = 3.40282347e38f;
     const bool inv_ok = fabsf(inv.x) > 0.5f && fabsf(inv.x) <= kMax && fabsf(inv.y) > 0.5f &&
                         fabsf(inv.y) <= kMax && fabsf(inv.z) > 0.5f && fabsf(inv.z) <= kMax;
     const bool o_ok = fabsf(o.x) <= kMax && fabsf(o.y) <= kMax && fabsf(o.z) <= kMax;
     const bool z_ok = !(plane_flags & kPlaneNegZero) || (fbits(o.x) != 0u && fbits(o.y) != 0u && fbits(o.z) != 0u);
-    return !(plane_flags & (kPlaneNaN | kEmptyEntry)) && inv_ok && o_ok && z_ok;
+    return !(plane_flags & kPlaneNaN) && inv_ok && o_ok && z_ok;
 }
 
 // nodes4f: the tree in the fast layout (k_prepare_quad): six plane rows and
 // the four stack entries, seven loads per node.
-CT_DEV void node4_fast(const float4* __restrict__ nodes4f, uint32_t e, f3 o, f3 inv, float t, LaneStack& st) {
-    const float4* n = nodes4f + 8 * (size_t)e;
+CT_DEV bool node4_fast(const float4* __restrict__ nodes4f, uint32_t e, const float4 (&n)[7], f3 o, f3 inv, float t,
+                       LaneStack& st, uint32_t& next) {
     const float4 bminx = n[0], bmaxx = n[1], bminy = n[2], bmaxy = n[3], bminz = n[4], bmaxz = n[5];
     const float4 ent = n[6];
     float m0, m1, m2, m3, x0, x1, x2, x3;
@@ -266,15 +288,15 @@ CT_DEV void node4_fast(const float4* __restrict__ nodes4f, uint32_t e, f3 o, f3 
     m1 = tag(m1, 1u);
     m2 = tag(m2, 2u);
     m3 = tag(m3, 3u);
-    // An empty slot's entry is kNoEntry (its child is 0xFFFFFFFF: no
-    // kEmptyEntry), so the count test is the entry test: the sorted path
-    // carries kNoEntry through the network and never pushes it.
+    // An empty slot's entry is kNoEntry, so the count test is the entry test:
+    // the sorted path carries kNoEntry through the network and never pushes
+    // it.
     const uint32_t e0 = fbits(ent.x), e1 = fbits(ent.y), e2 = fbits(ent.z), e3 = fbits(ent.w);
     const bool h0 = x0 > 0.0f && m0 <= x0 && m0 < t;
     const bool h1 = x1 > 0.0f && m1 <= x1 && m1 < t;
     const bool h2 = x2 > 0.0f && m2 <= x2 && m2 < t;
     const bool h3 = x3 > 0.0f && m3 <= x3 && m3 < t;
-    if (!(h0 || h1 || h2 || h3)) return;
+    if (!(h0 || h1 || h2 || h3)) return false;
     // comparators (0,1) and (2,3) on keys and entries, then (0,2) and (1,3)
     // on entries (their keys are not compared again)
     uint32_t q0 = h0 ? e0 : kNoEntry, q1 = h1 ? e1 : kNoEntry, q2 = h2 ? e2 : kNoEntry, q3 = h3 ? e3 : kNoEntry;
@@ -286,7 +308,7 @@ CT_DEV void node4_fast(const float4* __restrict__ nodes4f, uint32_t e, f3 o, f3 
     q2 = s02 ? ea : ec;
     q1 = s13 ? ed : eb;
     q3 = s13 ? eb : ed;
-    st.push4(q3, q3 != kNoEntry, q2, q2 != kNoEntry, q1, q1 != kNoEntry, q0, q0 != kNoEntry);
+    return st.push4(q3, q3 != kNoEntry, q2, q2 != kNoEntry, q1, q1 != kNoEntry, q0, q0 != kNoEntry, next);
 }
 
 // The compact quad tree (ACCEL kTreeCompact): node i of the quad tree in 16
@@ -318,9 +340,10 @@ CT_DEV bool compact_ray(f3 o, f3 inv) {
            fabsf(o.y) <= kMax && fabsf(o.z) <= kMax;
 }
 
-CT_DEV void cnode4_step(const uint4* __restrict__ cnodes, uint32_t e, f3 o, f3 inv, float t, LaneStack& st) {
-    const uint4* n = cnodes + 4 * (size_t)e;
-    const uint4 h = n[0], qa = n[1], qb = n[2], ent = n[3];
+CT_DEV uint4 ubits4(float4 v) { return make_uint4(fbits(v.x), fbits(v.y), fbits(v.z), fbits(v.w)); }
+
+CT_DEV bool cnode4_step(const float4 (&n)[7], f3 o, f3 inv, float t, LaneStack& st, uint32_t& next) {
+    const uint4 h = ubits4(n[0]), qa = ubits4(n[1]), qb = ubits4(n[2]), ent = ubits4(n[3]);
     const float ax = __uint_as_float((h.w & 0xFFu) << 23) * inv.x;
     const float ay = __uint_as_float(((h.w >> 8) & 0xFFu) << 23) * inv.y;
     const float az = __uint_as_float(((h.w >> 16) & 0xFFu) << 23) * inv.z;
@@ -348,7 +371,7 @@ CT_DEV void cnode4_step(const uint4* __restrict__ cnodes, uint32_t e, f3 o, f3 i
     const bool h1 = x1 > 0.0f && m1 <= x1 && m1 < t;
     const bool h2 = x2 > 0.0f && m2 <= x2 && m2 < t;
     const bool h3 = x3 > 0.0f && m3 <= x3 && m3 < t;
-    if (!(h0 || h1 || h2 || h3)) return;
+    if (!(h0 || h1 || h2 || h3)) return false;
     uint32_t q0 = h0 ? ent.x : kNoEntry, q1 = h1 ? ent.y : kNoEntry, q2 = h2 ? ent.z : kNoEntry,
              q3 = h3 ? ent.w : kNoEntry;
     const bool s01 = m0 > m1, s23 = m2 > m3;
@@ -359,7 +382,7 @@ CT_DEV void cnode4_step(const uint4* __restrict__ cnodes, uint32_t e, f3 o, f3 i
     q2 = s02 ? ea : ec;
     q1 = s13 ? ed : eb;
     q3 = s13 ? eb : ed;
-    st.push4(q3, q3 != kNoEntry, q2, q2 != kNoEntry, q1, q1 != kNoEntry, q0, q0 != kNoEntry);
+    return st.push4(q3, q3 != kNoEntry, q2, q2 != kNoEntry, q1, q1 != kNoEntry, q0, q0 != kNoEntry, next);
 }
 
 // Wide compressed node (128 B, up to 8 children, layout in host/cnode.h).
@@ -369,10 +392,9 @@ CT_DEV void cnode4_step(const uint4* __restrict__ cnodes, uint32_t e, f3 o, f3 i
 // rounding of this form).  The nearest hit child is pushed last (popped
 // first), the others in slot order: a full sort of 8 measured slower.
 // sort = false (any-hit) pushes in slot order.
-CT_DEV void fnode8_step(bool sort, const uint4* __restrict__ fnodes, uint32_t e, f3 o, f3 inv, float t,
-                        LaneStack& st) {
-    const uint4* n = fnodes + 8 * (size_t)e;
-    const uint4 h = n[0], qx = n[1], qy = n[2], qz = n[3], ca = n[4], cb = n[5];
+CT_DEV bool fnode8_step(bool sort, const float4 (&n)[7], f3 o, f3 inv, float t, LaneStack& st, uint32_t& next) {
+    const uint4 h = ubits4(n[0]), qx = ubits4(n[1]), qy = ubits4(n[2]), qz = ubits4(n[3]), ca = ubits4(n[4]),
+                cb = ubits4(n[5]);
     const float sx = __uint_as_float((h.w & 0xFFu) << 23), sy = __uint_as_float(((h.w >> 8) & 0xFFu) << 23),
                 sz = __uint_as_float(((h.w >> 16) & 0xFFu) << 23);
     // the ray in the node's grid: t = q * (s / d) + (p - o) / d
@@ -403,7 +425,7 @@ CT_DEV void fnode8_step(bool sort, const uint4* __restrict__ fnodes, uint32_t e,
         hm |= hit ? (1u << i) : 0u;
         if (hit && mn < best) { best = mn; bslot = (uint32_t)i; }
     }
-    if (hm == 0u) return;
+    if (hm == 0u) return false;
     const uint32_t ent[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
     if (sort) {
         // nearest hit child on top; slot 7 takes the nearest child's place
@@ -419,12 +441,14 @@ CT_DEV void fnode8_step(bool sort, const uint4* __restrict__ fnodes, uint32_t e,
             x[i] = at ? ent[7] : ent[i];
             k[i] = at ? h7 : ((hm >> i) & 1u);
         }
-        st.push4(x[0], k[0], x[1], k[1], x[2], k[2], x[3], k[3]);
-        st.push4(x[4], k[4], x[5], k[5], x[6], k[6], near, true);
-        return;
+        st.push4_all(x[0], k[0], x[1], k[1], x[2], k[2], x[3], k[3]);
+        return st.push4(x[4], k[4], x[5], k[5], x[6], k[6], near, true, next);
     }
-    st.push4(ent[0], hm & 1u, ent[1], (hm >> 1) & 1u, ent[2], (hm >> 2) & 1u, ent[3], (hm >> 3) & 1u);
-    st.push4(ent[4], (hm >> 4) & 1u, ent[5], (hm >> 5) & 1u, ent[6], (hm >> 6) & 1u, ent[7], (hm >> 7) & 1u);
+    st.push4_all(ent[0], hm & 1u, ent[1], (hm >> 1) & 1u, ent[2], (hm >> 2) & 1u, ent[3], (hm >> 3) & 1u);
+    if (st.push4(ent[4], (hm >> 4) & 1u, ent[5], (hm >> 5) & 1u, ent[6], (hm >> 6) & 1u, ent[7], (hm >> 7) & 1u, next))
+        return true;
+    next = st.top_pop();
+    return true;
 }
 
 // BVHNode::Intersect (BVHNode.cuh:50-62): no culling against the current t.
@@ -438,30 +462,38 @@ CT_DEV bool box2(float4 lo, float4 hi, f3 o, f3 inv, float& tmin) {
     return tmax >= 0.0f && tmin < tmax;
 }
 
+// The stack item of a binary node with rows {min, left_first}, {max, count}:
+// the pair of an interior node's children, kLeafBit | first triangle record
+// of a leaf, or kEmptyLeaf (count 0, only in user-supplied trees: pushed like
+// any other, skipped when popped).
+constexpr uint32_t kEmptyLeaf = 0xFFFFFFFEu;
+CT_DEV uint32_t item2(float4 lo, float4 hi) {
+    const int count = (int)fbits(hi.w);
+    return count < 0 ? fbits(lo.w) : (count > 0 ? (kLeafBit | fbits(lo.w)) : kEmptyLeaf);
+}
+
 // Binary interior step (traverseBVH, BVHNode.cuh:107-139): both children
-// tested; if both hit, the strictly nearer is pushed first.
-CT_DEV void node2_step(const float4* __restrict__ nodes2, uint32_t lf, f3 o, f3 inv, LaneStack& st) {
-    const float4 l0 = nodes2[2 * (size_t)lf], l1 = nodes2[2 * (size_t)lf + 1];
-    const float4 r0 = nodes2[2 * (size_t)(lf + 1)], r1 = nodes2[2 * (size_t)(lf + 1) + 1];
+// tested; if both hit, the strictly nearer is pushed first.  n: the rows of
+// the two children, which are adjacent; reading what a child is from its own
+// rows here makes a step one dependent load (fetching the popped node first
+// and then its children was two).
+CT_DEV bool node2_step(const float4 (&n)[7], f3 o, f3 inv, LaneStack& st, uint32_t& next) {
     float n1, n2;
-    const bool hl = box2(l0, l1, o, inv, n1);
-    const bool hr = box2(r0, r1, o, inv, n2);
+    const bool hl = box2(n[0], n[1], o, inv, n1);
+    const bool hr = box2(n[2], n[3], o, inv, n2);
     const bool left_first = !(hl && hr) || (n1 < n2);
-    const uint32_t a = left_first ? lf : lf + 1, b = left_first ? lf + 1 : lf;
+    const uint32_t l = item2(n[0], n[1]), r = item2(n[2], n[3]);
+    const uint32_t a = left_first ? l : r, b = left_first ? r : l;
     const bool ka = left_first ? hl : hr, kb = left_first ? hr : hl;
-    st.push4(a, ka, b, kb, 0u, false, 0u, false);
+    return st.push4(0u, false, 0u, false, a, ka, b, kb, next);
 }
 
 // ----------------------------------------------------------------------
 // Persistent traversal driver.  Source: how ray i is loaded; Sink: what is
 // done with the result.  ACCEL 4 = quad tree, kTreeCompact = the quad tree
 // in the compact layout, 8 = wide compressed tree, 2 = binary tree.
-struct RayIn {
-    f3 o, d;
-    float tmax;
-};
-
-constexpr uint32_t kNoLeaf = 0xFFFFFFFFu;
+// A lane without a ray.
+constexpr uint32_t kDead = 0xFFFFFFFFu;
 
 // What a launch traces: every ray closest-hit (extend, ray-level closest
 // hit), every ray any-hit (ray-level shadow rays), or two queues at once, a
@@ -483,167 +515,470 @@ enum TraceMode { kClosest = 0, kAny = 1, kDual = 2 };
 // as long as the grid has at least kFetchRanges of them, smaller grids move
 // on to the next ranges.
 //
-// A wave claims rays for its idle lanes once kRefillIdle of its 64 lanes are
-// idle (or all, near the end): 4% faster than waiting for the whole wave.
-constexpr uint32_t kRefillIdle = 48;
-
 struct Fetcher {
     uint32_t* base;  // counter of range 0 (range r at base + r * kFetchSlot)
     uint32_t n, n2;  // rays of the first and the second queue
-    int range;
-    bool steal;
+    int range, left;                    // the range, and how many more may be tried
+    uint32_t lo, nfirst, lo2, total;    // its claim space
 
-    // Claim up to `want` indices of a range's claim space: [first, first +
-    // count).  Index v < nfirst is ray lo + v of the first queue, otherwise
-    // ray lo2 + v - nfirst of the second.  Wave-uniform.
-    CT_DEV bool get(uint32_t want, uint32_t& first, uint32_t& count, uint32_t& lo, uint32_t& nfirst,
-                    uint32_t& lo2) {
-        for (int tries = 0; tries < kFetchRanges; ++tries) {
-            lo = (uint32_t)(((uint64_t)n * (uint32_t)range) / kFetchRanges);
-            const uint32_t hi = (uint32_t)(((uint64_t)n * (uint32_t)(range + 1)) / kFetchRanges);
-            lo2 = (uint32_t)(((uint64_t)n2 * (uint32_t)range) / kFetchRanges);
-            const uint32_t hi2 = (uint32_t)(((uint64_t)n2 * (uint32_t)(range + 1)) / kFetchRanges);
-            nfirst = hi - lo;
-            const uint32_t total = nfirst + (hi2 - lo2);
-            uint32_t got = 0;
-            if (lane_id() == 0) got = atomicAdd(base + range * kFetchSlot, want);
-            got = __shfl(got, 0);
-            if (got < total) {
-                first = got;
-                count = min(want, total - got);
-                return true;
-            }
-            if (!steal) return false;
-            range = (range + 1) % kFetchRanges;
-        }
-        return false;
+    // Index v < nfirst of a range's claim space [0, total) is ray lo + v of
+    // the first queue, otherwise ray lo2 + v - nfirst of the second.
+    CT_DEV void open() {
+        lo = (uint32_t)(((uint64_t)n * (uint32_t)range) / kFetchRanges);
+        const uint32_t hi = (uint32_t)(((uint64_t)n * (uint32_t)(range + 1)) / kFetchRanges);
+        lo2 = (uint32_t)(((uint64_t)n2 * (uint32_t)range) / kFetchRanges);
+        const uint32_t hi2 = (uint32_t)(((uint64_t)n2 * (uint32_t)(range + 1)) / kFetchRanges);
+        nfirst = hi - lo;
+        total = nfirst + (hi2 - lo2);
+    }
+    // Claim `want` indices; lane 0's result is the first.
+    CT_DEV uint32_t claim(uint32_t want) const {
+        // Only lane 0's is read (readfirstlane).  The others' is any value,
+        // not an uninitialised one, and not a constant, which would wait for
+        // the previous claim still in flight to this register.
+        uint32_t got;
+        __asm__ volatile("" : "=v"(got));
+        if (lane_id() == 0) got = atomicAdd(base + range * kFetchSlot, want);
+        return got;
+    }
+    // The range is drained: open the next one, false if there is none.
+    CT_DEV bool next() {
+        if (--left < 0) return false;
+        range = (range + 1) % kFetchRanges;
+        open();
+        return true;
     }
 };
 
+// A 16-byte row through a pointer the compiler must know to be global memory
+// (selected from two arrays, it would otherwise take the flat path).
+using gptr = const __attribute__((address_space(1))) char*;
+typedef float row4 __attribute__((ext_vector_type(4)));
+CT_DEV float4 load_row(gptr p) {
+    const row4 v = *(const __attribute__((address_space(1))) row4*)p;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// Node records of each tree: bytes apart, 16-byte rows read.
+template <int ACCEL>
+struct NodeFmt;
+template <>
+struct NodeFmt<4> {
+    static constexpr int kStride = 128, kRows = 7;
+    CT_DEV static const void* base(const DevScene& sc) { return sc.nodes4f; }
+};
+template <>
+struct NodeFmt<2> {
+    static constexpr int kStride = 32, kRows = 4;  // an item is a pair of nodes
+    CT_DEV static const void* base(const DevScene& sc) { return sc.nodes2; }
+};
+template <>
+struct NodeFmt<kTreeCompact> {
+    static constexpr int kStride = 64, kRows = 4;
+    CT_DEV static const void* base(const DevScene& sc) { return sc.cnodes; }
+};
+template <>
+struct NodeFmt<8> {
+    static constexpr int kStride = 128, kRows = 6;
+    CT_DEV static const void* base(const DevScene& sc) { return sc.fnodes; }
+};
+
+// The triangle of leaf item cur with rows a, b, c.  Returns true when an
+// any-hit ray is done; cur becomes the leaf's next triangle, or pop is set.
+CT_DEV bool leaf_step(float4 a, float4 b, float4 c, float eps, f3 o, f3 d, bool any, uint32_t& cur, float& t, int& prim,
+                      bool& pop) {
+    const uint32_t w = fbits(a.w);
+    bool done = false;
+    if (tri_test(o, d, t, xyz(a), xyz(b), xyz(c), eps)) {
+        prim = (int)(w & ~kLastInLeaf);
+        done = any;
+    }
+    pop = (w & kLastInLeaf) != 0u;
+    ++cur;
+    return done;
+}
+
+// One step of a lane's ray: the node test or the triangle test of the item
+// `cur` (a node, or kLeafBit | triangle record), which then becomes the next
+// item.  Returns true when the ray is done: any hit found, stack empty or
+// overflowed.
+//
+// What bounds the loop is the chain of dependent steps of a ray, each a round
+// trip to memory (about 900 cycles) plus the instructions of the tests.  A
+// wave holds lanes at nodes and lanes at triangles; testing the one kind and
+// then the other, each after its own loads, costs a wave two round trips per
+// step.  Here every lane loads the first three rows of whatever its item is
+// from one selected address, and the node lanes' remaining rows follow before
+// anything waits, so a step is one round trip.  The next item stays in a
+// register when it is the nearest child just tested, instead of going through
+// the LDS stack.
+template <int ACCEL, bool COUNT>
+CT_DEV bool trav_step(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool fast, bool any, bool sort, uint32_t& cur,
+                      float& t, int& prim, LaneStack& st, TravCount& cnt, const float4 (&n)[7], int kind) {
+    bool pop = false, done = false;
+    if (kind < 0) {
+        if (COUNT) {
+            if (any) ++cnt.stris;
+            else ++cnt.tris;
+        }
+        done = leaf_step(n[0], n[1], n[2], eps, o, d, any, cur, t, prim, pop);
+    } else {
+        if (COUNT) {
+            const uint32_t boxes = ACCEL == 2 ? 2u : 1u;
+            if (any) cnt.snodes += boxes;
+            else cnt.nodes += boxes;
+        }
+        // any-hit rays visit children nearest first too, like
+        // traverseMBVHShadow (MBVHNode.cuh:165-205): in a two-queue launch
+        // every lane then runs one code path (slot order for any-hit lanes
+        // measured 2% slower)
+        if constexpr (ACCEL == 4) {
+            if (fast) {
+                pop = !node4_fast(sc.nodes4f, (uint32_t)kind, n, o, inv, t, st, cur);
+            } else {
+                // an opaque copy of the origin: the slab values that both
+                // tests compute would otherwise be hoisted above the branch,
+                // 24 registers live through it
+                f3 oo = o;
+                __asm__ volatile("" : "+v"(oo.x), "+v"(oo.y), "+v"(oo.z));
+                pop = !node4_step(n, oo, inv, t, st, cur);
+            }
+        } else if constexpr (ACCEL == kTreeCompact) {
+            if (fast) {
+                pop = !cnode4_step(n, o, inv, t, st, cur);
+            } else {
+                float4 full[7];
+                for (int k = 0; k < 7; ++k) full[k] = sc.nodes4f[8 * (size_t)(uint32_t)kind + k];
+                pop = !node4_step(full, o, inv, t, st, cur);
+            }
+        } else if constexpr (ACCEL == 8) {
+            pop = !fnode8_step(sort, n, o, inv, t, st, cur);
+        } else {
+            pop = !node2_step(n, o, inv, st, cur);
+        }
+    }
+    if (pop) {
+        if (st.empty()) done = true;
+        else cur = st.top_pop();
+    }
+    if constexpr (ACCEL == 2) {
+        while (!done && cur == kEmptyLeaf) {
+            if (st.empty()) done = true;
+            else cur = st.top_pop();
+        }
+    }
+    return done || st.overflow;
+}
+
+// The loads of a step.  kind: the item, opaque to the compiler: otherwise the
+// uses of the item's kind before and after the loads merge, and each kind
+// gets its own loads and its own wait again.
+template <int ACCEL>
+CT_DEV void load_item(const DevScene& sc, uint32_t cur, float4 (&n)[7], int& kind) {
+    using F = NodeFmt<ACCEL>;
+    const bool leaf = (int)cur < 0;
+    const gptr base = leaf ? (gptr)sc.tris : (gptr)F::base(sc);
+    const gptr p = base + (uint64_t)(cur & ~kLeafBit) * (leaf ? 48u : (uint32_t)F::kStride);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) n[k] = load_row(p + 16 * k);
+    kind = (int)cur;
+    __asm__ volatile("" : "+v"(kind));
+    if (!leaf) {
+#pragma unroll
+        for (int k = 3; k < F::kRows; ++k) n[k] = load_row(p + 16 * k);
+    }
+    // One wait for all of them (vmcnt(0)).  Left to the compiler the rows of
+    // whichever kind the wave skips count as in flight around the loop, and
+    // the next step's loads wait for the last step's result stores.
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+}
+
+// The item a ray starts at.
+template <int ACCEL>
+CT_DEV uint32_t root_item(const DevScene& sc) {
+    return ACCEL == 2 ? sc.root2 : 0u;
+}
+
+// ------------------------------------------------------ four lanes a ray --
+// Once a launch's rays are spread so thin that a wave has at most 16 of them
+// (a small launch, or the last rays of a large one), what a ray waits for is
+// its own chain of steps: some 300 instructions of one wave and a round trip
+// to memory each, with most lanes idle.  trace_quads gives each ray the four
+// lanes of a quad instead: lane c tests child c of a node, or triangle c of
+// the next four of a leaf.  The quad makes the steps of the one-lane loop
+// (the same entry distances in the reference's float order, the same
+// comparators, pushes and visit order; the triangles of a leaf in order, the
+// first of equal distances kept), so the results are the same bits.  1,000
+// rays: 120 to 87 us per call; 1,048,576 rays, whose last ones took a third of
+// the launch: 0.597 to 0.511 ms; the textured atrium 6.5 to 5.9 ms.
+template <int CTRL>
+CT_DEV uint32_t quad_dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+CT_DEV float quad_dpp(float v) {
+    return __uint_as_float(quad_dpp<CTRL>(fbits(v)));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;  // quad_perm [1,0,3,2] and [2,3,0,1]
+
+// One comparator of the network on lane pairs: `low` marks the pair's first
+// lane, swaps as the reference does (if the first key is greater).
+template <int CTRL>
+CT_DEV void quad_comparator(bool low, bool on, float& key, uint32_t& e) {
+    const float ok = quad_dpp<CTRL>(key);
+    const uint32_t oe = quad_dpp<CTRL>(e);
+    const bool sw = on && (low ? key > ok : ok > key);
+    key = sw ? ok : key;
+    e = sw ? oe : e;
+}
+
+// The quad whose rays these are (all four lanes hold the same ray; cur ==
+// kDead: none), to their ends.  st.top: the ray's stack, in the column of one
+// of the wave's lanes.  Lane 0 of the quad gives the result to sink.
+template <int ACCEL, class Sink>
+CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool fast, bool any, uint32_t ray,
+                        uint32_t cur, float t, int prim, LaneStack& st, uint32_t* err, Sink sink) {
+    const uint32_t c = lane_id() & 3u, qbase = lane_id() & 60u;
+    while (__ballot(cur != kDead) != 0) {
+        if (cur == kDead) continue;
+        const uint32_t idx = cur & ~kLeafBit;
+        float4 a, b, e;
+        float pl[6];
+        uint32_t ent;
+        uint4 ch, cq;
+        uint2 cz;
+        const bool packed = ACCEL == kTreeCompact && fast;
+        if ((int)cur < 0) {
+            // records past the leaf's end are read (within the array) and ignored
+            const gptr p = (gptr)sc.tris + (uint64_t)min(idx + c, sc.n_tris - 1u) * 48u;
+            a = load_row(p);
+            b = load_row(p + 16);
+            e = load_row(p + 32);
+        } else if (packed) {
+            const uint4* n = sc.cnodes + 4 * (size_t)idx;
+            ch = n[0];
+            cq = n[1];
+            cz = *reinterpret_cast<const uint2*>(n + 2);
+            ent = reinterpret_cast<const uint32_t*>(n + 3)[c];
+        } else {
+            const float* n = reinterpret_cast<const float*>(sc.nodes4f) + 32 * (size_t)idx + c;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) pl[k] = n[4 * k];
+            ent = fbits(n[24]);
+        }
+        int kind = (int)cur;
+        __asm__ volatile("" : "+v"(kind));
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), see load_item
+        bool done = false, pop = false;
+        if (kind < 0) {
+            const uint32_t w = fbits(a.w);
+            const uint32_t last = (uint32_t)(__ballot((w & kLastInLeaf) != 0u) >> qbase) & 15u;
+            float tt = t;
+            const bool hit = tri_test(o, d, tt, xyz(a), xyz(b), xyz(e), eps) && (last & ((1u << c) - 1u)) == 0u;
+            tt = hit ? tt : t;
+            uint32_t pp = hit ? (w & ~kLastInLeaf) : (uint32_t)prim;
+            // the least distance, of equal ones the first triangle's
+            const float t1 = quad_dpp<kQuadXor1>(tt);
+            const uint32_t p1 = quad_dpp<kQuadXor1>(pp);
+            const bool k1 = t1 < tt || (t1 == tt && (c & 1u));
+            tt = k1 ? t1 : tt;
+            pp = k1 ? p1 : pp;
+            const float t2 = quad_dpp<kQuadXor2>(tt);
+            const uint32_t p2 = quad_dpp<kQuadXor2>(pp);
+            const bool k2 = t2 < tt || (t2 == tt && (c & 2u));
+            tt = k2 ? t2 : tt;
+            pp = k2 ? p2 : pp;
+            done = any && tt < t;
+            t = tt;
+            prim = (int)pp;
+            pop = last != 0u;
+            cur += 4u;
+        } else {
+            float mn, mx;
+            if (packed) {
+                const uint32_t sh = 8u * c;
+                const float ax = __uint_as_float((ch.w & 0xFFu) << 23) * inv.x;
+                const float ay = __uint_as_float(((ch.w >> 8) & 0xFFu) << 23) * inv.y;
+                const float az = __uint_as_float(((ch.w >> 16) & 0xFFu) << 23) * inv.z;
+                const float bx = (__uint_as_float(ch.x) - o.x) * inv.x, by = (__uint_as_float(ch.y) - o.y) * inv.y,
+                            bz = (__uint_as_float(ch.z) - o.z) * inv.z;
+                const float lx = fmaf((float)((cq.x >> sh) & 0xFFu), ax, bx), hx = fmaf((float)((cq.y >> sh) & 0xFFu), ax, bx);
+                const float ly = fmaf((float)((cq.z >> sh) & 0xFFu), ay, by), hy = fmaf((float)((cq.w >> sh) & 0xFFu), ay, by);
+                const float lz = fmaf((float)((cz.x >> sh) & 0xFFu), az, bz), hz = fmaf((float)((cz.y >> sh) & 0xFFu), az, bz);
+                mn = fmaxf(fmaxf(fminf(lx, hx), fminf(ly, hy)), fminf(lz, hz));
+                mx = fminf(fminf(fmaxf(lx, hx), fmaxf(ly, hy)), fmaxf(lz, hz));
+            } else {
+                const float ax = (pl[0] - o.x) * inv.x, bx = (pl[1] - o.x) * inv.x;
+                const float ay = (pl[2] - o.y) * inv.y, by = (pl[3] - o.y) * inv.y;
+                const float az = (pl[4] - o.z) * inv.z, bz = (pl[5] - o.z) * inv.z;
+                mn = gmax(gmax(gmin(ax, bx), gmin(ay, by)), gmin(az, bz));
+                mx = gmin(gmin(gmax(ax, bx), gmax(ay, by)), gmax(az, bz));
+            }
+            float key = tag(mn, c);
+            uint32_t x = (mx > 0.0f && key <= mx && key < t) ? ent : kNoEntry;
+            quad_comparator<kQuadXor1>((c & 1u) == 0u, true, key, x);     // (0,1) (2,3)
+            quad_comparator<kQuadXor2>((c & 2u) == 0u, true, key, x);     // (0,2) (1,3)
+            quad_comparator<kQuadXor1>((c & 1u) == 0u, c >= 2u, key, x);  // (2,3)
+            // the lane holds sorted position c: positions 3, 2, 1, 0 are
+            // pushed in this order, the last stays as the next item
+            const uint32_t vm = (uint32_t)(__ballot(x != kNoEntry) >> qbase) & 15u;
+            const uint32_t x0 = quad_dpp<0x00>(x), x1 = quad_dpp<0x55>(x), x2 = quad_dpp<0xAA>(x), x3 = quad_dpp<0xFF>(x);
+            pop = vm == 0u;
+            if (!pop) {
+                const uint32_t n = (uint32_t)__popc(vm);
+                if (x != kNoEntry && (vm & ((1u << c) - 1u)) != 0u) st.put(st.top + st.stride4 * (uint32_t)__popc(vm >> (c + 1u)), x);
+                if (st.top + st.stride4 * n >= st.max_end + st.stride4) st.overflow = true;
+                st.top += st.stride4 * (n - 1u);
+                cur = (vm & 1u) ? x0 : ((vm & 2u) ? x1 : ((vm & 4u) ? x2 : x3));
+            }
+        }
+        if (pop) {
+            if (st.empty()) done = true;
+            else cur = st.top_pop();
+        }
+        if (done || st.overflow) {
+            if (c == 0u) {
+                if (st.overflow) {
+                    atomicOr(err, 1u);
+                    prim = -2;
+                }
+                sink(ray, any, t, prim);
+            }
+            cur = kDead;
+        }
+    }
+}
+
+// Idle lanes of a wave from which it claims new rays.  12, 24, 32, 48 and 56
+// idle lanes: 16 uneven views of the small box on the binary tree 64.3, 64.5,
+// 65.1, 67.6 and 75.5 ms; the atrium frame 3.70, 3.66, 3.67, 3.65 and 3.65,
+// the 7.24M-triangle 4K frame 8.08, 8.00, 8.01, 7.97 and 7.98 ms (spread 1%).
+constexpr uint32_t kRefillIdle = 24;
+
 // n rays of the first queue and, with MODE kDual, n2 any-hit rays of the
-// second.  src(i, any) loads ray i of its queue, sink(i, any, t, prim) takes
-// the result: prim = the hit primitive, -1 none, -2 stack overflow (the
-// error flag is raised and the ray stops).
+// second.  src(i, any, o, d, t) loads ray i of its queue, sink(i, any, t, prim) takes the
+// result: prim = the hit primitive, -1 none, -2 stack overflow (the error
+// flag is raised and the ray stops).
+//
+// A refill costs the wave no wait of its own: the claim's result is read a
+// step later, and the new rays' origins and directions are loaded together
+// with the other lanes' nodes and triangles.
 template <int ACCEL, int MODE, bool COUNT, class Source, class Sink>
 CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t n2, uint32_t* fetch, LaneStack& st,
                              TravCount& cnt, uint32_t* err, Source src, Sink sink) {
-    bool alive = false, exhausted = false, fast = false;
+    bool exhausted = false, fast = false;
     bool any = MODE == kAny;  // the lane's ray is an any-hit query
-    uint32_t ray = 0, k = kNoLeaf;
+    uint32_t ray = 0, cur = kDead, isnew = 0;
     f3 o = mk3(0, 0, 0), d = mk3(0, 0, 0), inv = mk3(0, 0, 0);
     float t = 0.0f;
     int prim = -1;
-    Fetcher fe{fetch, n, MODE == kDual ? n2 : 0u, (int)(blockIdx.x % kFetchRanges), gridDim.x < (uint32_t)kFetchRanges};
-    while (true) {
-        // ---- refill the idle lanes once kRefillIdle of them are idle (or
-        // all of them), one claim per wave (wave-uniform)
-        const uint64_t idle = __ballot(!alive);
-        const uint32_t nidle = (uint32_t)__popcll(idle);
-        if (!exhausted && (nidle >= kRefillIdle || idle == __ballot(true))) {
-            uint32_t first = 0, count = 0, lo = 0, nfirst = 0, lo2 = 0;
-            if (!fe.get(nidle, first, count, lo, nfirst, lo2)) exhausted = true;
-            if (!alive && !exhausted) {
-                const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane_id()) - 1ull));
-                const uint32_t v = first + rank;
-                if (rank < count) {
-                    if (MODE == kDual) any = v >= nfirst;
-                    const uint32_t idx = (MODE == kDual && any) ? lo2 + (v - nfirst) : lo + v;
-                    const RayIn r = src(idx, any);
-                    ray = idx;
-                    o = r.o;
-                    d = r.d;
-                    t = r.tmax;
-                    prim = -1;
-                    inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-                    fast = (ACCEL == 4 && fast_ray(o, inv, sc.plane_flags)) ||
-                           (ACCEL == kTreeCompact && compact_ray(o, inv));
-                    st.reset();
-                    st.push4(0u, true, 0u, false, 0u, false, 0u, false);
-                    k = kNoLeaf;
-                    alive = true;
-                }
+    Fetcher fe;
+    fe.base = fetch;
+    fe.n = n;
+    fe.n2 = MODE == kDual ? n2 : 0u;
+    fe.range = (int)(blockIdx.x % kFetchRanges);
+    fe.left = gridDim.x < (uint32_t)kFetchRanges ? kFetchRanges - 1 : 0;
+    fe.open();
+    constexpr bool kQuads = (ACCEL == 4 || ACCEL == kTreeCompact) && !COUNT;
+    if constexpr (kQuads) {
+        // a small launch: the range's rays shared out evenly over its waves,
+        // at most 16 each, without claims
+        const uint32_t wpb = blockDim.x >> 6, waves = (gridDim.x / (uint32_t)kFetchRanges) * wpb;
+        if (waves != 0u && fe.total <= waves * 16u) {
+            const uint32_t per = (fe.total + waves - 1u) / waves, q = lane_id() >> 2;
+            const uint32_t v = ((blockIdx.x / (uint32_t)kFetchRanges) * wpb + (threadIdx.x >> 6)) * per + q;
+            st.reset();
+            if (q < per && v < fe.total) {
+                if (MODE == kDual) any = v >= fe.nfirst;
+                ray = (MODE == kDual && any) ? fe.lo2 + (v - fe.nfirst) : fe.lo + v;
+                src(ray, any, o, d, t);
+                inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+                fast = ACCEL == kTreeCompact && compact_ray(o, inv);
+                st.top = 4u * (threadIdx.x & ~3u);
+                cur = 0u;
             }
+            trace_quads<ACCEL>(sc, eps, o, d, inv, fast, any, ray, cur, t, prim, st, err, sink);
+            return;
         }
-        if (__ballot(alive) == 0) {
-            if (exhausted) break;
-            continue;
+    }
+    while (true) {
+        // claim rays for the idle lanes once kRefillIdle of them are idle
+        // (wave-uniform); the result is read after this step's tests
+        // (a lane whose new ray is on its way is not idle, and idle lanes stay
+        // idle until the result is there, so every claimed ray gets a lane)
+        const uint32_t want = (uint32_t)__popcll(__ballot(cur == kDead && isnew == 0u));
+        const bool refill = !exhausted && want >= kRefillIdle;
+        if (exhausted && want >= (kQuads ? 48u : 64u)) break;
+        uint32_t got;
+        if (refill) got = fe.claim(want);
+        bool done = false;
+        if (cur != kDead) {
+            float4 rows[7];
+            int kind;
+            load_item<ACCEL>(sc, cur, rows, kind);
+            // any-hit lanes of a two-queue launch of the wide tree sort too
+            // (one code path per wave)
+            done = trav_step<ACCEL, COUNT>(sc, eps, o, d, inv, fast, any, MODE != kAny, cur, t, prim, st, cnt, rows, kind);
         }
-        if (!alive) continue;
-        // ---- one step: pop (+ node test) and/or one triangle
-        if (k == kNoLeaf) {
-            const uint32_t e = st.top_pop();
-            if (ACCEL == 4 || ACCEL == kTreeCompact || ACCEL == 8) {
-                if (e & kLeafBit) {
-                    k = e & ~kLeafBit;
-                } else {
-                    if (COUNT) {
-                        if (any) ++cnt.snodes;
-                        else ++cnt.nodes;
-                    }
-                    if (ACCEL == 4) {
-                        // any-hit rays visit children nearest first too, like
-                        // traverseMBVHShadow (MBVHNode.cuh:165-205): in a
-                        // two-queue launch every lane then runs one code path
-                        // (slot order for any-hit lanes measured 2% slower)
-                        if (fast) node4_fast(sc.nodes4f, e, o, inv, t, st);
-                        else node4_step(sc.nodes4, e, o, inv, t, st);
-                    } else if (ACCEL == kTreeCompact) {
-                        if (fast) cnode4_step(sc.cnodes, e, o, inv, t, st);
-                        else node4_step(sc.nodes4, e, o, inv, t, st);
-                    } else {
-                        // any-hit lanes of a two-queue launch sort too (one
-                        // code path per wave)
-                        fnode8_step(MODE == kAny ? false : (MODE == kDual ? true : !any), sc.fnodes, e, o, inv, t,
-                                    st);
-                    }
+        if (isnew) {
+            // the ray loaded in the previous step
+            prim = -1;
+            inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+            fast = (ACCEL == 4 && fast_ray(o, inv, sc.plane_flags)) || (ACCEL == kTreeCompact && compact_ray(o, inv));
+            st.reset();
+            isnew = 0u;
+            cur = root_item<ACCEL>(sc);
+            if (ACCEL == 2 && cur == kEmptyLeaf) done = true;  // a tree without triangles
+        }
+        if (done) {
+            if (st.overflow) {
+                atomicOr(err, 1u);
+                prim = -2;
+            }
+            sink(ray, any, t, prim);
+            cur = kDead;
+        }
+        if (refill) {
+            const uint32_t first = __builtin_amdgcn_readfirstlane(got);
+            if (first < fe.total) {
+                const uint64_t m = __ballot(cur == kDead);
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                if (cur == kDead && rank < min(want, fe.total - first)) {
+                    const uint32_t v = first + rank;
+                    if (MODE == kDual) any = v >= fe.nfirst;
+                    ray = (MODE == kDual && any) ? fe.lo2 + (v - fe.nfirst) : fe.lo + v;
+                    // loads only, used a step later
+                    src(ray, any, o, d, t);
+                    isnew = 1u;
                 }
             } else {
-                const float4 lo = sc.nodes2[2 * (size_t)e];
-                const float4 hi = sc.nodes2[2 * (size_t)e + 1];
-                const int count = (int)fbits(hi.w);
-                if (count > -1) {
-                    // leaf: triangles until the end-of-leaf flag (an empty
-                    // leaf of a user-supplied tree has none)
-                    if (count > 0) k = fbits(lo.w);
-                } else {
-                    if (COUNT) {
-                        if (any) cnt.snodes += 2;
-                        else cnt.nodes += 2;
-                    }
-                    node2_step(sc.nodes2, fbits(lo.w), o, inv, st);
-                }
+                exhausted = !fe.next();
             }
         }
-        bool done = false;
-        if (k != kNoLeaf) {
-            if (COUNT) {
-                if (any) ++cnt.stris;
-                else ++cnt.tris;
-            }
-            const float4 a = sc.tris[3 * (size_t)k];
-            const float4 b = sc.tris[3 * (size_t)k + 1];
-            const float4 c = sc.tris[3 * (size_t)k + 2];
-            // p0 is needed only after the determinant test: left to the
-            // compiler its load follows that test, a second memory round trip
-            // on most triangle tests.  Held here, all three rows are in flight
-            // together.
-            __asm__ volatile("" ::"v"(a.x), "v"(a.y), "v"(a.z));
-            const uint32_t w = fbits(a.w);
-            if (tri_test(o, d, t, xyz(a), xyz(b), xyz(c), eps)) {
-                prim = (int)(w & ~kLastInLeaf);
-                if (any) done = true;
-            }
-            k = (w & kLastInLeaf) ? kNoLeaf : k + 1;
-        }
-        if (st.overflow) {
-            atomicOr(err, 1u);
-            done = true;
-            prim = -2;
-        }
-        if (done || (k == kNoLeaf && st.empty())) {
-            sink(ray, any, t, prim);
-            alive = false;
-        }
+    }
+    if constexpr (kQuads) {
+        // the wave's last rays, at most 16: lane r's alive ray number i moves
+        // to quad i (its stack stays where it is)
+        const uint64_t alive = __ballot(cur != kDead);
+        if (alive == 0) return;
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(alive >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)alive, 0u));
+        // idle lanes send to the quads past the last ray, where nothing reads
+        const uint32_t n_alive = (uint32_t)__popcll(alive);
+        const uint32_t dst = 4u * (cur != kDead ? rank : 0u);
+        const uint32_t from = quad_dpp<0x00>((uint32_t)__builtin_amdgcn_ds_permute((int)(4u * (cur != kDead ? dst : dst + 1u)), (int)lane_id()));
+        const bool live = (lane_id() >> 2) < n_alive;
+        const int sl = live ? (int)from : 0;
+        const uint32_t flags = __shfl((any ? 1u : 0u) | (fast ? 2u : 0u), sl);
+        const f3 qo = mk3(__shfl(o.x, sl), __shfl(o.y, sl), __shfl(o.z, sl));
+        const f3 qd = mk3(__shfl(d.x, sl), __shfl(d.y, sl), __shfl(d.z, sl));
+        const f3 qi = mk3(__shfl(inv.x, sl), __shfl(inv.y, sl), __shfl(inv.z, sl));
+        const float qt = __shfl(t, sl);
+        const int qp = __shfl(prim, sl);
+        const uint32_t qr = __shfl(ray, sl), qtop = __shfl(st.top, sl), qc = __shfl(cur, sl);
+        st.top = qtop;
+        st.overflow = false;
+        trace_quads<ACCEL>(sc, eps, qo, qd, qi, (flags & 2u) != 0u, (flags & 1u) != 0u, qr, live ? qc : kDead, qt, qp, st,
+                           err, sink);
     }
 }
 
@@ -661,51 +996,19 @@ CT_DEV int trace_single(const DevScene& sc, float eps, f3 o, f3 d, float& t, boo
     const bool fast = (ACCEL == 4 && fast_ray(o, inv, sc.plane_flags)) ||
                       (ACCEL == kTreeCompact && compact_ray(o, inv));
     int prim = -1;
-    uint32_t k = kNoLeaf;
+    uint32_t cur = root_item<ACCEL>(sc);
+    TravCount cnt{0u, 0u, 0u, 0u};
     st.reset();
-    st.push4(0u, true, 0u, false, 0u, false, 0u, false);
+    if (ACCEL == 2 && cur == kEmptyLeaf) return prim;  // a tree without triangles
     while (true) {
-        if (k == kNoLeaf) {
-            const uint32_t e = st.top_pop();
-            if (ACCEL == 4 || ACCEL == kTreeCompact || ACCEL == 8) {
-                if (e & kLeafBit) {
-                    k = e & ~kLeafBit;
-                } else if (ACCEL == 4) {
-                    if (fast) node4_fast(sc.nodes4f, e, o, inv, t, st);
-                    else node4_step(sc.nodes4, e, o, inv, t, st);
-                } else if (ACCEL == kTreeCompact) {
-                    if (fast) cnode4_step(sc.cnodes, e, o, inv, t, st);
-                    else node4_step(sc.nodes4, e, o, inv, t, st);
-                } else {
-                    fnode8_step(true, sc.fnodes, e, o, inv, t, st);
-                }
-            } else {
-                const float4 lo = sc.nodes2[2 * (size_t)e];
-                const float4 hi = sc.nodes2[2 * (size_t)e + 1];
-                const int count = (int)fbits(hi.w);
-                if (count > -1) {
-                    if (count > 0) k = fbits(lo.w);
-                } else {
-                    node2_step(sc.nodes2, fbits(lo.w), o, inv, st);
-                }
-            }
-        }
-        if (k != kNoLeaf) {
-            const float4 a = sc.tris[3 * (size_t)k];
-            const float4 b = sc.tris[3 * (size_t)k + 1];
-            const float4 c = sc.tris[3 * (size_t)k + 2];
-            const uint32_t w = fbits(a.w);
-            if (tri_test(o, d, t, xyz(a), xyz(b), xyz(c), eps)) {
-                prim = (int)(w & ~kLastInLeaf);
-                if (any) break;
-            }
-            k = (w & kLastInLeaf) ? kNoLeaf : k + 1;
-        }
-        if (st.overflow) {
-            atomicOr(err, 1u);
-            return -2;
-        }
-        if (k == kNoLeaf && st.empty()) break;
+        float4 n[7];
+        int kind;
+        load_item<ACCEL>(sc, cur, n, kind);
+        if (trav_step<ACCEL, false>(sc, eps, o, d, inv, fast, any, true, cur, t, prim, st, cnt, n, kind)) break;
+    }
+    if (st.overflow) {
+        atomicOr(err, 1u);
+        return -2;
     }
     return prim;
 }

@@ -310,6 +310,23 @@ int prepare_quad(ct_ctx* c, ctd::DevScene& sc) {
     return CT_OK;
 }
 
+// The binary root's traversal item (sc.root2; item2 in device/traverse.h):
+// its children's index, kLeafBit | first triangle record, or 0xFFFFFFFE for
+// an empty leaf.
+int prepare_binary(ct_ctx* c, ctd::DevScene& sc) {
+    sc.root2 = 0;
+    if (!sc.nodes2 || sc.n_nodes2 == 0) return CT_OK;
+    ct_bvh_node n;
+    // on the lane's stream: the null stream would take a hardware queue, and
+    // with it gone a later context's two lanes can share one (C2 frame 3.65
+    // against 4.80 ms)
+    const hipStream_t s = c->ln[0].stream;
+    HIPCHK(hipMemcpyAsync(&n, sc.nodes2, sizeof(n), hipMemcpyDeviceToHost, s), "binary root");
+    HIPCHK(hipStreamSynchronize(s), "binary root");
+    sc.root2 = n.count < 0 ? (uint32_t)n.left_first : (n.count > 0 ? ctd::kLeafBit | (uint32_t)n.left_first : 0xFFFFFFFEu);
+    return CT_OK;
+}
+
 // Make an uploaded scene current (tree fields of sc already set).
 void install_scene(ct_ctx* c, const ct_scene_view* v, ctd::DevScene sc, const Shading& sh, uint32_t wide_bound) {
     const uint32_t N = v->n_triangles;
@@ -408,7 +425,7 @@ int ct_scene_upload(ct_ctx* c, const ct_scene_view* v) {
     sc.n_nodes4 = v->n_mbvh_nodes;
     sc.n_nodes2 = v->n_bvh_nodes;
     sc.n_fnodes = (uint32_t)(fn.size() / ct::kWideNodeWords);
-    if ((r = prepare_quad(c, sc)) != CT_OK) { free_scene(c); return r; }
+    if ((r = prepare_quad(c, sc)) != CT_OK || (r = prepare_binary(c, sc)) != CT_OK) { free_scene(c); return r; }
     install_scene(c, v, sc, sh, wide_bound);
     return CT_OK;
 }
@@ -458,7 +475,7 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     }
     if (r != CT_OK) { free_scene(c); return r; }
     HIPCHK(hipStreamSynchronize(c->ln[0].stream), "scene upload");
-    if ((r = prepare_quad(c, sc)) != CT_OK) { free_scene(c); return r; }
+    if ((r = prepare_quad(c, sc)) != CT_OK || (r = prepare_binary(c, sc)) != CT_OK) { free_scene(c); return r; }
     install_scene(c, v, sc, sh, wide_bound);
     bs.total_ms = (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (st) *st = bs;
@@ -739,7 +756,7 @@ int ct_trace_rays(ct_ctx* c, const float* origins, const float* dirs, uint32_t n
         HIPCHK(hipMemcpyAsync(c->ln[0].q.ray_d[0], rd.data(), m * sizeof(float4), hipMemcpyHostToDevice, c->ln[0].stream), "rays");
         HIPCHK(hipMemcpyAsync(c->ln[0].d_hdr, &h, sizeof(h), hipMemcpyHostToDevice, c->ln[0].stream), "header");
         HIPCHK(ctk::launch_setup(c->ln[0].q.counters, c->ln[0].d_hdr, c->ln[0].stream), "setup");
-        HIPCHK(ctk::launch_extend(c->shape, c->sc, to, c->ln[0].q, 0, 0, c->ln[0].stream), "extend");
+        HIPCHK(ctk::launch_extend(c->shape, c->sc, to, c->ln[0].q, 0, 0, m, c->ln[0].stream), "extend");
         uint32_t errflag = 0;
         HIPCHK(hipMemcpyAsync(hits.data(), c->ln[0].q.hit, m * sizeof(float2), hipMemcpyDeviceToHost, c->ln[0].stream), "hits");
         HIPCHK(hipMemcpyAsync(&errflag, c->ln[0].q.err, 4, hipMemcpyDeviceToHost, c->ln[0].stream), "flags");
@@ -820,7 +837,7 @@ int ct_trace_rays_device(ct_ctx* c, const void* d_rays_o, const void* d_rays_d, 
     HIPCHK(hipMemcpyAsync(c->ln[0].d_hdr, &h, sizeof(h), hipMemcpyHostToDevice, c->ln[0].stream), "header");
     HIPCHK(ctk::launch_setup(c->ln[0].q.counters, c->ln[0].d_hdr, c->ln[0].stream), "setup");
     HIPCHK(hipEventRecord(c->ln[0].ev[0], c->ln[0].stream), "event");
-    HIPCHK(ctk::launch_extend(c->shape, c->sc, to, q, 0, 0, c->ln[0].stream), "extend");
+    HIPCHK(ctk::launch_extend(c->shape, c->sc, to, q, 0, 0, n, c->ln[0].stream), "extend");
     HIPCHK(hipEventRecord(c->ln[0].ev[1], c->ln[0].stream), "event");
     uint32_t errflag = 0;
     HIPCHK(hipMemcpyAsync(&errflag, c->ln[0].q.err, 4, hipMemcpyDeviceToHost, c->ln[0].stream), "flags");

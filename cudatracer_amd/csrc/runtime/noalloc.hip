@@ -98,7 +98,7 @@ extern "C" int ct_trace_rays_device_noalloc(ct_ctx* c, const void* d_rays_o, con
     hipStream_t s = c->ln[0].stream;
     HIPCHK(ctk::launch_setup_rays(q.counters, q.err, n, s), "setup");
     HIPCHK(hipEventRecord(c->ln[0].ev[0], s), "event");
-    HIPCHK(ctk::launch_extend(ls, c->sc, to, q, 0, 0, s), "extend");
+    HIPCHK(ctk::launch_extend(ls, c->sc, to, q, 0, 0, n, s), "extend");
     HIPCHK(hipEventRecord(c->ln[0].ev[1], s), "event");
     uint32_t errflag = 0;
     HIPCHK(hipMemcpyAsync(&errflag, q.err, 4, hipMemcpyDeviceToHost, s), "flags");
