@@ -1071,6 +1071,53 @@ hipError_t launch_prepare_quad(const float4* nodes4, uint32_t n4, float4* fast, 
     hipLaunchKernelGGL(k_prepare_quad, dim3(blocks), dim3(256), 0, s, nodes4, n4, fast, compact, flags);
     return hipGetLastError();
 }
+// The primitives' shading records (DevScene::sh_prim) from the scene's arrays.
+// Bound by its writes: 128 bytes a primitive.  Eight lanes write a record, one
+// row each, so a wave's stores are eight whole 128-byte lines; gathered on the
+// host and copied, the records of 1,000,003 triangles took 27 ms of a
+// 43 ms upload, from the raw arrays (a quarter of the bytes over PCIe) 2 ms.
+__global__ void k_shading_records(const float* __restrict__ vert, const float* __restrict__ norm,
+                                  const float* __restrict__ uv, const uint32_t* __restrict__ idx,
+                                  const float* __restrict__ cn, const uint32_t* __restrict__ mat, uint32_t n,
+                                  float4* __restrict__ out) {
+    const uint64_t rows = (uint64_t)n * kPrimRows;
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t row = (uint32_t)i % kPrimRows;
+        const uint64_t prim = i / kPrimRows;
+        float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (row < 6) {
+            const uint32_t j = row < 3 ? row : row - 3;
+            const uint64_t vi = idx[3 * prim + j];
+            const float* p = (row < 3 ? vert : norm) + 3 * vi;
+            r = make_float4(p[0], p[1], p[2], 0.0f);
+        } else if (row == 6) {
+            const float* p = cn + 3 * prim;
+            r = make_float4(p[0], p[1], p[2], 0.0f);
+        }
+        // .w: the material, then u0, v0, u1, v1, u2, v2 (TriangleList.cpp:148-178)
+        if (row == 0) r.w = __uint_as_float(mat[prim]);
+        else if (row < 7 && uv) r.w = uv[2 * (uint64_t)idx[3 * prim + (row - 1) / 2] + (row - 1) % 2];
+        out[i] = r;
+    }
+}
+hipError_t launch_shading_records(const float* vert, const float* norm, const float* uv, const uint32_t* idx,
+                                  const float* cn, const uint32_t* mat, uint32_t n, float4* out, hipStream_t s) {
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(((uint64_t)n * kPrimRows + 255) / 256, 65536u);
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_shading_records, dim3(blocks), dim3(256), 0, s, vert, norm, uv, idx, cn, mat, n, out);
+    return hipGetLastError();
+}
+// Primitive ids of the triangle records first ... first + n - 1.
+__global__ void k_prim_ids(const float4* __restrict__ tris, uint32_t first, uint32_t n, uint32_t* __restrict__ out) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        out[i] = __float_as_uint(tris[3 * ((size_t)first + i)].w) & ~kLastInLeaf;
+}
+hipError_t launch_prim_ids(const float4* tris, uint32_t first, uint32_t n, uint32_t* out, hipStream_t s) {
+    const uint32_t blocks = std::min<uint32_t>((n + 255) / 256, 65536u);
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_prim_ids, dim3(blocks), dim3(256), 0, s, tris, first, n, out);
+    return hipGetLastError();
+}
 hipError_t launch_tonemap(const float4* accum, uint32_t n, float samples, float4* out, hipStream_t s) {
     const uint32_t blocks = std::min<uint32_t>((n + 255) / 256, 65536u);
     if (blocks == 0) return hipSuccess;

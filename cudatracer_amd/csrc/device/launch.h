@@ -71,6 +71,12 @@ hipError_t launch_tonemap8(const float4* accum, uint32_t n, float samples, uint3
 // cleared first).
 hipError_t launch_prepare_quad(const float4* nodes4, uint32_t n4, float4* fast, uint4* compact, uint32_t* flags,
                                hipStream_t s);
+// The shading records of n primitives (kPrimRows rows each) from the scene's
+// arrays; uv may be null.
+hipError_t launch_shading_records(const float* vert, const float* norm, const float* uv, const uint32_t* idx,
+                                  const float* cn, const uint32_t* mat, uint32_t n, float4* out, hipStream_t s);
+// The primitive ids of n triangle records from `first` on.
+hipError_t launch_prim_ids(const float4* tris, uint32_t first, uint32_t n, uint32_t* out, hipStream_t s);
 hipError_t launch_shadow_flags(const LaunchShape& ls, const ctd::DevScene& sc, const ctd::TraceOpts& to,
                                const ctd::Queues& q, uint32_t n, uint8_t* out, hipStream_t s);
 

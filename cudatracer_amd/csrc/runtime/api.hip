@@ -16,8 +16,6 @@ using namespace ctr;
 
 namespace {
 
-bool finite3(const float* p) { return std::isfinite(p[0]) && std::isfinite(p[1]) && std::isfinite(p[2]); }
-
 // triangle::getArea (Triangle.cuh:89-96) in float, glm order.
 float heron_area(const float* p0, const float* p1, const float* p2) {
     auto len = [](const float* a, const float* b) {
@@ -166,12 +164,14 @@ int check_geometry(ct_ctx* c, const ct_scene_view* v) {
     if (!v->vertices || !v->normals || !v->indices || !v->center_normals || !v->material_idx || !v->materials ||
         v->n_materials == 0 || (v->n_lights && !v->light_indices))
         return fail(c, CT_ERR_INVALID_ARG, "scene view is missing an array");
-    for (uint64_t i = 0; i < 3ull * N; ++i)
-        if (v->indices[i] >= V) return fail(c, CT_ERR_INVALID_SCENE, "vertex index out of range");
-    for (uint32_t i = 0; i < V; ++i)
-        if (!finite3(v->vertices + 3 * (size_t)i)) return fail(c, CT_ERR_INVALID_SCENE, "non-finite vertex");
-    for (uint32_t i = 0; i < N; ++i)
-        if (v->material_idx[i] >= v->n_materials) return fail(c, CT_ERR_INVALID_SCENE, "material index out of range");
+    // reductions without early exits: the compiler makes them vector code
+    uint32_t bad = 0;
+    for (uint64_t i = 0; i < 3ull * N; ++i) bad |= v->indices[i] >= V ? 1u : 0u;
+    if (bad) return fail(c, CT_ERR_INVALID_SCENE, "vertex index out of range");
+    for (uint64_t i = 0; i < 3ull * V; ++i) bad |= std::isfinite(v->vertices[i]) ? 0u : 1u;
+    if (bad) return fail(c, CT_ERR_INVALID_SCENE, "non-finite vertex");
+    for (uint32_t i = 0; i < N; ++i) bad |= v->material_idx[i] >= v->n_materials ? 1u : 0u;
+    if (bad) return fail(c, CT_ERR_INVALID_SCENE, "material index out of range");
     for (uint32_t i = 0; i < v->n_lights; ++i)
         if (v->light_indices[i] >= N) return fail(c, CT_ERR_INVALID_SCENE, "light index out of range");
     if (v->n_textures > 0xFFFEu) return fail(c, CT_ERR_INVALID_SCENE, "too many textures");
@@ -191,9 +191,10 @@ int check_geometry(ct_ctx* c, const ct_scene_view* v) {
     return CT_OK;
 }
 
-// Host staging of the tree-independent device arrays.
+// Host staging of the tree-independent device arrays (the shading records
+// aside, which upload_prim_records makes).
 struct Shading {
-    std::vector<float4> prim, mats, lights;  // prim: ctd::kPrimRows rows per primitive
+    std::vector<float4> mats, lights;
     std::vector<float4> texels;
     std::vector<uint32_t> texels8;
     std::vector<uint4> tex_info;
@@ -215,12 +216,13 @@ bool is_8bit(const ct_texture& x) {
     return true;
 }
 
-void stage_shading(const ct_scene_view* v, Shading& sh) {
+// The shading records gathered on the host: kPrimRows rows per primitive.
+void stage_prim_records(const ct_scene_view* v, std::vector<float4>& prim_rows) {
     const uint32_t N = v->n_triangles;
     constexpr size_t R = ctd::kPrimRows;
-    sh.prim.assign((size_t)N * R, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+    prim_rows.assign((size_t)N * R, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     for (uint32_t prim = 0; prim < N; ++prim) {
-        float4* row = &sh.prim[R * prim];
+        float4* row = &prim_rows[R * prim];
         // texture coordinates u0, v0, u1, v1, u2, v2 (TriangleList.cpp:148-178)
         float t[6] = {0, 0, 0, 0, 0, 0};
         if (v->n_textures && v->texcoords)
@@ -236,6 +238,68 @@ void stage_shading(const ct_scene_view* v, Shading& sh) {
         }
         row[6] = f4(v->center_normals + 3 * (size_t)prim, t[5]);
     }
+}
+
+// The scene arrays that device kernels read, in temporary device memory.
+struct DeviceArrays {
+    ct_ctx* c;
+    std::vector<void*> bufs;
+    explicit DeviceArrays(ct_ctx* cc) : c(cc) {}
+    ~DeviceArrays() { release(); }
+    void release() {
+        for (void* p : bufs) dfree(c, p);
+        bufs.clear();
+    }
+    template <class T>
+    int put(const T* host, size_t count, const T** dev, const char* what) {
+        void* p = nullptr;
+        const int r = dalloc(c, &p, count * sizeof(T), what);
+        if (r != CT_OK) return r;
+        bufs.push_back(p);
+        HIPCHK(hipMemcpyAsync(p, host, count * sizeof(T), hipMemcpyHostToDevice, c->ln[0].stream), what);
+        *dev = static_cast<const T*>(p);
+        return CT_OK;
+    }
+};
+
+// The shading records, made on the device from the scene's arrays, or on the
+// host if these do not fit beside them.  tmp holds the arrays (vert and idx
+// may be there already) until the stream has run the kernel.
+int upload_prim_records(ct_ctx* c, const ct_scene_view* v, DeviceArrays& tmp, const float* vert, const uint32_t* idx,
+                        ctd::DevScene& sc) {
+    const size_t N = v->n_triangles, V = v->n_vertices;
+    void* out = nullptr;
+    int r = dalloc(c, &out, N * ctd::kPrimRows * sizeof(float4), "shading records");
+    if (r != CT_OK) return r;
+    c->scene_bufs.push_back(out);
+    sc.sh_prim = static_cast<const float4*>(out);
+    const float *norm = nullptr, *cn = nullptr, *uv = nullptr;
+    const uint32_t* mat = nullptr;
+    r = CT_OK;
+    if (!vert) r = tmp.put(v->vertices, 3 * V, &vert, "vertices");
+    if (r == CT_OK && !idx) r = tmp.put(v->indices, 3 * N, &idx, "indices");
+    if (r == CT_OK) r = tmp.put(v->normals, 3 * V, &norm, "normals");
+    if (r == CT_OK) r = tmp.put(v->center_normals, 3 * N, &cn, "centre normals");
+    if (r == CT_OK) r = tmp.put(v->material_idx, N, &mat, "material indices");
+    if (r == CT_OK && v->n_textures && v->texcoords) r = tmp.put(v->texcoords, 2 * V, &uv, "texture coordinates");
+    hipStream_t s = c->ln[0].stream;
+    if (r == CT_OK) {
+        HIPCHK(ctk::launch_shading_records(vert, norm, uv, idx, cn, mat, (uint32_t)N, static_cast<float4*>(out), s),
+               "shading records");
+    } else if (r == CT_ERR_OUT_OF_MEMORY) {
+        HIPCHK(hipStreamSynchronize(s), "shading records");
+        tmp.release();
+        std::vector<float4> rows;
+        stage_prim_records(v, rows);
+        HIPCHK(hipMemcpyAsync(out, rows.data(), rows.size() * sizeof(float4), hipMemcpyHostToDevice, s),
+               "shading records");
+        HIPCHK(hipStreamSynchronize(s), "shading records");
+        r = CT_OK;
+    }
+    return r;
+}
+
+void stage_shading(const ct_scene_view* v, Shading& sh) {
     sh.mats.resize((size_t)v->n_materials * 2);
     for (uint32_t m = 0; m < v->n_materials; ++m) mat_rows(v->materials[m], &sh.mats[2 * (size_t)m]);
     sh.lights.resize((size_t)std::max<uint32_t>(v->n_lights, 1u) * 5);
@@ -260,8 +324,7 @@ void stage_shading(const ct_scene_view* v, Shading& sh) {
 }
 
 int upload_shading(ct_ctx* c, const Shading& sh, ctd::DevScene& sc) {
-    int r = upload_vec(c, sh.prim, &sc.sh_prim, "shading records");
-    if (r == CT_OK) r = upload_vec(c, sh.mats, &sc.mats, "materials");
+    int r = upload_vec(c, sh.mats, &sc.mats, "materials");
     if (r == CT_OK) r = upload_vec(c, sh.lights, &sc.lights, "lights");
     if (r == CT_OK && !sh.tex_info.empty()) {
         r = upload_vec(c, sh.texels, &sc.texels, "textures");
@@ -411,7 +474,14 @@ int ct_scene_upload(ct_ctx* c, const ct_scene_view* v) {
     sync_lanes(c);
     free_scene(c);
     ctd::DevScene sc{};
-    r = upload_vec(c, tris, &sc.tris, "triangles");
+    {
+        // first, while the other arrays' memory is still free
+        DeviceArrays tmp(c);
+        r = upload_prim_records(c, v, tmp, nullptr, nullptr, sc);
+        if (r == CT_OK && hipStreamSynchronize(c->ln[0].stream) != hipSuccess)
+            r = fail(c, CT_ERR_DEVICE, "shading records");
+    }
+    if (r == CT_OK) r = upload_vec(c, tris, &sc.tris, "triangles");
     if (r == CT_OK) r = upload_shading(c, sh, sc);
     if (r == CT_OK && !n4.empty()) r = upload_vec(c, n4, &sc.nodes4, "quad nodes");
     if (r == CT_OK) {
@@ -444,7 +514,12 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     ctd::DevScene sc{};
     ct_build_stats bs{};
     DeviceTrees t;
-    r = device_build(c, v, &t, &bs);
+    DeviceArrays tmp(c);
+    const float* d_vert = nullptr;
+    const uint32_t* d_idx = nullptr;
+    r = tmp.put(v->vertices, 3 * (size_t)v->n_vertices, &d_vert, "build: vertices");
+    if (r == CT_OK) r = tmp.put(v->indices, 3 * (size_t)v->n_triangles, &d_idx, "build: indices");
+    if (r == CT_OK) r = device_build(c, v, d_vert, d_idx, &t, &bs);
     for (void* p : {(void*)t.tris, (void*)t.nodes2, (void*)t.nodes4})
         if (p) c->scene_bufs.push_back(p);
     if (r != CT_OK) { free_scene(c); return r; }
@@ -453,7 +528,8 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     sc.nodes4 = reinterpret_cast<const float4*>(t.nodes4);
     sc.n_nodes2 = t.n2;
     sc.n_nodes4 = t.n4;
-    r = upload_shading(c, sh, sc);
+    r = upload_prim_records(c, v, tmp, d_vert, d_idx, sc);
+    if (r == CT_OK) r = upload_shading(c, sh, sc);
     uint32_t wide_bound = 0;
     if (r == CT_OK && (flags & CT_BUILD_WIDE)) {
         // wide nodes are collapsed on the host from the device-built trees
@@ -475,6 +551,7 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     }
     if (r != CT_OK) { free_scene(c); return r; }
     HIPCHK(hipStreamSynchronize(c->ln[0].stream), "scene upload");
+    tmp.release();
     if ((r = prepare_quad(c, sc)) != CT_OK || (r = prepare_binary(c, sc)) != CT_OK) { free_scene(c); return r; }
     install_scene(c, v, sc, sh, wide_bound);
     bs.total_ms = (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -500,15 +577,27 @@ int ct_scene_read_trees(ct_ctx* c, ct_bvh_node* bvh, uint32_t cap_bvh, ct_mbvh_n
     const uint32_t n2 = c->has_bvh2 ? c->sc.n_nodes2 : 0, n4 = c->has_bvh4 ? c->sc.n_nodes4 : 0, N = c->sc.n_tris;
     if ((bvh && cap_bvh < n2) || (mbvh && cap_mbvh < n4) || (prim_indices && cap_prims < N))
         return fail(c, CT_ERR_INVALID_ARG, "output capacity too small");
-    if (bvh && n2) HIPCHK(hipMemcpy(bvh, c->sc.nodes2, n2 * sizeof(ct_bvh_node), hipMemcpyDeviceToHost), "read trees");
+    const hipStream_t s = c->ln[0].stream;
+    if (bvh && n2)
+        HIPCHK(hipMemcpyAsync(bvh, c->sc.nodes2, n2 * sizeof(ct_bvh_node), hipMemcpyDeviceToHost, s), "read trees");
     if (mbvh && n4)
-        HIPCHK(hipMemcpy(mbvh, c->sc.nodes4, n4 * sizeof(ct_mbvh_node), hipMemcpyDeviceToHost), "read trees");
+        HIPCHK(hipMemcpyAsync(mbvh, c->sc.nodes4, n4 * sizeof(ct_mbvh_node), hipMemcpyDeviceToHost, s), "read trees");
+    HIPCHK(hipStreamSynchronize(s), "read trees");
     if (prim_indices) {
-        // primitive id of slot k: the w word of its first record, without the last-in-leaf bit
-        HIPCHK(hipMemcpy2D(prim_indices, 4, reinterpret_cast<const char*>(c->sc.tris) + 12, 3 * sizeof(float4), 4, N,
-                           hipMemcpyDeviceToHost),
-               "read trees");
-        for (uint32_t k = 0; k < N; ++k) prim_indices[k] &= 0x7FFFFFFFu;
+        // gathered on the device, a part of at most 4M ids at a time (a
+        // strided copy of the records' id words cost 7 us a row)
+        const uint32_t part = std::min<uint32_t>(N, 1u << 22);
+        uint32_t* ids = nullptr;
+        HIPCHK(hipMalloc(&ids, (size_t)part * 4), "read trees");
+        hipError_t e = hipSuccess;
+        for (uint32_t k = 0; k < N && e == hipSuccess; k += part) {
+            const uint32_t m = std::min(part, N - k);
+            e = ctk::launch_prim_ids(c->sc.tris, k, m, ids, s);
+            if (e == hipSuccess) e = hipMemcpyAsync(prim_indices + k, ids, (size_t)m * 4, hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipStreamSynchronize(s);
+        }
+        (void)hipFree(ids);
+        if (e != hipSuccess) return hip_fail(c, e, "read trees");
     }
     return CT_OK;
 }

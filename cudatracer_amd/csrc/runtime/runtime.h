@@ -180,8 +180,10 @@ struct DeviceTrees {
     uint32_t n2 = 0, n4 = 0;
 };
 // Build the binary and quad trees of v's triangles on lane 0's stream; the
-// result equals the host build byte for byte.
-int device_build(ct_ctx* c, const ct_scene_view* v, DeviceTrees* out, ct_build_stats* st);
+// result equals the host build byte for byte.  d_vert, d_idx: the view's
+// vertices and indices in device memory.
+int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const uint32_t* d_idx, DeviceTrees* out,
+                 ct_build_stats* st);
 }  // namespace ctr
 
 namespace ctr {

@@ -151,3 +151,59 @@ def test_wide_tree_after_device_build(ct, gpu_ctx, c1):
     gpu_ctx.upload_build(scene)
     with pytest.raises(ct.CTError):
         gpu_ctx.trace_frame(cam, o)
+
+
+def test_shading_records_without_room_for_the_arrays(ct):
+    """The shading records are made on the device from the scene's arrays, or
+    on the host if these do not fit the budget beside them: the same frame
+    either way.  One leaf holds every triangle, so the arrays (about 228 bytes
+    a triangle with the records) need more than the finished scene (176)."""
+    import re
+
+    from conftest import ArrayView
+    from test_gpu_stack import chain_scene
+
+    def leaf_scene(n):
+        a = chain_scene(ct, 1, seed=8)
+        rng = np.random.default_rng(9)
+        v = rng.uniform(-8, 8, (n, 1, 3)) + rng.uniform(-0.5, 0.5, (n, 3, 3))
+        cn = np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0])
+        cn /= np.linalg.norm(cn, axis=1, keepdims=True)
+        a["vertices"] = v.reshape(-1, 3).astype(np.float32)
+        a["normals"] = np.repeat(cn, 3, axis=0).astype(np.float32)
+        a["center_normals"] = cn.astype(np.float32)
+        a["texcoords"] = np.zeros((3 * n, 2), np.float32)
+        a["indices"] = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+        a["material_idx"] = np.zeros(n, np.uint32)
+        a["prim_indices"] = np.arange(n, dtype=np.uint32)
+        m = np.zeros((1, 32), np.uint32)
+        f = m.view(np.float32)
+        f[0, 0:24:8], f[0, 4:24:8] = -10.0, 10.0
+        m[0, 24:28] = [0, 0xFFFFFFFF, 0xFFFFFFFF, 0xFFFFFFFF]
+        m[0, 28:32] = [n, 0, 0, 0]
+        a["mbvh"] = m.view(np.uint8).ravel()
+        return ArrayView(ct, a)
+
+    n = 20_000
+    small, large = leaf_scene(4), leaf_scene(n)
+    opts = ct.default_opts()
+    opts.max_depth = 2
+    cam = ct.look_at((-30.0, 0.5, 0.3), (0.0, 0.0, 0.0), 30.0)
+    frames = []
+    used = 0
+    for budget in (1 << 31, 0):
+        ctx = ct.Context(0, mem_budget=budget or used + 200 * n)
+        ctx.upload_view(small.view)
+        ctx.resize(8, 8)
+        ctx.trace_frame(cam, opts)
+        if budget:
+            with pytest.raises(ct.CTError) as e:
+                ctx.resize(16384, 16384)
+            used = int(re.search(r"(\d+) of \d+ in use", str(e.value)).group(1)) + 8 * 8 * 16
+            ctx.resize(8, 8)
+        ctx.upload_view(large.view)
+        ctx.reset()
+        ctx.trace_frame(cam, opts)
+        frames.append(ctx.read_accum()[0])
+        ctx.close()
+    assert np.array_equal(_bits(frames[0]), _bits(frames[1]))
