@@ -67,7 +67,7 @@ struct DevScene {
     int sky_tex;            // -1: the constant sky colour
     float sky_r, sky_g, sky_b;
     uint32_t root2;         // the binary root's traversal item (item2 in device/traverse.h)
-    uint32_t plane_flags;   // kPlaneNegZero | kPlaneNaN | kCompactBad over the quad tree
+    uint32_t plane_flags;   // kPlaneNegZero | kPlaneNaN | kCompactBad over the quad tree, kPlaneInf2
 };
 
 // A primitive's shading record (sh_prim), indexed by primitive id: what
@@ -79,10 +79,13 @@ struct DevScene {
 // (texture coordinates are zero without textures).
 constexpr int kPrimRows = 8;
 
-// Properties of the quad tree's box planes, found at upload (k_plane_flags).
+// Properties of the trees' box planes, found at upload (k_prepare_quad,
+// k_prepare_binary).
 constexpr uint32_t kPlaneNegZero = 1u;  // some plane is -0.0
 constexpr uint32_t kPlaneNaN = 2u;      // some plane is NaN
 constexpr uint32_t kCompactBad = 8u;    // some node's boxes have no compact encoding (not finite, or too large)
+
+constexpr uint32_t kPlaneInf2 = 16u;    // some plane of the binary tree is not finite
 
 // One camera view (plain frame, batch member or served request).
 struct ViewDesc {

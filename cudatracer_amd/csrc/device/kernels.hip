@@ -1071,6 +1071,21 @@ hipError_t launch_prepare_quad(const float4* nodes4, uint32_t n4, float4* fast, 
     hipLaunchKernelGGL(k_prepare_quad, dim3(blocks), dim3(256), 0, s, nodes4, n4, fast, compact, flags);
     return hipGetLastError();
 }
+// kPlaneInf2 over the binary tree's boxes (flags as in k_prepare_quad).
+__global__ void k_prepare_binary(const float4* __restrict__ nodes2, uint32_t n2, uint32_t* flags) {
+    bool bad = false;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 2u * n2; i += gridDim.x * blockDim.x) {
+        const float4 v = nodes2[i];
+        bad |= !(isfinite(v.x) && isfinite(v.y) && isfinite(v.z));
+    }
+    if (__ballot(bad) && __lane_id() == 0) atomicOr(flags, kPlaneInf2);
+}
+hipError_t launch_prepare_binary(const float4* nodes2, uint32_t n2, uint32_t* flags, hipStream_t s) {
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((2ull * n2 + 255) / 256, 4096u);
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_prepare_binary, dim3(blocks), dim3(256), 0, s, nodes2, n2, flags);
+    return hipGetLastError();
+}
 // The primitives' shading records (DevScene::sh_prim) from the scene's arrays.
 // Bound by its writes: 128 bytes a primitive.  Eight lanes write a record, one
 // row each, so a wave's stores are eight whole 128-byte lines; gathered on the

@@ -71,6 +71,8 @@ hipError_t launch_tonemap8(const float4* accum, uint32_t n, float samples, uint3
 // cleared first).
 hipError_t launch_prepare_quad(const float4* nodes4, uint32_t n4, float4* fast, uint4* compact, uint32_t* flags,
                                hipStream_t s);
+// The binary tree's plane flag (*flags cleared first).
+hipError_t launch_prepare_binary(const float4* nodes2, uint32_t n2, uint32_t* flags, hipStream_t s);
 // The shading records of n primitives (kPrimRows rows each) from the scene's
 // arrays; uv may be null.
 hipError_t launch_shading_records(const float* vert, const float* norm, const float* uv, const uint32_t* idx,

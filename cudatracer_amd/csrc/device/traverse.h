@@ -26,7 +26,7 @@
 //     limit (64) bounds the stack at 97 entries; the stack bound
 //     (Queues::max_stack, 128 by default) guards user-supplied trees.
 // 1,048,576 rays against 524,287 triangles: 0.641 ms per call with two round
-// trips per step, waited-for claims and one lane a ray throughout, 0.511 ms
+// trips per step, waited-for claims and one lane a ray throughout, 0.497 ms
 // as it is; the 1080p atrium frame 3.87 and 3.50 ms.
 #pragma once
 
@@ -462,6 +462,28 @@ CT_DEV bool box2(float4 lo, float4 hi, f3 o, f3 inv, float& tmin) {
     return tmax >= 0.0f && tmin < tmax;
 }
 
+// The same test with the hardware minimum and maximum.  Without NaN they give
+// box2's values up to the sign of a zero, which no comparison here sees, so a
+// ray that finite_ray() accepts visits the same nodes in the same order.  Two
+// boxes take 46 instructions instead of 70: the box's frame of 65,536 paths
+// spends its time in chains of these steps.
+CT_DEV bool box2_fast(float4 lo, float4 hi, f3 o, f3 inv, float& tmin) {
+    const f3 t1 = (xyz(lo) - o) * inv;
+    const f3 t2 = (xyz(hi) - o) * inv;
+    tmin = fmaxf(fmaxf(fminf(t1.x, t2.x), fminf(t1.y, t2.y)), fminf(t1.z, t2.z));
+    const float tmax = fminf(fminf(fmaxf(t1.x, t2.x), fmaxf(t1.y, t2.y)), fmaxf(t1.z, t2.z));
+    return tmax >= 0.0f && tmin < tmax;
+}
+// No slab value (plane - o) * inv of the binary tree is NaN: planes (checked
+// at upload) and origin are finite, and inv is neither infinite (0 * inf) nor
+// zero (an overflown difference times 0).
+CT_DEV bool finite_ray(f3 o, f3 inv, uint32_t plane_flags) {
+    constexpr float kMax = 3.40282347e38f;
+    auto ok = [](float v) { return fabsf(v) > 0.0f && fabsf(v) <= kMax; };
+    return !(plane_flags & kPlaneInf2) && ok(inv.x) && ok(inv.y) && ok(inv.z) && fabsf(o.x) <= kMax &&
+           fabsf(o.y) <= kMax && fabsf(o.z) <= kMax;
+}
+
 // The stack item of a binary node with rows {min, left_first}, {max, count}:
 // the pair of an interior node's children, kLeafBit | first triangle record
 // of a leaf, or kEmptyLeaf (count 0, only in user-supplied trees: pushed like
@@ -477,10 +499,16 @@ CT_DEV uint32_t item2(float4 lo, float4 hi) {
 // the two children, which are adjacent; reading what a child is from its own
 // rows here makes a step one dependent load (fetching the popped node first
 // and then its children was two).
-CT_DEV bool node2_step(const float4 (&n)[7], f3 o, f3 inv, LaneStack& st, uint32_t& next) {
+CT_DEV bool node2_step(const float4 (&n)[7], f3 o, f3 inv, bool fast, LaneStack& st, uint32_t& next) {
     float n1, n2;
-    const bool hl = box2(n[0], n[1], o, inv, n1);
-    const bool hr = box2(n[2], n[3], o, inv, n2);
+    bool hl, hr;
+    if (fast) {
+        hl = box2_fast(n[0], n[1], o, inv, n1);
+        hr = box2_fast(n[2], n[3], o, inv, n2);
+    } else {
+        hl = box2(n[0], n[1], o, inv, n1);
+        hr = box2(n[2], n[3], o, inv, n2);
+    }
     const bool left_first = !(hl && hr) || (n1 < n2);
     const uint32_t l = item2(n[0], n[1]), r = item2(n[2], n[3]);
     const uint32_t a = left_first ? l : r, b = left_first ? r : l;
@@ -654,7 +682,7 @@ CT_DEV bool trav_step(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool fa
         } else if constexpr (ACCEL == 8) {
             pop = !fnode8_step(sort, n, o, inv, t, st, cur);
         } else {
-            pop = !node2_step(n, o, inv, st, cur);
+            pop = !node2_step(n, o, inv, fast, st, cur);
         }
     }
     if (pop) {
@@ -693,6 +721,15 @@ CT_DEV void load_item(const DevScene& sc, uint32_t cur, float4 (&n)[7], int& kin
     __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
+// Whether a ray takes its tree's fast node test.
+template <int ACCEL>
+CT_DEV bool ray_is_fast(const DevScene& sc, f3 o, f3 inv) {
+    if constexpr (ACCEL == 4) return fast_ray(o, inv, sc.plane_flags);
+    else if constexpr (ACCEL == kTreeCompact) return compact_ray(o, inv);
+    else if constexpr (ACCEL == 2) return finite_ray(o, inv, sc.plane_flags);
+    else return false;
+}
+
 // The item a ray starts at.
 template <int ACCEL>
 CT_DEV uint32_t root_item(const DevScene& sc) {
@@ -704,13 +741,14 @@ CT_DEV uint32_t root_item(const DevScene& sc) {
 // (a small launch, or the last rays of a large one), what a ray waits for is
 // its own chain of steps: some 300 instructions of one wave and a round trip
 // to memory each, with most lanes idle.  trace_quads gives each ray the four
-// lanes of a quad instead: lane c tests child c of a node, or triangle c of
-// the next four of a leaf.  The quad makes the steps of the one-lane loop
+// lanes of a quad instead: lane c tests child c of a node (of a binary tree's
+// two children, child c & 1), or triangle c of the next four of a leaf.  The quad makes the steps of the one-lane loop
 // (the same entry distances in the reference's float order, the same
 // comparators, pushes and visit order; the triangles of a leaf in order, the
 // first of equal distances kept), so the results are the same bits.  1,000
 // rays: 120 to 87 us per call; 1,048,576 rays, whose last ones took a third of
-// the launch: 0.597 to 0.511 ms; the textured atrium 6.5 to 5.9 ms.
+// the launch: 0.597 to 0.497 ms; the textured atrium 6.5 to 5.9 ms; a frame of
+// 65,536 paths through the binary tree 0.93 to 0.75 ms.
 template <int CTRL>
 CT_DEV uint32_t quad_dpp(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
@@ -721,13 +759,18 @@ CT_DEV float quad_dpp(float v) {
 }
 constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;  // quad_perm [1,0,3,2] and [2,3,0,1]
 
-// One comparator of the network on lane pairs: `low` marks the pair's first
-// lane, swaps as the reference does (if the first key is greater).
+// key with its sign flipped where `flip` is the sign bit: comparing flipped
+// keys turns a pair's second lane's view of a comparison into the first's.
+CT_DEV float flip_sign(float key, uint32_t flip) { return __uint_as_float(fbits(key) ^ flip); }
+
+// One comparator of the network on lane pairs: swaps as the reference does,
+// if the first lane's key is greater.  flip: 0 in a pair's first lane, the
+// sign bit in its second.
 template <int CTRL>
-CT_DEV void quad_comparator(bool low, bool on, float& key, uint32_t& e) {
+CT_DEV void quad_comparator(uint32_t flip, bool on, float& key, uint32_t& e) {
     const float ok = quad_dpp<CTRL>(key);
     const uint32_t oe = quad_dpp<CTRL>(e);
-    const bool sw = on && (low ? key > ok : ok > key);
+    const bool sw = (flip_sign(key, flip) > flip_sign(ok, flip)) & on;
     key = sw ? ok : key;
     e = sw ? oe : e;
 }
@@ -739,14 +782,14 @@ template <int ACCEL, class Sink>
 CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool fast, bool any, uint32_t ray,
                         uint32_t cur, float t, int prim, LaneStack& st, uint32_t* err, Sink sink) {
     const uint32_t c = lane_id() & 3u, qbase = lane_id() & 60u;
+    const uint32_t flip1 = (c & 1u) << 31, flip2 = (c & 2u) << 30;
     while (__ballot(cur != kDead) != 0) {
         if (cur == kDead) continue;
         const uint32_t idx = cur & ~kLeafBit;
+        // a triangle's rows; a binary child's rows; a quad child's six planes
+        // (a, b.xy) and entry (e.z); or a compact node's grid (a), offsets
+        // (b, e.xy) and the child's entry (e.z)
         float4 a, b, e;
-        float pl[6];
-        uint32_t ent;
-        uint4 ch, cq;
-        uint2 cz;
         const bool packed = ACCEL == kTreeCompact && fast;
         if ((int)cur < 0) {
             // records past the leaf's end are read (within the array) and ignored
@@ -754,17 +797,25 @@ CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool 
             a = load_row(p);
             b = load_row(p + 16);
             e = load_row(p + 32);
+        } else if constexpr (ACCEL == 2) {
+            // lanes 0 and 2 the left child, 1 and 3 the right
+            const gptr p = (gptr)sc.nodes2 + (uint64_t)(idx + (c & 1u)) * 32u;
+            a = load_row(p);
+            b = load_row(p + 16);
         } else if (packed) {
             const uint4* n = sc.cnodes + 4 * (size_t)idx;
-            ch = n[0];
-            cq = n[1];
-            cz = *reinterpret_cast<const uint2*>(n + 2);
-            ent = reinterpret_cast<const uint32_t*>(n + 3)[c];
+            a = *reinterpret_cast<const float4*>(n);
+            b = *reinterpret_cast<const float4*>(n + 1);
+            const float2 z = *reinterpret_cast<const float2*>(n + 2);
+            e.x = z.x;
+            e.y = z.y;
+            e.z = reinterpret_cast<const float*>(n + 3)[c];
         } else {
             const float* n = reinterpret_cast<const float*>(sc.nodes4f) + 32 * (size_t)idx + c;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) pl[k] = n[4 * k];
-            ent = fbits(n[24]);
+            a = make_float4(n[0], n[4], n[8], n[12]);
+            b.x = n[16];
+            b.y = n[20];
+            e.z = n[24];
         }
         int kind = (int)cur;
         __asm__ volatile("" : "+v"(kind));
@@ -774,28 +825,51 @@ CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool 
             const uint32_t w = fbits(a.w);
             const uint32_t last = (uint32_t)(__ballot((w & kLastInLeaf) != 0u) >> qbase) & 15u;
             float tt = t;
-            const bool hit = tri_test(o, d, tt, xyz(a), xyz(b), xyz(e), eps) && (last & ((1u << c) - 1u)) == 0u;
+            const bool hit = tri_test(o, d, tt, xyz(a), xyz(b), xyz(e), eps) & ((last & ((1u << c) - 1u)) == 0u);
             tt = hit ? tt : t;
             uint32_t pp = hit ? (w & ~kLastInLeaf) : (uint32_t)prim;
             // the least distance, of equal ones the first triangle's
             const float t1 = quad_dpp<kQuadXor1>(tt);
             const uint32_t p1 = quad_dpp<kQuadXor1>(pp);
-            const bool k1 = t1 < tt || (t1 == tt && (c & 1u));
+            const bool k1 = (t1 < tt) | ((t1 == tt) & ((c & 1u) != 0u));
             tt = k1 ? t1 : tt;
             pp = k1 ? p1 : pp;
             const float t2 = quad_dpp<kQuadXor2>(tt);
             const uint32_t p2 = quad_dpp<kQuadXor2>(pp);
-            const bool k2 = t2 < tt || (t2 == tt && (c & 2u));
+            const bool k2 = (t2 < tt) | ((t2 == tt) & ((c & 2u) != 0u));
             tt = k2 ? t2 : tt;
             pp = k2 ? p2 : pp;
-            done = any && tt < t;
+            done = any & (tt < t);
             t = tt;
             prim = (int)pp;
             pop = last != 0u;
             cur += 4u;
+        } else if constexpr (ACCEL == 2) {
+            float n1;
+            bool h;
+            if (fast) h = box2_fast(a, b, o, inv, n1);
+            else h = box2(a, b, o, inv, n1);
+            const uint32_t it = item2(a, b), oi = quad_dpp<kQuadXor1>(it);
+            const float n2 = quad_dpp<kQuadXor1>(n1);
+            const uint32_t hm = (uint32_t)(__ballot(h) >> qbase) & 3u;  // bit 0: left, bit 1: right
+            const uint32_t il = flip1 ? oi : it, ir = flip1 ? it : oi;
+            // both hit: the strictly nearer is pushed, the other is next
+            const bool near_left = flip_sign(n1, flip1) < flip_sign(n2, flip1);
+            pop = hm == 0u;
+            if (hm == 3u) {
+                if (c == 0u) st.put(st.top, near_left ? il : ir);
+                st.top += st.stride4;
+                cur = near_left ? ir : il;
+            } else if (!pop) {
+                cur = (hm & 1u) ? il : ir;
+            }
+            if (!pop && st.top >= st.max_end) st.overflow = true;
         } else {
             float mn, mx;
+            const uint32_t ent = fbits(e.z);
             if (packed) {
+                const uint4 ch = ubits4(a), cq = ubits4(b);
+                const uint2 cz = make_uint2(fbits(e.x), fbits(e.y));
                 const uint32_t sh = 8u * c;
                 const float ax = __uint_as_float((ch.w & 0xFFu) << 23) * inv.x;
                 const float ay = __uint_as_float(((ch.w >> 8) & 0xFFu) << 23) * inv.y;
@@ -808,17 +882,26 @@ CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool 
                 mn = fmaxf(fmaxf(fminf(lx, hx), fminf(ly, hy)), fminf(lz, hz));
                 mx = fminf(fminf(fmaxf(lx, hx), fmaxf(ly, hy)), fmaxf(lz, hz));
             } else {
-                const float ax = (pl[0] - o.x) * inv.x, bx = (pl[1] - o.x) * inv.x;
-                const float ay = (pl[2] - o.y) * inv.y, by = (pl[3] - o.y) * inv.y;
-                const float az = (pl[4] - o.z) * inv.z, bz = (pl[5] - o.z) * inv.z;
-                mn = gmax(gmax(gmin(ax, bx), gmin(ay, by)), gmin(az, bz));
-                mx = gmin(gmin(gmax(ax, bx), gmax(ay, by)), gmax(az, bz));
+                const float ax = (a.x - o.x) * inv.x, bx = (a.y - o.x) * inv.x;
+                const float ay = (a.z - o.y) * inv.y, by = (a.w - o.y) * inv.y;
+                const float az = (b.x - o.z) * inv.z, bz = (b.y - o.z) * inv.z;
+                if (ACCEL == 4 && fast) {
+                    // node4_fast's arithmetic
+                    const float nx = fminf(ax, bx), ny = fminf(ay, by), nz = fminf(az, bz);
+                    mn = fmaxf(fmaxf(nx, ny), nz);
+                    mx = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
+                    if (mn == 0.0f) mn = gmax(gmax(nx, ny), nz);
+                } else {
+                    mn = gmax(gmax(gmin(ax, bx), gmin(ay, by)), gmin(az, bz));
+                    mx = gmin(gmin(gmax(ax, bx), gmax(ay, by)), gmax(az, bz));
+                }
             }
             float key = tag(mn, c);
-            uint32_t x = (mx > 0.0f && key <= mx && key < t) ? ent : kNoEntry;
-            quad_comparator<kQuadXor1>((c & 1u) == 0u, true, key, x);     // (0,1) (2,3)
-            quad_comparator<kQuadXor2>((c & 2u) == 0u, true, key, x);     // (0,2) (1,3)
-            quad_comparator<kQuadXor1>((c & 1u) == 0u, c >= 2u, key, x);  // (2,3)
+            uint32_t x = ((mx > 0.0f) & (key <= mx) & (key < t)) ? ent : kNoEntry;
+            quad_comparator<kQuadXor1>(flip1, true, key, x);  // (0,1) (2,3)
+            quad_comparator<kQuadXor2>(flip2, true, key, x);  // (0,2) (1,3)
+            // (2,3), which swaps only where a key is NaN (see node4_fast)
+            if (!fast) quad_comparator<kQuadXor1>(flip1, c >= 2u, key, x);
             // the lane holds sorted position c: positions 3, 2, 1, 0 are
             // pushed in this order, the last stays as the next item
             const uint32_t vm = (uint32_t)(__ballot(x != kNoEntry) >> qbase) & 15u;
@@ -835,6 +918,12 @@ CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool 
         if (pop) {
             if (st.empty()) done = true;
             else cur = st.top_pop();
+        }
+        if constexpr (ACCEL == 2) {
+            while (!done && cur == kEmptyLeaf) {
+                if (st.empty()) done = true;
+                else cur = st.top_pop();
+            }
         }
         if (done || st.overflow) {
             if (c == 0u) {
@@ -879,7 +968,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
     fe.range = (int)(blockIdx.x % kFetchRanges);
     fe.left = gridDim.x < (uint32_t)kFetchRanges ? kFetchRanges - 1 : 0;
     fe.open();
-    constexpr bool kQuads = (ACCEL == 4 || ACCEL == kTreeCompact) && !COUNT;
+    constexpr bool kQuads = ACCEL != 8 && !COUNT;
     if constexpr (kQuads) {
         // a small launch: the range's rays shared out evenly over its waves,
         // at most 16 each, without claims
@@ -893,9 +982,13 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
                 ray = (MODE == kDual && any) ? fe.lo2 + (v - fe.nfirst) : fe.lo + v;
                 src(ray, any, o, d, t);
                 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-                fast = ACCEL == kTreeCompact && compact_ray(o, inv);
+                fast = ray_is_fast<ACCEL>(sc, o, inv);
                 st.top = 4u * (threadIdx.x & ~3u);
-                cur = 0u;
+                cur = root_item<ACCEL>(sc);
+                if (ACCEL == 2 && cur == kEmptyLeaf) {  // a tree without triangles
+                    if ((lane_id() & 3u) == 0u) sink(ray, any, t, prim);
+                    cur = kDead;
+                }
             }
             trace_quads<ACCEL>(sc, eps, o, d, inv, fast, any, ray, cur, t, prim, st, err, sink);
             return;
@@ -924,7 +1017,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
             // the ray loaded in the previous step
             prim = -1;
             inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-            fast = (ACCEL == 4 && fast_ray(o, inv, sc.plane_flags)) || (ACCEL == kTreeCompact && compact_ray(o, inv));
+            fast = ray_is_fast<ACCEL>(sc, o, inv);
             st.reset();
             isnew = 0u;
             cur = root_item<ACCEL>(sc);
@@ -993,8 +1086,7 @@ template <int ACCEL>
 CT_DEV int trace_single(const DevScene& sc, float eps, f3 o, f3 d, float& t, bool any, LaneStack& st,
                         uint32_t* err) {
     const f3 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    const bool fast = (ACCEL == 4 && fast_ray(o, inv, sc.plane_flags)) ||
-                      (ACCEL == kTreeCompact && compact_ray(o, inv));
+    const bool fast = ray_is_fast<ACCEL>(sc, o, inv);
     int prim = -1;
     uint32_t cur = root_item<ACCEL>(sc);
     TravCount cnt{0u, 0u, 0u, 0u};

@@ -338,55 +338,53 @@ int upload_shading(ct_ctx* c, const Shading& sh, ctd::DevScene& sc) {
     return r;
 }
 
-// The fast node test's copy of the uploaded quad tree (sc.nodes4f), its
-// compact layout (sc.cnodes, 64 bytes per node) and the tree's flags
-// (sc.plane_flags): the fast test needs planes that are not NaN, empty slots
-// whose child is 0xFFFFFFFF, and origins without +0 components only where
-// some plane is -0; the compact traversal needs every node encoded.
-int prepare_quad(ct_ctx* c, ctd::DevScene& sc) {
+// What the traversals need of the uploaded trees: the fast node test's copy
+// of the quad tree (sc.nodes4f), its compact layout (sc.cnodes, 64 bytes per
+// node), the trees' flags (sc.plane_flags: the fast tests need planes that
+// are not NaN, origins without +0 components only where some plane is -0, the
+// binary one's finite planes; the compact traversal needs every node encoded)
+// and the binary root's traversal item (sc.root2; item2 in
+// device/traverse.h): its children's index, kLeafBit | first triangle
+// record, or 0xFFFFFFFE for an empty leaf.
+int prepare_trees(ct_ctx* c, ctd::DevScene& sc) {
     sc.plane_flags = 0;
     sc.nodes4f = nullptr;
     sc.cnodes = nullptr;
-    if (!sc.nodes4 || sc.n_nodes4 == 0) return CT_OK;
-    void* fast = nullptr;
-    int r = dalloc(c, &fast, (size_t)sc.n_nodes4 * sizeof(ct_mbvh_node), "fast quad nodes");
-    if (r != CT_OK) return r;
-    c->scene_bufs.push_back(fast);
-    void* compact = nullptr;
-    r = dalloc(c, &compact, (size_t)sc.n_nodes4 * 64, "compact quad nodes");
-    if (r != CT_OK) return r;
-    c->scene_bufs.push_back(compact);
+    sc.root2 = 0;
+    const bool quad = sc.nodes4 && sc.n_nodes4 != 0, binary = sc.nodes2 && sc.n_nodes2 != 0;
+    void *fast = nullptr, *compact = nullptr;
+    if (quad) {
+        int r = dalloc(c, &fast, (size_t)sc.n_nodes4 * sizeof(ct_mbvh_node), "fast quad nodes");
+        if (r != CT_OK) return r;
+        c->scene_bufs.push_back(fast);
+        r = dalloc(c, &compact, (size_t)sc.n_nodes4 * 64, "compact quad nodes");
+        if (r != CT_OK) return r;
+        c->scene_bufs.push_back(compact);
+    }
     uint32_t* d = nullptr;
-    HIPCHK(hipMalloc(&d, sizeof(uint32_t)), "quad tree flags");
+    HIPCHK(hipMalloc(&d, sizeof(uint32_t)), "tree flags");
+    // on the lane's stream: the null stream would take a hardware queue, and
+    // with it gone a later context's two lanes ran at the speed of one (the
+    // 1080p atrium frame 4.80 against 3.65 ms)
     const hipStream_t s = c->ln[0].stream;
     uint32_t h = 0;
+    ct_bvh_node root{};
     hipError_t e = hipMemsetAsync(d, 0, sizeof(uint32_t), s);
-    if (e == hipSuccess) e = ctk::launch_prepare_quad(sc.nodes4, sc.n_nodes4, reinterpret_cast<float4*>(fast),
-                                                           static_cast<uint4*>(compact), d, s);
+    if (e == hipSuccess && quad)
+        e = ctk::launch_prepare_quad(sc.nodes4, sc.n_nodes4, reinterpret_cast<float4*>(fast),
+                                     static_cast<uint4*>(compact), d, s);
+    if (e == hipSuccess && binary) e = ctk::launch_prepare_binary(sc.nodes2, sc.n_nodes2, d, s);
+    if (e == hipSuccess && binary) e = hipMemcpyAsync(&root, sc.nodes2, sizeof(root), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipMemcpyAsync(&h, d, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     (void)hipFree(d);
-    if (e != hipSuccess) return ctr::hip_fail(c, e, "quad tree flags");
+    if (e != hipSuccess) return ctr::hip_fail(c, e, "tree flags");
     sc.nodes4f = reinterpret_cast<const float4*>(fast);
     sc.cnodes = static_cast<const uint4*>(compact);
     sc.plane_flags = h;
-    return CT_OK;
-}
-
-// The binary root's traversal item (sc.root2; item2 in device/traverse.h):
-// its children's index, kLeafBit | first triangle record, or 0xFFFFFFFE for
-// an empty leaf.
-int prepare_binary(ct_ctx* c, ctd::DevScene& sc) {
-    sc.root2 = 0;
-    if (!sc.nodes2 || sc.n_nodes2 == 0) return CT_OK;
-    ct_bvh_node n;
-    // on the lane's stream: the null stream would take a hardware queue, and
-    // with it gone a later context's two lanes can share one (C2 frame 3.65
-    // against 4.80 ms)
-    const hipStream_t s = c->ln[0].stream;
-    HIPCHK(hipMemcpyAsync(&n, sc.nodes2, sizeof(n), hipMemcpyDeviceToHost, s), "binary root");
-    HIPCHK(hipStreamSynchronize(s), "binary root");
-    sc.root2 = n.count < 0 ? (uint32_t)n.left_first : (n.count > 0 ? ctd::kLeafBit | (uint32_t)n.left_first : 0xFFFFFFFEu);
+    if (binary)
+        sc.root2 = root.count < 0 ? (uint32_t)root.left_first
+                                  : (root.count > 0 ? ctd::kLeafBit | (uint32_t)root.left_first : 0xFFFFFFFEu);
     return CT_OK;
 }
 
@@ -495,7 +493,7 @@ int ct_scene_upload(ct_ctx* c, const ct_scene_view* v) {
     sc.n_nodes4 = v->n_mbvh_nodes;
     sc.n_nodes2 = v->n_bvh_nodes;
     sc.n_fnodes = (uint32_t)(fn.size() / ct::kWideNodeWords);
-    if ((r = prepare_quad(c, sc)) != CT_OK || (r = prepare_binary(c, sc)) != CT_OK) { free_scene(c); return r; }
+    if ((r = prepare_trees(c, sc)) != CT_OK) { free_scene(c); return r; }
     install_scene(c, v, sc, sh, wide_bound);
     return CT_OK;
 }
@@ -552,7 +550,7 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     if (r != CT_OK) { free_scene(c); return r; }
     HIPCHK(hipStreamSynchronize(c->ln[0].stream), "scene upload");
     tmp.release();
-    if ((r = prepare_quad(c, sc)) != CT_OK || (r = prepare_binary(c, sc)) != CT_OK) { free_scene(c); return r; }
+    if ((r = prepare_trees(c, sc)) != CT_OK) { free_scene(c); return r; }
     install_scene(c, v, sc, sh, wide_bound);
     bs.total_ms = (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (st) *st = bs;

@@ -72,8 +72,8 @@ def _binary_tree(nodes):
     return b.view(np.uint8).ravel()
 
 
-@pytest.mark.parametrize("tree", ["empty_leaf_left", "empty_leaf_right", "leaf_root", "empty_root"])
-def test_binary_trees_with_odd_leaves(ct, orc, gpu_ctx, tree):
+@pytest.mark.parametrize("tree", ["empty_leaf_left", "empty_leaf_right", "leaf_root", "empty_root", "infinite_box"])
+def test_odd_binary_trees(ct, orc, gpu_ctx, tree):
     arrays = chain_scene(ct, 3, seed=6)
     n = len(arrays["prim_indices"])
     # an interior root has its children at 2 and 3, node 1 is padding
@@ -82,7 +82,10 @@ def test_binary_trees_with_odd_leaves(ct, orc, gpu_ctx, tree):
         "empty_leaf_right": [(2, -1), (0, 0), (0, n), (3, 0)],
         "leaf_root": [(0, n)],
         "empty_root": [(0, 0)],
+        "infinite_box": [(2, -1), (0, 0), (4, -1), (0, 2), (2, 2), (4, n - 4)],
     }[tree])
+    if tree == "infinite_box":  # of an interior node: 0 * inf for the axis-parallel rays
+        arrays["bvh"].view(np.float32).reshape(-1, 8)[2, [0, 5]] = -np.inf, np.inf
     arrays["mbvh"] = np.zeros(0, np.uint8)
     gpu_ctx.upload_view(ArrayView(ct, arrays).view)
     osc = orc.Scene(arrays, build=False)
@@ -90,4 +93,5 @@ def test_binary_trees_with_odd_leaves(ct, orc, gpu_ctx, tree):
     opts = ct.default_opts()
     opts.accel = ct.ACCEL_BVH2
     o, d = chain_rays(1000, 9)
+    d[::5] = [1.0, 0.0, 0.0]
     _same(gpu_ctx, osc, o, d, np.full(1000, 40.0, np.float32), opts, 0)
