@@ -10,7 +10,7 @@ render identical frames.
 
 roofline: the traversal kernel k_trace (one launch per bounce b traces the
 extension rays of bounce b and the shadow rays of bounce b - 1; with
-roulette, k_tail traces and shades the bounces from rr_start on).  Algorithmic
+roulette, k_paths traces and shades the bounces from rr_start on).  Algorithmic
 bytes per closest-hit ray = 28 (origin, direction, tmax) + 8 (t, id) + 64 *
 quad-node tests + 36 * triangle tests, per shadow ray 48 + 64 * node tests +
 36 * triangle tests; node and triangle tests are counted by an instrumented,
@@ -237,7 +237,7 @@ def trace_roofline(ctx, cam, opts, tm: dict, config: int, traversal: str) -> dic
     and triangle test counts) against three times: the summed durations of
     the launches that trace the timed frames' rays, the same launches in a
     serial frame (each alone on the device), and the frame wall time.  With
-    roulette, the bounces from rr_start on are traced inside k_tail, which
+    roulette, the bounces from rr_start on are traced inside k_paths, which
     also shades them: its whole duration counts as traversal time, so the
     first two figures are lower bounds there."""
     cst, work = ctx.trace_frame_counted(cam, opts)  # the same frame: identical counts (deterministic)
@@ -249,7 +249,7 @@ def trace_roofline(ctx, cam, opts, tm: dict, config: int, traversal: str) -> dic
     launches = tm["launches"] / steps
     trace_ms = (tm["stage_ms"]["trace"] + tm["stage_ms"]["trace_last_shadow"]) / steps
     tail_ms = tm["stage_ms"]["tail"] / steps
-    tail_launches = tm["chunks"] / steps if tail_ms > 0 else 0  # one k_tail launch per chunk
+    tail_launches = tm["chunks"] / steps if tail_ms > 0 else 0  # one k_paths launch per chunk
     bytes_per_launch = bytes_frame / max(launches + tail_launches, 1)
     mean_launch_ms = (trace_ms + tail_ms) / max(launches + tail_launches, 1)
     achieved = bytes_per_launch / (mean_launch_ms * 1e-3) / 1e9
@@ -258,7 +258,7 @@ def trace_roofline(ctx, cam, opts, tm: dict, config: int, traversal: str) -> dic
     dev = bytes_frame / (tm["ms_per_step"] * 1e-3) / 1e9
     out = {
         "kernel": "k_trace (closest hit of bounce b + any hit of bounce b-1, quad BVH)" +
-                  ("; k_tail from bounce rr_start" if tail_ms > 0 else ""),
+                  ("; k_paths from bounce rr_start" if tail_ms > 0 else ""),
         "bound": "hbm",
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,
@@ -267,7 +267,7 @@ def trace_roofline(ctx, cam, opts, tm: dict, config: int, traversal: str) -> dic
         "traffic": measured_traffic(config, traversal),
         "label": "per launch: algorithmic traversal bytes per traversal launch / the launches' mean duration "
                  "over the timed frames (two chunks in flight, so launches share the device)" +
-                 ("; the launches are k_trace's and one k_tail per chunk, whose whole duration counts (it also "
+                 ("; the launches are k_trace's and one k_paths per chunk, whose whole duration counts (it also "
                   "shades): a lower bound" if tail_ms > 0 else ""),
         "bytes_per_launch": int(bytes_per_launch),
         "mean_launch_ms": round(mean_launch_ms, 4),

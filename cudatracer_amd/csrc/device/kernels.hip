@@ -66,31 +66,38 @@ __global__ void k_setup_rays(uint32_t* counters, uint32_t* err, uint32_t n) {
 
 // ------------------------------------------------------------- generate --
 // generatePrimaryRays + Ray::generate (Kernel.cu:208-234, Ray.cuh:53-61,85-95)
+CT_DEV void primary_ray(const ViewDesc* __restrict__ views, const Segment* __restrict__ segs, int nseg, uint32_t i,
+                        f3& org, f3& dir) {
+    const Segment sg = segs[find_seg(segs, nseg, i)];
+    const ViewDesc& v = views[sg.view];
+    const uint32_t local = sg.first_path + (i - sg.chunk_offset);
+    const uint32_t spp = (uint32_t)v.spp;
+    const uint32_t ord = local / spp;
+    const uint32_t frame = v.frame_base + (local - ord * spp);
+    const uint32_t pixel = pixel_of(ord, (uint32_t)v.width, (uint32_t)v.height, v.strip_mul);
+    const uint32_t x = pixel % (uint32_t)v.width, y = pixel / (uint32_t)v.width;
+    uint32_t seed = ct_primary_seed(pixel, frame);
+    const float jx = ct_rand_float(&seed);
+    const float jy = ct_rand_float(&seed);
+    const float px = (float)x + jx - 0.5f;
+    const float py = (float)y + jy - 0.5f;
+    const float sx = 2.0f * (px * v.invw) - 1.0f;
+    const float sy = 1.0f - 2.0f * (py * v.invh);
+    const f3 w = mk3(v.w[0], v.w[1], v.w[2]);
+    const f3 hor = mk3(v.hor[0], v.hor[1], v.hor[2]);
+    const f3 ver = mk3(v.ver[0], v.ver[1], v.ver[2]);
+    dir = normalize(w + hor * sx + ver * sy);
+    org = mk3(v.pos[0], v.pos[1], v.pos[2]);
+}
+
 __global__ void k_generate(const ViewDesc* __restrict__ views, const Segment* __restrict__ segs,
                            const ChunkHdr* hdr, Queues q) {
     const uint32_t n = hdr->n;
     const int nseg = (int)hdr->nseg;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const Segment sg = segs[find_seg(segs, nseg, i)];
-        const ViewDesc& v = views[sg.view];
-        const uint32_t local = sg.first_path + (i - sg.chunk_offset);
-        const uint32_t spp = (uint32_t)v.spp;
-        const uint32_t ord = local / spp;
-        const uint32_t frame = v.frame_base + (local - ord * spp);
-        const uint32_t pixel = pixel_of(ord, (uint32_t)v.width, (uint32_t)v.height, v.strip_mul);
-        const uint32_t x = pixel % (uint32_t)v.width, y = pixel / (uint32_t)v.width;
-        uint32_t seed = ct_primary_seed(pixel, frame);
-        const float jx = ct_rand_float(&seed);
-        const float jy = ct_rand_float(&seed);
-        const float px = (float)x + jx - 0.5f;
-        const float py = (float)y + jy - 0.5f;
-        const float sx = 2.0f * (px * v.invw) - 1.0f;
-        const float sy = 1.0f - 2.0f * (py * v.invh);
-        const f3 w = mk3(v.w[0], v.w[1], v.w[2]);
-        const f3 hor = mk3(v.hor[0], v.hor[1], v.hor[2]);
-        const f3 ver = mk3(v.ver[0], v.ver[1], v.ver[2]);
-        const f3 d = normalize(w + hor * sx + ver * sy);
-        q.ray_o[0][i] = make_float4(v.pos[0], v.pos[1], v.pos[2], 0.0f);
+        f3 o, d;
+        primary_ray(views, segs, nseg, i, o, d);
+        q.ray_o[0][i] = make_float4(o.x, o.y, o.z, 0.0f);
         q.ray_d[0][i] = make_float4(d.x, d.y, d.z, 0.0f);
         q.thr[0][i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
         q.path[0][i] = i | (LT_SPECULAR << 30);
@@ -291,7 +298,7 @@ CT_DEV void block_append2(bool pe, bool ps, uint32_t* ce, uint32_t* cs, uint32_t
 // slot `slot` at `bounce`, with throughput thr, the last bounce's pdf and
 // type.  Out: the hit's radiance term (add, when contrib), the light
 // sample's shadow ray (push_sh) and the continuation ray (push_ext).  k_shade
-// and k_tail both shade through it.
+// and k_paths both shade through it.
 struct ShadeOut {
     f3 add, s_o, s_d, s_c, e_o, e_d, e_thr;
     float s_tmax, e_pdf;
@@ -592,124 +599,143 @@ k_shade(DevScene sc, ShadeOpts so, const ViewDesc* __restrict__ views, const Seg
     }
 }
 
-// ----------------------------------------------------------------- tail --
-// A chunk's roulette tail in one launch.  Once roulette has thinned the
-// paths, a bounce's trace and shade launches hold few rays each and last as
-// long as their slowest ray, plus a dependent-launch gap each.  From bounce
-// b0 on, k_tail instead gives each pair of lanes one path of bounce b0's
-// extension queue (its hit already traced by trace(b0)) and runs the path's
-// remaining bounces itself: the even lane shades (shade_one), then traces
-// the continuation ray while the odd lane traces the light sample's shadow
-// ray, both in one trace_single loop, so a bounce costs the longer of the
-// two traversals rather than their sum.  Per path the steps and their
-// arithmetic are those of the queue pipeline, so the results are the same;
-// the radiance terms are added in the same order (bounce b0 - 2's and
-// b0 - 1's pairs first, which shade(b0) and shade(b0 + 1) would fold, then
-// each bounce's shade term and light sample in turn), and the path's sum is
-// marked fully folded for k_resolve.  The rays it traces are counted in
-// cnt_tail_ext / cnt_tail_shadow.  Both lanes of a pair make the same loop
-// decisions (exchanged with lane shuffles), so each shuffle reads an active
-// partner.
-template <int ACCEL>
-__global__ void __launch_bounds__(1024)
-k_tail(DevScene sc, TraceOpts to, ShadeOpts so, const ViewDesc* __restrict__ views, const Segment* __restrict__ segs,
-       const ChunkHdr* hdr, Queues q, int sel, int bounce0, int lds_depth) {
+// ---------------------------------------------------------------- paths --
+// Whole paths in one launch, G lanes a path, from the primary ray (FIRST) or
+// from bounce0's extension queue, whose hits trace(bounce0) has found.  All
+// lanes of a group shade the same hit (the same loads, so the same lines),
+// then one half traces the continuation ray while the other traces the light
+// sample's shadow ray: a quad each (G = 8, trace_quads) or a lane each (G = 2,
+// trace_single).  Per path the steps and their arithmetic are those of the
+// queue pipeline, so the results are the same; the radiance terms are added
+// in the same order (first the pairs of the two bounces before bounce0, which
+// shade(bounce0) and shade(bounce0 + 1) would fold, then each bounce's shade
+// term and light sample in turn), and the path's sum is marked fully folded
+// for k_resolve.  The rays it traces are counted in cnt_tail_ext /
+// cnt_tail_shadow.  The lanes of a group make the same loop decisions, so the
+// shuffles read active partners; a group takes its next path as soon as its
+// own has ended.
+//
+// When a chunk's paths are few, the pipeline's launches last as long as their
+// longest rays, one after the other with a launch gap each, while a path on
+// its own needs the sum of its own rays.  Used for
+//  - small workloads, with eight lanes while each path can have them at once,
+//    and with two while each path can (launch_paths); five waves per SIMD for
+//    eight lanes (four and six were up to 8% slower at 49,284 paths);
+//  - a chunk's bounces from rr_start on, once roulette has thinned its paths,
+//    with two (the 4K displaced frame is 0.5% slower with eight).
+// Frame times in us of the pipeline / two / eight lanes:
+//   paths                    3,072          32,761         65,536          131,044
+//   box, binary tree, 4   442 565 342    585 498 410    664 515 670     781 607 1093
+//   box, quad tree, 8     489 584 328    694 561 417    802 564 624     953 706 1172
+//   atrium, quad tree, 8  488 540 333    658 551 407    692 536 687     810 678 1095
+template <int ACCEL, int G, bool FIRST>
+__global__ void __attribute__((amdgpu_waves_per_eu(G == 8 ? 5 : 4)))
+k_paths(DevScene sc, TraceOpts to, ShadeOpts so, const ViewDesc* __restrict__ views, const Segment* __restrict__ segs,
+        const ChunkHdr* hdr, Queues q, int sel, int bounce0, int lds_depth) {
     LaneStack st = make_stack(q, lds_depth);
-    const uint32_t n = *cnt_active(q.counters, bounce0);
+    const uint32_t n = FIRST ? hdr->n : *cnt_active(q.counters, bounce0);
     const int nseg = (int)hdr->nseg;
     const uint32_t gen = hdr->gen;
-    const bool shader = (__lane_id() & 1u) == 0u;  // the even lane of a pair
-    const int partner = (int)(__lane_id() ^ 1u);
+    constexpr uint32_t kHalf = G / 2;
+    const bool second = (__lane_id() & kHalf) != 0u;  // the shadow ray's half
+    const bool lead = (__lane_id() & (uint32_t)(G - 1)) == 0u;
     uint32_t n_ext = 0, n_sh = 0;
-    const uint32_t pairs = (gridDim.x * blockDim.x) / 2u;
-    for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / 2u; i < n; i += pairs) {
-        uint32_t slot = 0, type = 0;
-        float4 L = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        f3 org = mk3(0, 0, 0), dir = mk3(0, 0, 0), thr = mk3(0, 0, 0);
-        float pdf = 0.0f, t = 0.0f;
-        int prim = -1;
-        if (shader) {
-            const float4 o4 = q.ray_o[sel][i], d4 = q.ray_d[sel][i], th4 = q.thr[sel][i];
-            const uint32_t pw = q.path[sel][i];
-            const float2 h = q.hit[i];
-            slot = pw & kSlotMask;
-            type = pw >> 30;
-            L = q.lpath[slot];
-            for (int b = bounce0 - 2; b < bounce0; ++b) {
-                if (b < 0) continue;
-                const uint32_t stamp = term_stamp(gen, b);
-                const float4 e = q.ebuf[b & 1][slot], nn = q.nbuf[b & 1][slot];
-                if (__float_as_uint(e.w) == stamp) add_term(L, e);
-                if (__float_as_uint(nn.w) == stamp) add_term(L, nn);
-            }
-            org = xyz(o4);
-            dir = xyz(d4);
-            thr = xyz(th4);
-            pdf = th4.w;
-            t = h.x;
-            prim = __float_as_int(h.y);
-        }
-        for (int b = bounce0;; ++b) {
-            // zeroed: the odd lane's copy is only read through the shuffles
-            ShadeOut sh{};
-            if (shader) {
-                shade_one(sc, so, views, segs, nseg, b, slot, type, org, dir, thr, pdf, t, prim, sh);
-                if (sh.contrib) add_term(L, term(sh.add, 0u));
-            }
-            // the shadow ray to the odd lane; the even lane traces the
-            // continuation, the odd lane the shadow ray, in one loop
-            const float sx = __shfl(sh.s_o.x, partner), sy = __shfl(sh.s_o.y, partner),
-                        sz = __shfl(sh.s_o.z, partner);
-            const float dx = __shfl(sh.s_d.x, partner), dy = __shfl(sh.s_d.y, partner),
-                        dz = __shfl(sh.s_d.z, partner);
-            const float tmax = __shfl(sh.s_tmax, partner);
-            const bool has_sh = __shfl((int)sh.push_sh, partner) != 0;
-            f3 ro, rd;
-            float rt;
-            bool go;
-            if (shader) {
-                ro = sh.e_o;
-                rd = sh.e_d;
-                rt = 1e34f;
-                go = sh.push_ext;
+    const uint32_t groups = (gridDim.x * blockDim.x) / (uint32_t)G;
+    uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / (uint32_t)G;
+    uint32_t slot = 0, type = 0;
+    float4 L = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    f3 org = mk3(0, 0, 0), dir = mk3(0, 0, 0), thr = mk3(0, 0, 0);
+    float pdf = 0.0f, t = 0.0f;
+    int prim = -1, b = bounce0;
+    bool fresh = true;  // the group takes a new path
+    while (i < n) {
+        ShadeOut sh{};
+        if (fresh) {
+            b = bounce0;
+            L = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (FIRST) {
+                // the primary ray is traced as a continuation ray below
+                slot = i;
+                primary_ray(views, segs, nseg, i, sh.e_o, sh.e_d);
+                sh.e_thr = mk3(1.0f, 1.0f, 1.0f);
+                sh.e_pdf = 1.0f;
+                sh.e_type = LT_SPECULAR;
+                sh.push_ext = true;
+                b = bounce0 - 1;
             } else {
-                ro = mk3(sx, sy, sz);
-                rd = mk3(dx, dy, dz);
-                rt = tmax;
-                go = has_sh;
-            }
-            int hit = -1;
-            if (go) hit = trace_single<ACCEL>(sc, to.teps, ro, rd, rt, !shader, st, q.err);
-            const int occ = __shfl(hit, partner);
-            if (shader) {
-                if (sh.push_sh) {
-                    ++n_sh;
-                    if (occ == -1) add_term(L, term(sh.s_c, 0u));
+                const float4 o4 = q.ray_o[sel][i], d4 = q.ray_d[sel][i], th4 = q.thr[sel][i];
+                const uint32_t pw = q.path[sel][i];
+                const float2 h = q.hit[i];
+                slot = pw & kSlotMask;
+                type = pw >> 30;
+                L = q.lpath[slot];
+                for (int k = bounce0 - 2; k < bounce0; ++k) {
+                    if (k < 0) continue;
+                    const uint32_t stamp = term_stamp(gen, k);
+                    const float4 e = q.ebuf[k & 1][slot], nn = q.nbuf[k & 1][slot];
+                    if (__float_as_uint(e.w) == stamp) add_term(L, e);
+                    if (__float_as_uint(nn.w) == stamp) add_term(L, nn);
                 }
-                if (sh.push_ext) {
-                    ++n_ext;
-                    org = sh.e_o;
-                    dir = sh.e_d;
-                    thr = sh.e_thr;
-                    pdf = sh.e_pdf;
-                    type = sh.e_type;
-                    t = rt;
-                    prim = hit;
-                    if (prim == -2) {
-                        t = 1e34f;
-                        prim = -1;
-                    }
-                }
+                org = xyz(o4);
+                dir = xyz(d4);
+                thr = xyz(th4);
+                pdf = th4.w;
+                t = h.x;
+                prim = __float_as_int(h.y);
             }
-            const bool more = __shfl((int)sh.push_ext, (int)(__lane_id() & ~1u)) != 0;
-            if (!more) break;
         }
-        if (shader) {
-            L.w = __uint_as_float((uint32_t)kMaxBounce);  // every term folded
-            q.lpath[slot] = L;
+        if (!(FIRST && fresh)) {
+            shade_one(sc, so, views, segs, nseg, b, slot, type, org, dir, thr, pdf, t, prim, sh);
+            if (sh.contrib) add_term(L, term(sh.add, 0u));
+        }
+        // the first quad's continuation ray, the second quad's shadow ray
+        const f3 ro = second ? sh.s_o : sh.e_o, rd = second ? sh.s_d : sh.e_d;
+        float rt = second ? sh.s_tmax : 1e34f;
+        int hit = -1;
+        const bool go = second ? sh.push_sh : sh.push_ext;
+        if constexpr (G == 8) {
+            const f3 inv = mk3(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+            uint32_t cur = go ? root_item<ACCEL>(sc) : kDead;
+            if (ACCEL == 2 && cur == kEmptyLeaf) cur = kDead;  // a tree without triangles
+            st.top = 4u * (threadIdx.x & ~3u);
+            st.overflow = false;
+            trace_quads<ACCEL>(sc, to.teps, ro, rd, inv, ray_is_fast<ACCEL>(sc, ro, inv), second, 0u, cur, rt, hit, st,
+                               q.err, [](uint32_t, bool, float, int) {});
+        } else {
+            if (go) hit = trace_single<ACCEL>(sc, to.teps, ro, rd, rt, second, st, q.err);
+        }
+        const int occ = __shfl(hit, (int)(__lane_id() | kHalf));
+        prim = __shfl(hit, (int)(__lane_id() & ~kHalf));
+        t = __shfl(rt, (int)(__lane_id() & ~kHalf));
+        if (sh.push_sh) {
+            ++n_sh;
+            if (occ == -1) add_term(L, term(sh.s_c, 0u));
+        }
+        if (sh.push_ext) {
+            if (!(FIRST && fresh)) ++n_ext;
+            org = sh.e_o;
+            dir = sh.e_d;
+            thr = sh.e_thr;
+            pdf = sh.e_pdf;
+            type = sh.e_type;
+            if (prim == -2) {
+                t = 1e34f;
+                prim = -1;
+            }
+            ++b;
+            fresh = false;
+        } else {
+            if (lead) {
+                L.w = __uint_as_float((uint32_t)kMaxBounce);  // every term folded
+                q.lpath[slot] = L;
+            }
+            i += groups;
+            fresh = true;
         }
     }
     // one atomic per wave and counter
+    n_ext = lead ? n_ext : 0u;
+    n_sh = lead ? n_sh : 0u;
     for (int off = 32; off > 0; off >>= 1) {
         n_ext += __shfl_xor(n_ext, off);
         n_sh += __shfl_xor(n_sh, off);
@@ -894,30 +920,43 @@ hipError_t launch_trace(const LaunchShape& ls, const DevScene& sc, const TraceOp
     }
     return hipGetLastError();
 }
-hipError_t launch_tail(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const ShadeOpts& so,
-                       const ViewDesc* views, const Segment* segs, const ChunkHdr* hdr, const Queues& q, int sel,
-                       int bounce0, hipStream_t s) {
+template <int G, bool FIRST>
+static hipError_t launch_paths_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const ShadeOpts& so,
+                                 const ViewDesc* views, const Segment* segs, const ChunkHdr* hdr, const Queues& q,
+                                 int sel, int bounce0, uint32_t n, hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
-    const dim3 grid(ls.tail_blocks), block(ls.block);
+    const uint32_t per_block = (uint32_t)ls.block / (uint32_t)G;
+    const uint32_t most = (uint32_t)(G == 8 ? ls.path_blocks : ls.tail_blocks);
+    const dim3 grid(std::max(1u, std::min(most, (n + per_block - 1) / per_block))), block(ls.block);
+#define CT_PATHS(TREE)                                                                                               \
+    hipLaunchKernelGGL((k_paths<TREE, G, FIRST>), grid, block, lds, s, sc, to, so, views, segs, hdr, q, sel, bounce0, \
+                       ls.lds_depth)
     switch (tree_of(to)) {
-        case 2:
-            hipLaunchKernelGGL(k_tail<2>, grid, block, lds, s, sc, to, so, views, segs, hdr, q, sel, bounce0,
-                               ls.lds_depth);
-            break;
-        case 4:
-            hipLaunchKernelGGL(k_tail<4>, grid, block, lds, s, sc, to, so, views, segs, hdr, q, sel, bounce0,
-                               ls.lds_depth);
-            break;
-        case kTreeCompact:
-            hipLaunchKernelGGL(k_tail<kTreeCompact>, grid, block, lds, s, sc, to, so, views, segs, hdr, q, sel,
-                               bounce0, ls.lds_depth);
-            break;
+        case 2: CT_PATHS(2); break;
+        case 4: CT_PATHS(4); break;
+        case kTreeCompact: CT_PATHS(kTreeCompact); break;
         default:
-            hipLaunchKernelGGL(k_tail<8>, grid, block, lds, s, sc, to, so, views, segs, hdr, q, sel, bounce0,
-                               ls.lds_depth);
+            if constexpr (G == 2) CT_PATHS(8);
+            else return hipErrorInvalidValue;  // trace_quads has no wide tree
             break;
     }
+#undef CT_PATHS
     return hipGetLastError();
+}
+hipError_t launch_tail(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const ShadeOpts& so,
+                       const ViewDesc* views, const Segment* segs, const ChunkHdr* hdr, const Queues& q, int sel,
+                       int bounce0, uint32_t n, hipStream_t s) {
+    return launch_paths_t<2, false>(ls, sc, to, so, views, segs, hdr, q, sel, bounce0, n, s);
+}
+hipError_t launch_paths(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const ShadeOpts& so,
+                        const ViewDesc* views, const Segment* segs, const ChunkHdr* hdr, const Queues& q, uint32_t n,
+                        hipStream_t s) {
+    // eight lanes a path while the grid that fits the GPU at once holds them
+    // all (40,960 paths on 256 CUs): beyond it the second generation of paths
+    // doubles the time
+    if (n <= (uint32_t)ls.path_blocks * (uint32_t)ls.block / 8u && to.traversal != CT_TRAV_FAST)
+        return launch_paths_t<8, true>(ls, sc, to, so, views, segs, hdr, q, 0, 0, n, s);
+    return launch_paths_t<2, true>(ls, sc, to, so, views, segs, hdr, q, 0, 0, n, s);
 }
 hipError_t launch_shade(const LaunchShape& ls, const DevScene& sc, const ShadeOpts& so, const ViewDesc* views,
                         const Segment* segs, const ChunkHdr* hdr, const Queues& q, int sel, int bounce,
@@ -1187,16 +1226,24 @@ bool set_trace_grids(LaunchShape& ls, int num_cus) {
     ls.grid8 = std::max(lo, ls.full8 * fill / 8);
     ls.gridc = std::max(lo, ls.fullc * fill / 8);
     ls.trace_blocks = std::max(std::max(ls.full2, ls.full4), std::max(ls.full8, ls.fullc));
-    // k_tail: the blocks of its most register-hungry tree that fit at once
-    int pt = 1 << 30;
-    for (const void* f : {reinterpret_cast<const void*>(&ctd::k_tail<2>), reinterpret_cast<const void*>(&ctd::k_tail<4>),
-                          reinterpret_cast<const void*>(&ctd::k_tail<ctd::kTreeCompact>),
-                          reinterpret_cast<const void*>(&ctd::k_tail<8>)}) {
-        int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, ls.block, lds) != hipSuccess || nb <= 0) return false;
-        pt = std::min(pt, nb);
-    }
-    ls.tail_blocks = std::min(ls.trace_blocks, std::max(1, num_cus * pt));
+    // k_paths: the blocks of its most register-hungry tree that fit at once
+    auto resident = [&](std::initializer_list<const void*> kernels, int& blocks) {
+        int least = 1 << 30;
+        for (const void* f : kernels) {
+            int nb = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, ls.block, lds) != hipSuccess || nb <= 0) return false;
+            least = std::min(least, nb);
+        }
+        blocks = std::min(ls.trace_blocks, std::max(1, num_cus * least));
+        return true;
+    };
+#define CT_K(...) reinterpret_cast<const void*>(&ctd::k_paths<__VA_ARGS__>)
+    if (!resident({CT_K(2, 2, false), CT_K(4, 2, false), CT_K(ctd::kTreeCompact, 2, false), CT_K(8, 2, false),
+                   CT_K(2, 2, true), CT_K(4, 2, true), CT_K(ctd::kTreeCompact, 2, true), CT_K(8, 2, true)},
+                  ls.tail_blocks) ||
+        !resident({CT_K(2, 8, true), CT_K(4, 8, true), CT_K(ctd::kTreeCompact, 8, true)}, ls.path_blocks))
+        return false;
+#undef CT_K
     return true;
 }
 }  // namespace ctk

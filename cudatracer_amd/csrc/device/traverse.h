@@ -775,12 +775,13 @@ CT_DEV void quad_comparator(uint32_t flip, bool on, float& key, uint32_t& e) {
     e = sw ? oe : e;
 }
 
-// The quad whose rays these are (all four lanes hold the same ray; cur ==
-// kDead: none), to their ends.  st.top: the ray's stack, in the column of one
-// of the wave's lanes.  Lane 0 of the quad gives the result to sink.
+// The quads' rays (all four lanes of a quad hold the same ray; cur == kDead:
+// none), to their ends.  st.top: the ray's stack, in the column of one of the
+// wave's lanes.  t and prim end as the ray's result (prim -1: none, -2: the
+// stack bound was exceeded); lane 0 of the quad gives it to sink as well.
 template <int ACCEL, class Sink>
 CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool fast, bool any, uint32_t ray,
-                        uint32_t cur, float t, int prim, LaneStack& st, uint32_t* err, Sink sink) {
+                        uint32_t cur, float& t, int& prim, LaneStack& st, uint32_t* err, Sink sink) {
     const uint32_t c = lane_id() & 3u, qbase = lane_id() & 60u;
     const uint32_t flip1 = (c & 1u) << 31, flip2 = (c & 2u) << 30;
     while (__ballot(cur != kDead) != 0) {
@@ -926,11 +927,9 @@ CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool 
             }
         }
         if (done || st.overflow) {
+            if (st.overflow) prim = -2;
             if (c == 0u) {
-                if (st.overflow) {
-                    atomicOr(err, 1u);
-                    prim = -2;
-                }
+                if (st.overflow) atomicOr(err, 1u);
                 sink(ray, any, t, prim);
             }
             cur = kDead;
@@ -1065,8 +1064,8 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
         const f3 qo = mk3(__shfl(o.x, sl), __shfl(o.y, sl), __shfl(o.z, sl));
         const f3 qd = mk3(__shfl(d.x, sl), __shfl(d.y, sl), __shfl(d.z, sl));
         const f3 qi = mk3(__shfl(inv.x, sl), __shfl(inv.y, sl), __shfl(inv.z, sl));
-        const float qt = __shfl(t, sl);
-        const int qp = __shfl(prim, sl);
+        float qt = __shfl(t, sl);
+        int qp = __shfl(prim, sl);
         const uint32_t qr = __shfl(ray, sl), qtop = __shfl(st.top, sl), qc = __shfl(cur, sl);
         st.top = qtop;
         st.overflow = false;
@@ -1078,7 +1077,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
 // One ray per lane, traced to its end: the step loop of trace_persistent
 // (the same node and triangle tests, pushes and visit order, so the same
 // result for the ray) for kernels whose lanes each follow a ray of their own
-// (k_tail).  t: in, the ray's extent; out, the closest hit's distance.
+// (k_paths).  t: in, the ray's extent; out, the closest hit's distance.
 // Returns the hit primitive, -1 for none, -2 when the stack bound was
 // exceeded (the error flag is raised).  any: stop at the first hit (a
 // per-lane flag, so closest-hit and any-hit lanes step together).

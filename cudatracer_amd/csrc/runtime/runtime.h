@@ -25,7 +25,7 @@ struct ChunkStats {
 #endif
 // Pipelines the chunk driver rotates through.
 constexpr int kLanes = CT_LANES;
-// The bounce from which a chunk's remaining bounces run in one k_tail
+// The bounce from which a chunk's remaining bounces run in one k_paths
 // launch (tail_bounce): with roulette, rr_start + CT_TAIL_AFTER_ROULETTE;
 // without, max_depth - CT_TAIL_BEFORE_END (0: no tail).
 #ifndef CT_TAIL_AFTER_ROULETTE
@@ -67,10 +67,11 @@ struct Lane {
     int max_depth = 0;
     bool timed = false, count = false;
     bool nee = false;  // the chunk ends with a launch for the last bounce's shadow rays
-    int tail = -1;     // the chunk's k_tail bounce, or -1
+    int tail = -1;     // the chunk's k_paths bounce, or -1
+    bool paths = false;  // the chunk runs as whole paths (k_paths)
 };
 // h_read layout (uint32 words)
-constexpr int kReadCounters = 2 * (ctd::kMaxBounce + 1) + 2;  // per-bounce counts, then k_tail's two
+constexpr int kReadCounters = 2 * (ctd::kMaxBounce + 1) + 2;  // per-bounce counts, then k_paths's two
 constexpr int kReadErr = kReadCounters;
 constexpr int kReadWork = kReadCounters + 2;  // 4 x uint64, 8-byte aligned
 constexpr int kReadWords = kReadWork + 8;

@@ -341,8 +341,8 @@ static ctd::ShadeOpts shade_opts(const ct_frame_opts& o) {
 // so every lane starts at once instead of after the host has enqueued the
 // whole of the previous lanes' chunks.  timed records an event pair around
 // every kernel.
-// The bounce from which a chunk's remaining bounces run in one k_tail
-// launch, or -1 (a counting frame: k_tail does not count node and triangle
+// The bounce from which a chunk's remaining bounces run in one k_paths
+// launch, or -1 (a counting frame: k_paths does not count node and triangle
 // tests).
 int tail_bounce(const ct_frame_opts& o, bool count) {
     if (count) return -1;
@@ -350,6 +350,15 @@ int tail_bounce(const ct_frame_opts& o, bool count) {
     if (o.rr_start >= 0) b0 = std::max(0, o.rr_start + kTailAfterRoulette);
     else if (kTailBeforeEnd > 0) b0 = std::max(0, o.max_depth - kTailBeforeEnd);
     return b0 >= 0 && b0 + 1 < o.max_depth ? b0 : -1;
+}
+
+// Whether a workload of `total` paths runs as whole paths in one launch
+// (k_paths) instead of the queue pipeline: while the GPU holds all of them at
+// once, two lanes each (131,072 paths on 256 CUs; above, the pipeline is
+// faster: 262,144 paths in two chunks 0.90 against 1.04 ms).  Not for a
+// counting frame: k_paths does not count node and triangle tests.
+static bool whole_paths(const ct_ctx* c, uint64_t total, bool count) {
+    return !count && total <= (uint64_t)c->shape.tail_blocks * (uint64_t)c->shape.block / 2u;
 }
 
 struct BounceSeq {
@@ -360,14 +369,15 @@ struct BounceSeq {
     ctd::ShadeOpts so{};
     unsigned long long* ws = nullptr;
     bool timed = false, nee = false;
-    int tail = -1;  // k_tail from this bounce on, or -1
+    int tail = -1;  // k_paths from this bounce on, or -1
+    uint32_t paths = 0;  // whole paths (k_paths): the chunk's size
     int e = 0, sel = 0;
 
     BounceSeq() = default;
-    BounceSeq(ct_ctx* c_, Lane* L_, const ct_frame_opts& o_, bool count, bool timed_)
+    BounceSeq(ct_ctx* c_, Lane* L_, const ct_frame_opts& o_, bool count, bool timed_, uint32_t paths_ = 0)
         : c(c_), L(L_), o(o_), to(trace_opts(o_)), so(shade_opts(o_)), ws(count ? L_->wstats : nullptr),
-          timed(timed_), nee(o_.shadow && c_->sc.n_lights > 0), tail(tail_bounce(o_, count)) {}
-    int steps() const { return 1 + (tail >= 0 ? tail + 1 : o.max_depth); }
+          timed(timed_), nee(o_.shadow && c_->sc.n_lights > 0), tail(tail_bounce(o_, count)), paths(paths_) {}
+    int steps() const { return paths ? 2 : 1 + (tail >= 0 ? tail + 1 : o.max_depth); }
     void rec() {
         if (timed) (void)hipEventRecord(L->ev[e++], L->stream);
     }
@@ -377,6 +387,10 @@ struct BounceSeq {
         if (k == 0) {
             rec();
             if ((r = ctk::launch_setup(L->q.counters, L->d_hdr, s)) != hipSuccess) return r;
+            if (paths) {
+                rec();
+                return hipSuccess;
+            }
             if ((r = ctk::launch_generate(c->shape, L->d_views, L->d_segs, L->d_hdr, c->lane_cap, L->q, s)) !=
                 hipSuccess)
                 return r;
@@ -386,15 +400,24 @@ struct BounceSeq {
         // trace(b): the extension rays of bounce b and the shadow rays of
         // bounce b - 1 (their radiance terms are added by shade(b + 1) or
         // resolve, in order); then shade(b) appends bounce b + 1's extension
-        // rays and bounce b's shadow rays, or, at the tail bounce, k_tail
+        // rays and bounce b's shadow rays, or, at the tail bounce, k_paths
         // runs every remaining bounce
         const int b = k - 1;
+        if (paths) {
+            rec();
+            if ((r = ctk::launch_paths(c->shape, c->sc, to, so, L->d_views, L->d_segs, L->d_hdr, L->q, paths, s)) !=
+                hipSuccess)
+                return r;
+            rec();
+            return hipSuccess;
+        }
         rec();
         if ((r = ctk::launch_trace(c->shape, c->sc, to, L->q, L->d_hdr, sel, b, ws, s)) != hipSuccess) return r;
         rec();
         rec();
         if (b == tail)
-            r = ctk::launch_tail(c->shape, c->sc, to, so, L->d_views, L->d_segs, L->d_hdr, L->q, sel, b, s);
+            r = ctk::launch_tail(c->shape, c->sc, to, so, L->d_views, L->d_segs, L->d_hdr, L->q, sel, b,
+                                 c->lane_cap, s);
         else
             r = ctk::launch_shade(c->shape, c->sc, so, L->d_views, L->d_segs, L->d_hdr, L->q, sel, b, s);
         if (r != hipSuccess) return r;
@@ -402,10 +425,14 @@ struct BounceSeq {
         sel ^= 1;
         return hipSuccess;
     }
-    // the last bounce's shadow rays (the launch has no extension rays; k_tail
+    // the last bounce's shadow rays (the launch has no extension rays; k_paths
     // traces its own)
     hipError_t finish() {
         hipError_t r;
+        if (paths) {
+            L->n_events = e;
+            return hipSuccess;
+        }
         rec();
         if (nee && tail < 0 &&
             (r = ctk::launch_trace(c->shape, c->sc, to, L->q, L->d_hdr, sel, o.max_depth, ws, L->stream)) !=
@@ -509,7 +536,7 @@ static int graph_chunk(ct_ctx* c, Lane& L, const ct_frame_opts& o) {
 }
 
 static int close_chunk(ct_ctx* c, Lane& L, uint32_t n, float4* accum, const ct_frame_opts& o, bool timed,
-                       bool count, hipEvent_t prev_resolved) {
+                       bool count, bool whole, hipEvent_t prev_resolved) {
     hipStream_t s = L.stream;
     // accumulator updates in chunk order
     if (prev_resolved) HIPCHK(hipStreamWaitEvent(s, prev_resolved, 0), "order resolves");
@@ -528,6 +555,7 @@ static int close_chunk(ct_ctx* c, Lane& L, uint32_t n, float4* accum, const ct_f
     L.max_depth = o.max_depth;
     L.nee = o.shadow && c->sc.n_lights > 0;
     L.tail = tail_bounce(o, count);
+    L.paths = whole;
     L.timed = timed;
     L.count = count;
     return CT_OK;
@@ -548,14 +576,14 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
     st->primary += cnt[0];
     for (int b = 1; b < L.max_depth; ++b) st->extension += cnt[b];
     for (int b = 0; b < L.max_depth; ++b) st->shadow += cnt[(ctd::kMaxBounce + 1) + b];
-    st->extension += cnt[2 * (ctd::kMaxBounce + 1)];  // k_tail's (cnt_tail_ext, cnt_tail_shadow)
+    st->extension += cnt[2 * (ctd::kMaxBounce + 1)];  // k_paths's (cnt_tail_ext, cnt_tail_shadow)
     st->shadow += cnt[2 * (ctd::kMaxBounce + 1) + 1];
     st->samples += L.n_paths;
     float ms = 0;
     if (hipEventElapsedTime(&ms, L.ev[kEvTotal0], L.ev[kEvTotal0 + 1]) == hipSuccess) st->total_ms += ms;
     if (L.timed) {
         // event pairs: [generate] then per bounce [trace][shade] (at the tail
-        // bounce [trace][k_tail], the last bounce the chunk launches); [trace
+        // bounce [trace][k_paths], the last bounce the chunk launches); [trace
         // of the last shadow rays]; [resolve]
         int e = 0;
         auto pair = [&](int i) {
@@ -565,7 +593,8 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
         };
         st->other_ms += pair(e);
         e += 2;
-        const int nb = L.tail >= 0 ? L.tail + 1 : L.max_depth;
+        if (L.paths) st->tail_ms += pair(e);
+        const int nb = L.paths ? 0 : (L.tail >= 0 ? L.tail + 1 : L.max_depth);
         for (int b = 0; b < nb; ++b) {
             st->extend_ms += pair(e);
             st->extend_launches += 1;
@@ -573,7 +602,7 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
             else st->shade_ms += pair(e + 2);
             e += 4;
         }
-        if (L.nee && L.tail < 0) {
+        if (L.nee && L.tail < 0 && !L.paths) {
             st->connect_ms += pair(e);
             st->extend_launches += 1;
         }
@@ -616,6 +645,7 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
     int r = ensure_paths(c, cap);
     if (r != CT_OK) return r;
     cap = std::min(cap, c->lane_cap);
+    const bool whole = whole_paths(c, total, count);
     // work queued on lane 0 by the caller (accumulator clears) comes first
     HIPCHK(hipEventRecord(c->ln[0].resolved, c->ln[0].stream), "event");
     for (int k = 1; k < kLanes; ++k) HIPCHK(hipStreamWaitEvent(c->ln[k].stream, c->ln[0].resolved, 0), "order lanes");
@@ -640,19 +670,29 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
             if ((rr = stage_chunk(c, L, views, group[i].segs, group[i].fill, group[i].tasks, count)) != CT_OK)
                 return rr;
         }
-        if (use_graph && !count && !timed) {
-            for (int i = 0; i < g; ++i)
-                if ((rr = graph_chunk(c, c->ln[(lane + i) % kLanes], o)) != CT_OK) return rr;
-        } else {
-            BounceSeq seq[kLanes];
-            for (int i = 0; i < g; ++i) seq[i] = BounceSeq(c, &c->ln[(lane + i) % kLanes], o, count, timed);
-            for (int k = 0; k < seq[0].steps(); ++k)
-                for (int i = 0; i < g; ++i) HIPCHK(seq[i].step(k), "launch chunk");
-            for (int i = 0; i < g; ++i) HIPCHK(seq[i].finish(), "launch chunk");
-        }
+        // a chunk's loop from the lane's graph, or enqueued here
+        BounceSeq seq[kLanes];
+        bool here[kLanes];
+        int steps = 0;
         for (int i = 0; i < g; ++i) {
             Lane& L = c->ln[(lane + i) % kLanes];
-            if ((rr = close_chunk(c, L, group[i].fill, accum, o, timed, count, prev)) != CT_OK) return rr;
+            here[i] = whole || !(use_graph && !count && !timed);
+            if (!here[i]) {
+                if ((rr = graph_chunk(c, L, o)) != CT_OK) return rr;
+                continue;
+            }
+            seq[i] = BounceSeq(c, &L, o, count, timed, whole ? group[i].fill : 0u);
+            steps = std::max(steps, seq[i].steps());
+        }
+        for (int k = 0; k < steps; ++k)
+            for (int i = 0; i < g; ++i)
+                if (here[i] && k < seq[i].steps()) HIPCHK(seq[i].step(k), "launch chunk");
+        for (int i = 0; i < g; ++i)
+            if (here[i]) HIPCHK(seq[i].finish(), "launch chunk");
+        for (int i = 0; i < g; ++i) {
+            Lane& L = c->ln[(lane + i) % kLanes];
+            if ((rr = close_chunk(c, L, group[i].fill, accum, o, timed, count, whole, prev)) != CT_OK)
+                return rr;
             prev = L.resolved;
             if (serial && (rr = finish_chunk(c, L, st)) != CT_OK) return rr;  // done before the next starts
         }
@@ -740,7 +780,7 @@ void ctr_apply_shape(ct_ctx* c, int block, int lds_depth) {
     c->shape.lds_depth = lds_depth;
     if (!ctk::set_trace_grids(c->shape, c->num_cus)) {
         c->shape.grid2 = c->shape.grid4 = c->shape.grid8 = c->shape.gridc = c->shape.full2 = c->shape.full4 =
-            c->shape.full8 = c->shape.fullc = c->shape.trace_blocks = c->shape.tail_blocks = std::max(8, c->num_cus * 4);
+            c->shape.full8 = c->shape.fullc = c->shape.trace_blocks = c->shape.tail_blocks = c->shape.path_blocks = std::max(8, c->num_cus * 4);
     }
     c->shape.shade_blocks = std::max(1, c->num_cus * 8);
 }

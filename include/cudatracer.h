@@ -203,11 +203,13 @@ typedef struct ct_frame_stats {
                                  plus one per chunk for the last shadow rays
                                  when NEE is on; with roulette, the bounces
                                  up to the tail's first)                      */
-    double tail_ms;           /* with roulette (rr_start >= 0): the device time of
-                                 the launches that run each chunk's remaining
-                                 bounces once roulette has thinned its paths
-                                 (a lane per path: shading, the light sample's
-                                 shadow ray and the next ray traced in turn) */
+    double tail_ms;           /* the device time of the launches that run whole paths:
+                                 with roulette (rr_start >= 0) each chunk's
+                                 remaining bounces once roulette has thinned its
+                                 paths; for a small frame (while the GPU holds all
+                                 its paths at once: 131,072 on 256 CUs) all of it,
+                                 extend_ms, shade_ms, connect_ms and
+                                 extend_launches then being 0                   */
 } ct_frame_stats;
 
 /* Fill with the reference defaults (depth 5, 1 spp, no RR, BVH4, reference BSDF,
