@@ -178,7 +178,7 @@ struct Queues {
     float4* nbuf[2];    // connect's radiance term of bounce b at [b % 2] (xyz), .w = stamp (bits)
     uint32_t* counters; // see CounterIndex
     uint32_t* spill;    // traversal stack overflow area: per block (max_stack - LDS depth) x blockDim words
-    uint32_t* err;      // error flags
+    uint32_t* err;      // error flag, in pinned host memory
     int max_stack = kMaxStack;  // traversal stack entries (LDS + spill); deeper trees report an overflow
 };
 
@@ -215,6 +215,10 @@ constexpr int kFetchBase = 192;
 static_assert(2 * (kMaxBounce + 1) + 2 <= kFetchBase, "counters overlap");
 CT_DEV uint32_t* cnt_fetch_ext(uint32_t* c, int b) { return c + kFetchBase + b; }
 CT_DEV uint32_t* cnt_fetch_sh(uint32_t* c, int b) { return c + kFetchBase + kFetchRanges * kFetchSlot + b; }
+// The words the host reads back: the per-bounce counts, then k_paths' two.
+constexpr int kReadCounters = 2 * (kMaxBounce + 1) + 2;
+// First word of the views in a chunk's staging buffer (k_stage).
+constexpr uint32_t kStageViews = 64;
 constexpr int kCounterWords = kFetchBase + 2 * kFetchRanges * kFetchSlot + 64;
 
 }  // namespace ctd

@@ -1,7 +1,7 @@
 // Wavefront path-tracing kernels for gfx950 (MI355X).
 //
 // Reference stages (src/CUDA/Kernel.cu):        here:
-//   setGlobals          :75-86                  k_setup (all bounce counters zeroed once per chunk)
+//   setGlobals          :75-86                  k_stage (all bounce counters zeroed once per chunk)
 //   generatePrimaryRays :208-234                k_generate
 //   extend              :236-245                k_trace    (persistent, wave-fetched; bounce b's
 //   connect             :247-256                            extension rays with bounce b - 1's
@@ -49,19 +49,25 @@ CT_DEV SlotInfo decode_slot(const ViewDesc* __restrict__ views, const Segment* _
 }
 
 // ---------------------------------------------------------------- setup --
-__global__ void k_setup(uint32_t* counters, const ChunkHdr* hdr) {
-    for (int i = threadIdx.x; i < kCounterWords; i += blockDim.x) counters[i] = 0u;
-    __syncthreads();
-    if (threadIdx.x == 0) *cnt_active(counters, 0) = hdr->n;
+// A chunk's start in one launch: its header and tables from the pinned staging
+// buffer (words: header at 0, views at kStageViews, segments behind them) to
+// device memory, and its counters cleared.  Three copies and a clearing kernel
+// before it were four dependent operations, some 25 us of a small frame.
+__global__ void k_stage(const uint32_t* __restrict__ stage, uint32_t view_words, uint32_t seg_words, ChunkHdr* hdr,
+                        ViewDesc* views, Segment* segs, uint32_t* counters) {
+    uint32_t* h = reinterpret_cast<uint32_t*>(hdr);
+    uint32_t* v = reinterpret_cast<uint32_t*>(views);
+    uint32_t* g = reinterpret_cast<uint32_t*>(segs);
+    for (uint32_t i = threadIdx.x; i < sizeof(ChunkHdr) / 4; i += blockDim.x) h[i] = stage[i];
+    for (uint32_t i = threadIdx.x; i < view_words; i += blockDim.x) v[i] = stage[kStageViews + i];
+    for (uint32_t i = threadIdx.x; i < seg_words; i += blockDim.x) g[i] = stage[kStageViews + view_words + i];
+    const uint32_t n = stage[0];  // ChunkHdr::n
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kCounterWords; i += blockDim.x) counters[i] = i == 0u ? n : 0u;
 }
 
-// The same for a ray-level launch of n rays, with the size as an argument
-// (no header in device memory) and the error flags cleared too.
-__global__ void k_setup_rays(uint32_t* counters, uint32_t* err, uint32_t n) {
+// The counters of a ray-level launch cleared.
+__global__ void k_setup_rays(uint32_t* counters) {
     for (int i = threadIdx.x; i < kCounterWords; i += blockDim.x) counters[i] = 0u;
-    if (threadIdx.x < 16) err[threadIdx.x] = 0u;
-    __syncthreads();
-    if (threadIdx.x == 0) *cnt_active(counters, 0) = n;
 }
 
 // ------------------------------------------------------------- generate --
@@ -109,15 +115,13 @@ __global__ void k_generate(const ViewDesc* __restrict__ views, const Segment* __
 // Persistent closest-hit over a queue of rays (see trace_persistent): the
 // ray-level entry points.
 template <int ACCEL>
-CT_DEV void extend_impl(const DevScene& sc, const TraceOpts& to, const Queues& q, int sel, int bounce,
-                        LaneStack& st) {
-    const uint32_t n = *cnt_active(q.counters, bounce);
-    const float4* __restrict__ ro = q.ray_o[sel];
-    const float4* __restrict__ rd = q.ray_d[sel];
+CT_DEV void extend_impl(const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n, LaneStack& st) {
+    const float4* __restrict__ ro = q.ray_o[0];
+    const float4* __restrict__ rd = q.ray_d[0];
     float2* hit = q.hit;
     TravCount tc{0u, 0u, 0u, 0u};
     trace_persistent<ACCEL, kClosest, false>(
-        sc, to.teps, n, 0u, cnt_fetch_ext(q.counters, bounce), st, tc, q.err,
+        sc, to.teps, n, 0u, cnt_fetch_ext(q.counters, 0), st, tc, q.err,
         [&](uint32_t i, bool, f3& o, f3& d, float& t) {
             o = xyz(ro[i]);
             d = xyz(rd[i]);
@@ -156,9 +160,9 @@ CT_DEV LaneStack make_stack(const Queues& q, int lds_depth) {
 // reaches it without spills (the counting copies spill a register).
 template <int TREE>
 __global__ void __attribute__((amdgpu_waves_per_eu(8)))
-k_extend(DevScene sc, TraceOpts to, Queues q, int sel, int bounce, int lds_depth) {
+k_extend(DevScene sc, TraceOpts to, Queues q, uint32_t n, int lds_depth) {
     LaneStack st = make_stack(q, lds_depth);
-    extend_impl<TREE>(sc, to, q, sel, bounce, st);
+    extend_impl<TREE>(sc, to, q, n, st);
 }
 
 // ---------------------------------------------------------------- trace --
@@ -772,9 +776,12 @@ CT_DEV void fold_open_terms(float4& L, const Queues& q, uint32_t s, uint32_t gen
     }
 }
 
-// accum[pixel] += per-sample radiance, samples in increasing order.
+// accum[pixel] += per-sample radiance, samples in increasing order; and the
+// chunk's ray counts, final by now, to the host's pinned words `counts`.
 __global__ void k_resolve(const ViewDesc* __restrict__ views, const Segment* __restrict__ segs,
-                          const ChunkHdr* hdr, Queues q, float4* accum) {
+                          const ChunkHdr* hdr, Queues q, float4* accum, uint32_t* counts) {
+    static_assert(kReadCounters <= 256, "one word a thread of the first block");
+    if (blockIdx.x == 0 && threadIdx.x < (uint32_t)kReadCounters) counts[threadIdx.x] = q.counters[threadIdx.x];
     const uint32_t n_tasks = hdr->n_tasks;
     const int nseg = (int)hdr->nseg;
     const uint32_t gen = hdr->gen;
@@ -844,12 +851,9 @@ namespace ctk {
 
 using namespace ctd;
 
-hipError_t launch_setup(uint32_t* counters, const ChunkHdr* hdr, hipStream_t s) {
-    hipLaunchKernelGGL(k_setup, dim3(1), dim3(256), 0, s, counters, hdr);
-    return hipGetLastError();
-}
-hipError_t launch_setup_rays(uint32_t* counters, uint32_t* err, uint32_t n, hipStream_t s) {
-    hipLaunchKernelGGL(k_setup_rays, dim3(1), dim3(256), 0, s, counters, err, n);
+hipError_t launch_stage(const uint32_t* stage, uint32_t view_words, uint32_t seg_words, ChunkHdr* hdr, ViewDesc* views,
+                        Segment* segs, uint32_t* counters, hipStream_t s) {
+    hipLaunchKernelGGL(k_stage, dim3(1), dim3(1024), 0, s, stage, view_words, seg_words, hdr, views, segs, counters);
     return hipGetLastError();
 }
 hipError_t launch_generate(const LaunchShape& ls, const ViewDesc* views, const Segment* segs,
@@ -880,12 +884,21 @@ int ray_grid(const LaunchShape& ls, int tree, uint32_t n) {
     return (int)std::min<uint64_t>((uint64_t)full_of(ls, tree), std::max<uint64_t>(need, kFetchRanges));
 }
 
+// Clears the counters of a ray-level launch, unless it is small on every fetch
+// range: trace_persistent then makes no claims (the wide tree always does).
+static hipError_t setup_rays(const LaunchShape& ls, int tree, const Queues& q, uint32_t n, hipStream_t s) {
+    const uint64_t waves = (uint64_t)(ray_grid(ls, tree, n) / kFetchRanges) * (uint64_t)(ls.block / 64);
+    if (tree != 8 && ((uint64_t)n + kFetchRanges - 1) / kFetchRanges <= waves * 16u) return hipSuccess;
+    hipLaunchKernelGGL(k_setup_rays, dim3(1), dim3(1024), 0, s, q.counters);
+    return hipGetLastError();
+}
+
 template <int TREE>
-void extend_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, int sel, int bounce,
-              uint32_t n, hipStream_t s) {
+void extend_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n,
+              hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
     const dim3 grid(ray_grid(ls, TREE, n)), block(ls.block);
-    hipLaunchKernelGGL((k_extend<TREE>), grid, block, lds, s, sc, to, q, sel, bounce, ls.lds_depth);
+    hipLaunchKernelGGL((k_extend<TREE>), grid, block, lds, s, sc, to, q, n, ls.lds_depth);
 }
 template <int TREE>
 void trace_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, const ChunkHdr* hdr,
@@ -900,13 +913,16 @@ void trace_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, con
                            wstats);
 }
 
-hipError_t launch_extend(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, int sel,
-                         int bounce, uint32_t n, hipStream_t s) {
-    switch (tree_of(to)) {
-        case 2: extend_t<2>(ls, sc, to, q, sel, bounce, n, s); break;
-        case 4: extend_t<4>(ls, sc, to, q, sel, bounce, n, s); break;
-        case kTreeCompact: extend_t<kTreeCompact>(ls, sc, to, q, sel, bounce, n, s); break;
-        default: extend_t<8>(ls, sc, to, q, sel, bounce, n, s); break;
+hipError_t launch_extend(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n,
+                         hipStream_t s) {
+    const int tree = tree_of(to);
+    const hipError_t e = setup_rays(ls, tree, q, n, s);
+    if (e != hipSuccess) return e;
+    switch (tree) {
+        case 2: extend_t<2>(ls, sc, to, q, n, s); break;
+        case 4: extend_t<4>(ls, sc, to, q, n, s); break;
+        case kTreeCompact: extend_t<kTreeCompact>(ls, sc, to, q, n, s); break;
+        default: extend_t<8>(ls, sc, to, q, n, s); break;
     }
     return hipGetLastError();
 }
@@ -970,10 +986,10 @@ hipError_t launch_shade(const LaunchShape& ls, const DevScene& sc, const ShadeOp
     return hipGetLastError();
 }
 hipError_t launch_resolve(const LaunchShape& ls, const ViewDesc* views, const Segment* segs, const ChunkHdr* hdr,
-                          uint32_t max_tasks, const Queues& q, float4* accum, hipStream_t s) {
+                          uint32_t max_tasks, const Queues& q, float4* accum, uint32_t* counts, hipStream_t s) {
     const uint32_t blocks =
         std::max<uint32_t>(1u, std::min<uint32_t>((max_tasks + 255) / 256, (uint32_t)ls.max_blocks));
-    hipLaunchKernelGGL(k_resolve, dim3(blocks), dim3(256), 0, s, views, segs, hdr, q, accum);
+    hipLaunchKernelGGL(k_resolve, dim3(blocks), dim3(256), 0, s, views, segs, hdr, q, accum, counts);
     return hipGetLastError();
 }
 // The tonemapped image as 8-bit RGBA (alpha 255): byte = clamp(v, 0, 1) * 255 + 0.5, truncated.
@@ -1182,6 +1198,8 @@ hipError_t launch_shadow_flags(const LaunchShape& ls, const DevScene& sc, const 
                                uint32_t n, uint8_t* out, hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
     const int tree = tree_of(to);
+    const hipError_t e = setup_rays(ls, tree, q, n, s);
+    if (e != hipSuccess) return e;
     const dim3 grid(ray_grid(ls, tree, n)), block(ls.block);
     if (tree == 2) hipLaunchKernelGGL(k_shadow_flags<2>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
     else if (tree == 4) hipLaunchKernelGGL(k_shadow_flags<4>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);

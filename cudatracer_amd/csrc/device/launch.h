@@ -34,15 +34,16 @@ struct LaunchShape {
 // with that shape.
 bool set_trace_grids(LaunchShape& ls, int num_cus);
 
-hipError_t launch_setup(uint32_t* counters, const ctd::ChunkHdr* hdr, hipStream_t s);
-// Counters for a ray-level launch of n rays (error flags, 16 words, cleared).
-hipError_t launch_setup_rays(uint32_t* counters, uint32_t* err, uint32_t n, hipStream_t s);
+// A chunk's header, views and segments (word counts) from its staging buffer
+// to device memory, and its counters cleared.
+hipError_t launch_stage(const uint32_t* stage, uint32_t view_words, uint32_t seg_words, ctd::ChunkHdr* hdr,
+                        ctd::ViewDesc* views, ctd::Segment* segs, uint32_t* counters, hipStream_t s);
 hipError_t launch_generate(const LaunchShape& ls, const ctd::ViewDesc* views, const ctd::Segment* segs,
                            const ctd::ChunkHdr* hdr, uint32_t max_n, const ctd::Queues& q, hipStream_t s);
-// Closest hit for the n rays [0, active[bounce]) of q.ray_o/ray_d[sel] into
-// q.hit (the ray-level entry points).
+// Closest hit for the n rays of q.ray_o/ray_d[0] into q.hit (the ray-level
+// entry points); clears the counters it needs.
 hipError_t launch_extend(const LaunchShape& ls, const ctd::DevScene& sc, const ctd::TraceOpts& to,
-                         const ctd::Queues& q, int sel, int bounce, uint32_t n, hipStream_t s);
+                         const ctd::Queues& q, uint32_t n, hipStream_t s);
 // The frame loop's traversal of bounce b: closest hit for the extension rays
 // of bounce b and any hit for the shadow rays of bounce b - 1 in one launch
 // (bounce = max_depth: the last bounce's shadow rays).  wstats (may be null)
@@ -67,7 +68,7 @@ hipError_t launch_shade(const LaunchShape& ls, const ctd::DevScene& sc, const ct
                         const ctd::Queues& q, int sel, int bounce, hipStream_t s);
 hipError_t launch_resolve(const LaunchShape& ls, const ctd::ViewDesc* views, const ctd::Segment* segs,
                           const ctd::ChunkHdr* hdr, uint32_t max_tasks, const ctd::Queues& q, float4* accum,
-                          hipStream_t s);
+                          uint32_t* counts, hipStream_t s);
 hipError_t launch_tonemap(const float4* accum, uint32_t n, float samples, float4* out, hipStream_t s);
 hipError_t launch_tonemap8(const float4* accum, uint32_t n, float samples, uint32_t* out, hipStream_t s);
 // The fast node test's copy of a quad tree (8 float4 per node), its compact

@@ -523,6 +523,10 @@ CT_DEV bool node2_step(const float4 (&n)[7], f3 o, f3 inv, bool fast, LaneStack&
 // A lane without a ray.
 constexpr uint32_t kDead = 0xFFFFFFFFu;
 
+// Raises the error flag, a word in pinned host memory: a plain store (every
+// writer stores the same), which the host sees once the stream has finished.
+CT_DEV void raise(uint32_t* err) { *reinterpret_cast<volatile uint32_t*>(err) = 1u; }
+
 // What a launch traces: every ray closest-hit (extend, ray-level closest
 // hit), every ray any-hit (ray-level shadow rays), or two queues at once, a
 // closest-hit queue and an any-hit queue, each lane in the mode of the ray
@@ -929,7 +933,7 @@ CT_DEV void trace_quads(const DevScene& sc, float eps, f3 o, f3 d, f3 inv, bool 
         if (done || st.overflow) {
             if (st.overflow) prim = -2;
             if (c == 0u) {
-                if (st.overflow) atomicOr(err, 1u);
+                if (st.overflow) raise(err);
                 sink(ray, any, t, prim);
             }
             cur = kDead;
@@ -1024,7 +1028,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
         }
         if (done) {
             if (st.overflow) {
-                atomicOr(err, 1u);
+                raise(err);
                 prim = -2;
             }
             sink(ray, any, t, prim);
@@ -1098,7 +1102,7 @@ CT_DEV int trace_single(const DevScene& sc, float eps, f3 o, f3 d, float& t, boo
         if (trav_step<ACCEL, false>(sc, eps, o, d, inv, fast, any, true, cur, t, prim, st, cnt, n, kind)) break;
     }
     if (st.overflow) {
-        atomicOr(err, 1u);
+        raise(err);
         return -2;
     }
     return prim;

@@ -810,6 +810,14 @@ int ct_read_image_rgba8(ct_ctx* c, uint8_t* rgba, size_t n_bytes) {
     return CT_OK;
 }
 
+// The error flag of lane 0's finished launch, cleared for the next call.
+static bool take_error(ct_ctx* c) {
+    volatile uint32_t* e = c->ln[0].h_read + kReadErr;
+    const bool raised = *e != 0;
+    *e = 0;
+    return raised;
+}
+
 static int ray_prologue(ct_ctx* c, const ct_frame_opts* opts, ct_frame_opts& o) {
     if (opts) o = *opts;
     else ct_frame_opts_default(&o);
@@ -838,18 +846,12 @@ int ct_trace_rays(ct_ctx* c, const float* origins, const float* dirs, uint32_t n
             ro[i] = f4(origins + 3 * (size_t)(base + i), 0.0f);
             rd[i] = f4(dirs + 3 * (size_t)(base + i), 0.0f);
         }
-        const ctd::ChunkHdr h{m, 0u, 0u, 0u};
         HIPCHK(hipMemcpyAsync(c->ln[0].q.ray_o[0], ro.data(), m * sizeof(float4), hipMemcpyHostToDevice, c->ln[0].stream), "rays");
         HIPCHK(hipMemcpyAsync(c->ln[0].q.ray_d[0], rd.data(), m * sizeof(float4), hipMemcpyHostToDevice, c->ln[0].stream), "rays");
-        HIPCHK(hipMemcpyAsync(c->ln[0].d_hdr, &h, sizeof(h), hipMemcpyHostToDevice, c->ln[0].stream), "header");
-        HIPCHK(ctk::launch_setup(c->ln[0].q.counters, c->ln[0].d_hdr, c->ln[0].stream), "setup");
-        HIPCHK(ctk::launch_extend(c->shape, c->sc, to, c->ln[0].q, 0, 0, m, c->ln[0].stream), "extend");
-        uint32_t errflag = 0;
+        HIPCHK(ctk::launch_extend(c->shape, c->sc, to, c->ln[0].q, m, c->ln[0].stream), "extend");
         HIPCHK(hipMemcpyAsync(hits.data(), c->ln[0].q.hit, m * sizeof(float2), hipMemcpyDeviceToHost, c->ln[0].stream), "hits");
-        HIPCHK(hipMemcpyAsync(&errflag, c->ln[0].q.err, 4, hipMemcpyDeviceToHost, c->ln[0].stream), "flags");
         HIPCHK(hipStreamSynchronize(c->ln[0].stream), "trace rays");
-        if (errflag) {
-            (void)hipMemsetAsync(c->ln[0].q.err, 0, 4, c->ln[0].stream);
+        if (take_error(c)) {
             return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded");
         }
         for (uint32_t i = 0; i < m; ++i) {
@@ -879,30 +881,23 @@ int ct_trace_shadow_rays(ct_ctx* c, const float* origins, const float* dirs, con
     ctd::TraceOpts to{o.accel, o.traversal, o.triangle_epsilon};
     std::vector<float4> so(cap), sd(cap);
     hipError_t e = hipSuccess;
-    uint32_t errflag = 0;
+    bool overflow = false;
     for (uint32_t base = 0; base < n && e == hipSuccess; base += cap) {
         const uint32_t m = std::min(cap, n - base);
         for (uint32_t i = 0; i < m; ++i) {
             so[i] = f4(origins + 3 * (size_t)(base + i), tmax[base + i]);
             sd[i] = f4(dirs + 3 * (size_t)(base + i), 0.0f);
         }
-        const ctd::ChunkHdr h{m, 0u, 0u, 0u};
         e = hipMemcpyAsync(c->ln[0].q.sh_o[0], so.data(), m * sizeof(float4), hipMemcpyHostToDevice, c->ln[0].stream);
         if (e == hipSuccess) e = hipMemcpyAsync(c->ln[0].q.sh_d[0], sd.data(), m * sizeof(float4), hipMemcpyHostToDevice, c->ln[0].stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(c->ln[0].d_hdr, &h, sizeof(h), hipMemcpyHostToDevice, c->ln[0].stream);
-        if (e == hipSuccess) e = ctk::launch_setup(c->ln[0].q.counters, c->ln[0].d_hdr, c->ln[0].stream);
         if (e == hipSuccess) e = ctk::launch_shadow_flags(c->shape, c->sc, to, c->ln[0].q, m, (uint8_t*)dout, c->ln[0].stream);
         if (e == hipSuccess) e = hipMemcpyAsync(occluded_out + base, dout, m, hipMemcpyDeviceToHost, c->ln[0].stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(&errflag, c->ln[0].q.err, 4, hipMemcpyDeviceToHost, c->ln[0].stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->ln[0].stream);
-        if (errflag) break;
+        if (e == hipSuccess && (overflow = take_error(c))) break;
     }
     dfree(c, dout);
     if (e != hipSuccess) return hip_fail(c, e, "trace shadow rays");
-    if (errflag) {
-        (void)hipMemsetAsync(c->ln[0].q.err, 0, 4, c->ln[0].stream);
-        return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded");
-    }
+    if (overflow) return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded");
     return CT_OK;
 }
 
@@ -920,24 +915,14 @@ int ct_trace_rays_device(ct_ctx* c, const void* d_rays_o, const void* d_rays_d, 
     q.ray_d[0] = (float4*)d_rays_d;
     q.hit = (float2*)d_hits;
     ctd::TraceOpts to{o.accel, o.traversal, o.triangle_epsilon};
-    const ctd::ChunkHdr h{n, 0u, 0u, 0u};
-    HIPCHK(hipMemcpyAsync(c->ln[0].d_hdr, &h, sizeof(h), hipMemcpyHostToDevice, c->ln[0].stream), "header");
-    HIPCHK(ctk::launch_setup(c->ln[0].q.counters, c->ln[0].d_hdr, c->ln[0].stream), "setup");
-    HIPCHK(hipEventRecord(c->ln[0].ev[0], c->ln[0].stream), "event");
-    HIPCHK(ctk::launch_extend(c->shape, c->sc, to, q, 0, 0, n, c->ln[0].stream), "extend");
-    HIPCHK(hipEventRecord(c->ln[0].ev[1], c->ln[0].stream), "event");
-    uint32_t errflag = 0;
-    HIPCHK(hipMemcpyAsync(&errflag, c->ln[0].q.err, 4, hipMemcpyDeviceToHost, c->ln[0].stream), "flags");
-    HIPCHK(hipStreamSynchronize(c->ln[0].stream), "trace rays");
-    float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, c->ln[0].ev[0], c->ln[0].ev[1]), "elapsed");
-    if (kernel_ms) *kernel_ms = ms;
-    if (errflag) {
-        // cleared here, so the next call on the context does not report it
-        HIPCHK(hipMemsetAsync(c->ln[0].q.err, 0, 4, c->ln[0].stream), "clear error flags");
-        HIPCHK(hipStreamSynchronize(c->ln[0].stream), "clear error flags");
+    hipStream_t s = c->ln[0].stream;
+    if (kernel_ms) HIPCHK(hipEventRecord(c->ln[0].ev[0], s), "event");
+    HIPCHK(ctk::launch_extend(c->shape, c->sc, to, q, n, s), "extend");
+    if (kernel_ms) HIPCHK(hipEventRecord(c->ln[0].ev[1], s), "event");
+    HIPCHK(hipStreamSynchronize(s), "trace rays");
+    if (kernel_ms) HIPCHK(hipEventElapsedTime(kernel_ms, c->ln[0].ev[0], c->ln[0].ev[1]), "elapsed");
+    if (take_error(c))
         return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded (rays reported as misses)");
-    }
     return CT_OK;
 }
 
@@ -974,7 +959,7 @@ int ct_render_batch(ct_ctx* c, const ct_view* views, int32_t n_views, const ct_f
     ChunkStats st;
     int chunks_before = 0;
     (void)chunks_before;
-    r = run_paths(c, vd, runs, cap, arena, o, kRunGraph, &st);
+    r = run_paths(c, vd, runs, cap, arena, o, kRunGraph | (stats ? kRunClock : 0), &st);
     if (r == CT_OK) {
         for (int32_t i = 0; i < n_views && e == hipSuccess; ++i)
             e = hipMemcpyAsync(views[i].accum_out, arena + vd[i].accum_offset,
@@ -1031,7 +1016,7 @@ int ct_autotune(ct_ctx* c, const ct_camera* cam, const ct_frame_opts* opts, int3
         *t = 0;
         for (int rep = 0; rep < 3; ++rep) {
             ChunkStats st;
-            const int rr = run_paths(c, views, runs, (uint32_t)(npix * spp_shape), acc, o, 0, &st);
+            const int rr = run_paths(c, views, runs, (uint32_t)(npix * spp_shape), acc, o, kRunClock, &st);
             if (rr != CT_OK) return rr;
             if (rep > 0) *t += st.total_ms;
         }
@@ -1066,7 +1051,7 @@ int ct_autotune(ct_ctx* c, const ct_camera* cam, const ct_frame_opts* opts, int3
     std::vector<Run> r2{{0u, 0u, (uint32_t)(npix * spp_chunk)}};
     auto time_chunk = [&](uint32_t ch, double* t) -> int {
         ChunkStats st;
-        const int rr = run_paths(c, v2, r2, ch, acc, o, 0, &st);
+        const int rr = run_paths(c, v2, r2, ch, acc, o, kRunClock, &st);
         if (rr == CT_OK) { *t = st.total_ms; ++trials; }
         return rr;
     };

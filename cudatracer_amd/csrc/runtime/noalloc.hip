@@ -3,26 +3,25 @@
 // Callers that cannot allocate device memory (code under HIP graph capture,
 // tight serving loops, harnesses that forbid hipMalloc) get the closest-hit
 // kernel of ct_trace_rays_device with every buffer beyond their rays and
-// hits in one file-scope device array, `scratch`: the work counters and
-// error flags (kScratchCtl bytes) and the traversal stack's spill region
-// (kScratchSpill bytes).  Each GPU the library runs on holds its own copy of
+// hits in one file-scope device array, `scratch`: the work counters
+// (kScratchCtl bytes) and the traversal stack's spill region (kScratchSpill
+// bytes); the error flag is a word of the context's pinned memory.  Each GPU the library runs on holds its own copy of
 // the array, at its own address, until the process ends; ct_ctx_create looks
 // that address up once per device (hipGetSymbolAddress) and every later use
 // goes through it.  All calls on one GPU share its array: calls that overlap
 // on one GPU (two contexts, two threads) race and must be serialised by the
-// caller.  The setup kernel of each call clears what must start at zero
-// (counters, error flags), so a call does not depend on the previous one.
+// caller.  Each call clears the counters it uses (launch_extend) and the flag,
+// so a call does not depend on the previous one.
 #include <mutex>
 
 #include "runtime.h"
 
 namespace {
 
-constexpr size_t kScratchCtl = 64u << 10;     // counters (kCounterWords words) + error flags
+constexpr size_t kScratchCtl = 64u << 10;     // counters (kCounterWords words)
 constexpr size_t kScratchSpill = 32u << 20;   // traversal stack spill
 constexpr size_t kScratchBytes = kScratchCtl + kScratchSpill;
-constexpr size_t kScratchErr = kScratchCtl - 256;  // error flags: the last 256 bytes of the control part
-static_assert((size_t)ctd::kCounterWords * 4 <= kScratchErr, "counters do not fit the control part");
+static_assert((size_t)ctd::kCounterWords * 4 <= kScratchCtl, "counters do not fit the control part");
 // Stack bound of the allocation-free launch (LDS + spill).  The reference's
 // traversal stack holds 32 entries (MBVHNode.cuh:128); 48 covers every tree
 // of the configuration scenes (deepest quad tree: 16 levels) with room, and
@@ -91,21 +90,19 @@ extern "C" int ct_trace_rays_device_noalloc(ct_ctx* c, const void* d_rays_o, con
     q.ray_d[0] = (float4*)d_rays_d;
     q.hit = (float2*)d_hits;
     q.counters = reinterpret_cast<uint32_t*>(base);
-    q.err = reinterpret_cast<uint32_t*>(base + kScratchErr);
+    q.err = c->h_flag_dev;
     q.spill = reinterpret_cast<uint32_t*>(base + kScratchCtl);
     q.max_stack = kNoAllocStack;
     const ctd::TraceOpts to{o.accel, o.traversal, o.triangle_epsilon};
     hipStream_t s = c->ln[0].stream;
-    HIPCHK(ctk::launch_setup_rays(q.counters, q.err, n, s), "setup");
-    HIPCHK(hipEventRecord(c->ln[0].ev[0], s), "event");
-    HIPCHK(ctk::launch_extend(ls, c->sc, to, q, 0, 0, n, s), "extend");
-    HIPCHK(hipEventRecord(c->ln[0].ev[1], s), "event");
-    uint32_t errflag = 0;
-    HIPCHK(hipMemcpyAsync(&errflag, q.err, 4, hipMemcpyDeviceToHost, s), "flags");
+    if (kernel_ms) HIPCHK(hipEventRecord(c->ln[0].ev[0], s), "event");
+    HIPCHK(ctk::launch_extend(ls, c->sc, to, q, n, s), "extend");
+    if (kernel_ms) HIPCHK(hipEventRecord(c->ln[0].ev[1], s), "event");
     HIPCHK(hipStreamSynchronize(s), "trace rays");
-    float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, c->ln[0].ev[0], c->ln[0].ev[1]), "elapsed");
-    if (kernel_ms) *kernel_ms = ms;
+    if (kernel_ms) HIPCHK(hipEventElapsedTime(kernel_ms, c->ln[0].ev[0], c->ln[0].ev[1]), "elapsed");
+    volatile uint32_t* flag = c->h_flag;
+    const bool errflag = *flag != 0;
+    *flag = 0;
     if (errflag)
         return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound (48 entries without allocation) exceeded; "
                                               "the rays that needed more are reported as misses");

@@ -52,8 +52,10 @@ struct Lane {
     ctd::Segment* d_segs = nullptr;
     uint32_t d_segs_cap = 0;
     ctd::ChunkHdr* d_hdr = nullptr;
-    uint32_t* h_read = nullptr;      // pinned read-back: counters, error flag, work counters
-    uint8_t* h_stage = nullptr;      // pinned upload staging of the chunk tables
+    uint32_t* h_read = nullptr;      // pinned, written by the device: counters, error flag (Queues::err), work counters
+    uint32_t* h_read_dev = nullptr;  // its device address
+    uint32_t* h_stage = nullptr;     // pinned upload staging of the chunk tables, read by k_stage
+    uint32_t* h_stage_dev = nullptr; // its device address
     size_t h_stage_bytes = 0;
     // captured bounce loop
     hipGraphExec_t graph_exec = nullptr;
@@ -65,15 +67,14 @@ struct Lane {
     bool pending = false;
     uint32_t n_paths = 0;
     int max_depth = 0;
-    bool timed = false, count = false;
+    bool timed = false, count = false, clock = false;
     bool nee = false;  // the chunk ends with a launch for the last bounce's shadow rays
     int tail = -1;     // the chunk's k_paths bounce, or -1
     bool paths = false;  // the chunk runs as whole paths (k_paths)
 };
 // h_read layout (uint32 words)
-constexpr int kReadCounters = 2 * (ctd::kMaxBounce + 1) + 2;  // per-bounce counts, then k_paths's two
-constexpr int kReadErr = kReadCounters;
-constexpr int kReadWork = kReadCounters + 2;  // 4 x uint64, 8-byte aligned
+constexpr int kReadErr = ctd::kReadCounters;
+constexpr int kReadWork = ctd::kReadCounters + 2;  // 4 x uint64, 8-byte aligned
 constexpr int kReadWords = kReadWork + 8;
 
 struct ct_ctx {
@@ -110,6 +111,9 @@ struct ct_ctx {
     std::vector<void*> path_bufs;
     uint32_t spill_threads = 0;
 
+    // error flag of the allocation-free entry point (pinned; its device address)
+    uint32_t* h_flag = nullptr;
+    uint32_t* h_flag_dev = nullptr;
     // this device's copy of the allocation-free entry point's scratch array
     // (its device address; runtime/noalloc.hip)
     void* scratch = nullptr;
@@ -141,6 +145,8 @@ bool camera_ok(const ct_camera* cam);
 // words (two), hit, shadow origin, direction and colour (two sets), path
 // radiance and the radiance terms (two sets each of shade's and connect's).
 constexpr size_t kPathSlotBytes = 6 * 16 + 2 * 4 + 8 + 6 * 16 + 16 + 4 * 16;
+// Zeroed pinned words the device can access, and their device address.
+bool pinned_words(size_t words, uint32_t** host, uint32_t** dev);
 // Path buffers for chunks of up to cap paths on each lane.
 int ensure_paths(ct_ctx* c, uint32_t cap);
 int ensure_tables(ct_ctx* c, Lane& L, uint32_t nviews, uint32_t nsegs);
@@ -164,8 +170,9 @@ struct Run {
 // kernel (per-stage times in ChunkStats), kRunCount counts node / triangle
 // tests, kRunGraph replays each lane's captured bounce loop, kRunSerial
 // runs one chunk at a time (nothing overlaps: per-kernel times are the
-// kernels' own, for measurement).
-enum RunFlags { kRunTimed = 1, kRunCount = 2, kRunGraph = 4, kRunSerial = 8 };
+// kernels' own, for measurement), kRunClock measures the chunks' device time
+// (ChunkStats::total_ms; kRunTimed does too).
+enum RunFlags { kRunTimed = 1, kRunCount = 2, kRunGraph = 4, kRunSerial = 8, kRunClock = 16 };
 int run_paths(ct_ctx* c, const std::vector<ctd::ViewDesc>& views, const std::vector<Run>& runs, uint32_t cap,
               float4* accum, const ct_frame_opts& o, int flags, ChunkStats* st);
 

@@ -139,6 +139,22 @@ static void free_paths(ct_ctx* c) {
     drop_graphs(c);
 }
 
+// Zeroed pinned host memory that the device writes (coherent: the host reads
+// it after the stream without a copy), and its device address.
+bool pinned_words(size_t words, uint32_t** host, uint32_t** dev) {
+    if (hipHostMalloc((void**)host, words * 4, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) {
+        *host = nullptr;
+        return false;
+    }
+    std::memset(*host, 0, words * 4);
+    if (hipHostGetDevicePointer((void**)dev, *host, 0) != hipSuccess) {
+        (void)hipHostFree(*host);
+        *host = nullptr;
+        return false;
+    }
+    return true;
+}
+
 int ensure_paths(ct_ctx* c, uint32_t cap) {
     cap = std::max<uint32_t>(cap, 64u);
     const uint32_t threads = (uint32_t)(c->shape.trace_blocks * c->shape.block);
@@ -199,16 +215,12 @@ int ensure_paths(ct_ctx* c, uint32_t cap) {
         }
         L.gen = 0;
         r = A((void**)&L.q.counters, ctd::kCounterWords * 4, "counters");
-        if (r == CT_OK) r = A((void**)&L.q.err, 64, "error flags");
         if (r == CT_OK) r = A((void**)&L.q.spill, (size_t)threads * ctd::kMaxStack * 4, "stack spill");
         if (r == CT_OK) r = A((void**)&L.wstats, 64, "work counters");
         if (r == CT_OK) r = A((void**)&L.d_hdr, sizeof(ChunkHdr), "chunk header");
-        if (r == CT_OK && hipHostMalloc((void**)&L.h_read, kReadWords * 4, hipHostMallocDefault) != hipSuccess) {
-            L.h_read = nullptr;
+        if (r == CT_OK && !pinned_words(kReadWords, &L.h_read, &L.h_read_dev))
             r = fail(c, CT_ERR_OUT_OF_MEMORY, "pinned read-back buffer");
-        }
-        if (r == CT_OK && hipMemsetAsync(L.q.err, 0, 64, L.stream) != hipSuccess)
-            r = fail(c, CT_ERR_DEVICE, "clear error flags");
+        if (r == CT_OK) L.q.err = L.h_read_dev + kReadErr;
     }
     if (r == CT_OK && hipStreamSynchronize(c->ln[0].stream) != hipSuccess)
         r = fail(c, CT_ERR_DEVICE, "clear radiance terms");
@@ -386,7 +398,6 @@ struct BounceSeq {
         hipError_t r;
         if (k == 0) {
             rec();
-            if ((r = ctk::launch_setup(L->q.counters, L->d_hdr, s)) != hipSuccess) return r;
             if (paths) {
                 rec();
                 return hipSuccess;
@@ -470,23 +481,24 @@ static constexpr int kEvResolve = 2 * (3 * ctd::kMaxBounce + 8) - 4;  // resolve
 // BounceSeq enqueues it; close_chunk queues the resolve after the previous
 // chunk's resolve (prev_resolved, may be null) and the read-back.
 static int stage_chunk(ct_ctx* c, Lane& L, const std::vector<ViewDesc>& views, const std::vector<Segment>& segs,
-                       uint32_t n, uint32_t n_tasks, bool count) {
+                       uint32_t n, uint32_t n_tasks, bool count, bool clock) {
     int r = ensure_tables(c, L, (uint32_t)views.size(), (uint32_t)segs.size());
     if (r != CT_OK) return r;
     hipStream_t s = L.stream;
-    // tables staged in pinned memory: the copies run after this call returns,
-    // and the lane's staging is rewritten only once its chunk has finished
+    // tables staged in pinned memory: k_stage reads them after this call
+    // returns, and the lane's staging is rewritten only once its chunk has
+    // finished
+    constexpr size_t kViews = 4 * (size_t)ctd::kStageViews;
+    static_assert(sizeof(ViewDesc) % 4 == 0 && sizeof(Segment) % 4 == 0 && sizeof(ChunkHdr) <= kViews, "staging words");
     const size_t vb = views.size() * sizeof(ViewDesc), sb = segs.size() * sizeof(Segment);
-    const size_t need = 256 + vb + sb;
+    const size_t need = kViews + vb + sb;
     if (need > L.h_stage_bytes) {
         if (L.h_stage) (void)hipHostFree(L.h_stage);
         L.h_stage = nullptr;
         L.h_stage_bytes = 0;
         const size_t bytes = std::max<size_t>(need * 2, 1u << 16);
-        if (hipHostMalloc((void**)&L.h_stage, bytes, hipHostMallocDefault) != hipSuccess) {
-            L.h_stage = nullptr;
+        if (!pinned_words(bytes / 4, &L.h_stage, &L.h_stage_dev))
             return fail(c, CT_ERR_OUT_OF_MEMORY, "pinned staging of chunk tables");
-        }
         L.h_stage_bytes = bytes;
     }
     // the chunk's generation: its radiance terms' stamps differ from any
@@ -500,14 +512,15 @@ static int stage_chunk(ct_ctx* c, Lane& L, const std::vector<ViewDesc>& views, c
         }
     }
     const ChunkHdr h{n, n_tasks, (uint32_t)segs.size(), L.gen};
-    std::memcpy(L.h_stage, &h, sizeof(h));
-    std::memcpy(L.h_stage + 256, views.data(), vb);
-    std::memcpy(L.h_stage + 256 + vb, segs.data(), sb);
-    HIPCHK(hipMemcpyAsync(L.d_views, L.h_stage + 256, vb, hipMemcpyHostToDevice, s), "upload views");
-    HIPCHK(hipMemcpyAsync(L.d_segs, L.h_stage + 256 + vb, sb, hipMemcpyHostToDevice, s), "upload segments");
-    HIPCHK(hipMemcpyAsync(L.d_hdr, L.h_stage, sizeof(h), hipMemcpyHostToDevice, s), "upload chunk header");
+    char* stage = reinterpret_cast<char*>(L.h_stage);
+    std::memcpy(stage, &h, sizeof(h));
+    std::memcpy(stage + kViews, views.data(), vb);
+    std::memcpy(stage + kViews + vb, segs.data(), sb);
+    if (clock) HIPCHK(hipEventRecord(L.ev[kEvTotal0], s), "event");
+    HIPCHK(ctk::launch_stage(L.h_stage_dev, (uint32_t)(vb / 4), (uint32_t)(sb / 4), L.d_hdr, L.d_views, L.d_segs,
+                             L.q.counters, s),
+           "stage chunk");
     if (count) HIPCHK(hipMemsetAsync(L.wstats, 0, 32, s), "clear work counters");
-    HIPCHK(hipEventRecord(L.ev[kEvTotal0], s), "event");
     return CT_OK;
 }
 
@@ -536,19 +549,17 @@ static int graph_chunk(ct_ctx* c, Lane& L, const ct_frame_opts& o) {
 }
 
 static int close_chunk(ct_ctx* c, Lane& L, uint32_t n, float4* accum, const ct_frame_opts& o, bool timed,
-                       bool count, bool whole, hipEvent_t prev_resolved) {
+                       bool count, bool clock, bool whole, bool alone, hipEvent_t prev_resolved) {
     hipStream_t s = L.stream;
     // accumulator updates in chunk order
     if (prev_resolved) HIPCHK(hipStreamWaitEvent(s, prev_resolved, 0), "order resolves");
     if (timed) HIPCHK(hipEventRecord(L.ev[kEvResolve], s), "event");
-    HIPCHK(ctk::launch_resolve(c->shape, L.d_views, L.d_segs, L.d_hdr, c->lane_cap, L.q, accum, s),
+    HIPCHK(ctk::launch_resolve(c->shape, L.d_views, L.d_segs, L.d_hdr, std::min(c->lane_cap, n), L.q, accum,
+                               L.h_read_dev, s),
            "launch resolve");
     if (timed) HIPCHK(hipEventRecord(L.ev[kEvResolve + 1], s), "event");
-    HIPCHK(hipEventRecord(L.resolved, s), "event");
-    HIPCHK(hipEventRecord(L.ev[kEvTotal0 + 1], s), "event");
-    // queue sizes (ray counts), error flags and work counters
-    HIPCHK(hipMemcpyAsync(L.h_read, L.q.counters, kReadCounters * 4, hipMemcpyDeviceToHost, s), "read counters");
-    HIPCHK(hipMemcpyAsync(L.h_read + kReadErr, L.q.err, 4, hipMemcpyDeviceToHost, s), "read error flags");
+    if (!alone) HIPCHK(hipEventRecord(L.resolved, s), "event");
+    if (clock) HIPCHK(hipEventRecord(L.ev[kEvTotal0 + 1], s), "event");
     if (count) HIPCHK(hipMemcpyAsync(L.h_read + kReadWork, L.wstats, 32, hipMemcpyDeviceToHost, s), "read work");
     L.pending = true;
     L.n_paths = n;
@@ -558,6 +569,7 @@ static int close_chunk(ct_ctx* c, Lane& L, uint32_t n, float4* accum, const ct_f
     L.paths = whole;
     L.timed = timed;
     L.count = count;
+    L.clock = clock;
     return CT_OK;
 }
 
@@ -566,9 +578,9 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
     if (!L.pending) return CT_OK;
     L.pending = false;
     HIPCHK(hipStreamSynchronize(L.stream), "chunk");
-    const uint32_t* cnt = L.h_read;
+    const volatile uint32_t* cnt = L.h_read;
     if (cnt[kReadErr]) {
-        (void)hipMemsetAsync(L.q.err, 0, 4, L.stream);
+        L.h_read[kReadErr] = 0;
         return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded (malformed tree)");
     }
     if (!st) return CT_OK;
@@ -580,7 +592,7 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
     st->shadow += cnt[2 * (ctd::kMaxBounce + 1) + 1];
     st->samples += L.n_paths;
     float ms = 0;
-    if (hipEventElapsedTime(&ms, L.ev[kEvTotal0], L.ev[kEvTotal0 + 1]) == hipSuccess) st->total_ms += ms;
+    if (L.clock && hipEventElapsedTime(&ms, L.ev[kEvTotal0], L.ev[kEvTotal0 + 1]) == hipSuccess) st->total_ms += ms;
     if (L.timed) {
         // event pairs: [generate] then per bounce [trace][shade] (at the tail
         // bounce [trace][k_paths], the last bounce the chunk launches); [trace
@@ -610,7 +622,7 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
     }
     if (L.count) {
         unsigned long long w[4];
-        std::memcpy(w, cnt + kReadWork, sizeof(w));
+        std::memcpy(w, L.h_read + kReadWork, sizeof(w));
         for (int k = 0; k < 4; ++k) st->work[k] += w[k];
     }
     return CT_OK;
@@ -621,10 +633,8 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
 // a later call.  The accumulator may hold part of the failed call's samples.
 static void abort_lanes(ct_ctx* c) {
     sync_lanes(c);
-    for (Lane& L : c->ln) {
-        if (L.q.err) (void)hipMemsetAsync(L.q.err, 0, 4, L.stream);
-        if (L.stream) (void)hipStreamSynchronize(L.stream);
-    }
+    for (Lane& L : c->ln)
+        if (L.h_read) L.h_read[kReadErr] = 0;
 }
 
 // Paths of a workload below which it is not split over the lanes.
@@ -633,7 +643,7 @@ static constexpr uint64_t kSplitMin = 1u << 18;
 int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<Run>& runs, uint32_t cap,
               float4* accum, const ct_frame_opts& o, int flags, ChunkStats* st) {
     const bool timed = flags & kRunTimed, count = flags & kRunCount, use_graph = flags & kRunGraph,
-               serial = flags & kRunSerial;
+               serial = flags & kRunSerial, clock = flags & (kRunClock | kRunTimed);
     uint64_t total = 0;
     for (const Run& run : runs) total += run.n;
     if (total >= kSplitMin && cap > 0) {
@@ -647,8 +657,9 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
     cap = std::min(cap, c->lane_cap);
     const bool whole = whole_paths(c, total, count);
     // work queued on lane 0 by the caller (accumulator clears) comes first
-    HIPCHK(hipEventRecord(c->ln[0].resolved, c->ln[0].stream), "event");
-    for (int k = 1; k < kLanes; ++k) HIPCHK(hipStreamWaitEvent(c->ln[k].stream, c->ln[0].resolved, 0), "order lanes");
+    const bool alone = total <= cap;  // one chunk, on lane 0
+    if (!alone) HIPCHK(hipEventRecord(c->ln[0].resolved, c->ln[0].stream), "event");
+    for (int k = 1; k < kLanes && !alone; ++k) HIPCHK(hipStreamWaitEvent(c->ln[k].stream, c->ln[0].resolved, 0), "order lanes");
     hipEvent_t prev = nullptr;
     int lane = 0;
     // The first kLanes chunks (one per lane) are launched together, their
@@ -667,7 +678,8 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
         for (int i = 0; i < g; ++i) {
             Lane& L = c->ln[(lane + i) % kLanes];
             if ((rr = finish_chunk(c, L, st)) != CT_OK) return rr;  // the lane's previous chunk
-            if ((rr = stage_chunk(c, L, views, group[i].segs, group[i].fill, group[i].tasks, count)) != CT_OK)
+            if ((rr = stage_chunk(c, L, views, group[i].segs, group[i].fill, group[i].tasks, count, clock)) !=
+                CT_OK)
                 return rr;
         }
         // a chunk's loop from the lane's graph, or enqueued here
@@ -691,7 +703,8 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
             if (here[i]) HIPCHK(seq[i].finish(), "launch chunk");
         for (int i = 0; i < g; ++i) {
             Lane& L = c->ln[(lane + i) % kLanes];
-            if ((rr = close_chunk(c, L, group[i].fill, accum, o, timed, count, whole, prev)) != CT_OK)
+            if ((rr = close_chunk(c, L, group[i].fill, accum, o, timed, count, clock, whole, alone, prev)) !=
+                CT_OK)
                 return rr;
             prev = L.resolved;
             if (serial && (rr = finish_chunk(c, L, st)) != CT_OK) return rr;  // done before the next starts
@@ -832,7 +845,7 @@ int ct_ctx_create(const ct_device_opts* opts, ct_ctx** out) {
             return CT_ERR_DEVICE;
         }
     }
-    if (scratch_init(c) != CT_OK) {
+    if (!pinned_words(16, &c->h_flag, &c->h_flag_dev) || scratch_init(c) != CT_OK) {
         ct_ctx_destroy(c);
         return CT_ERR_DEVICE;
     }
@@ -849,6 +862,7 @@ void ct_ctx_destroy(ct_ctx* c) {
     drop_graphs(c);
     for (auto& a : c->allocs) (void)hipFree(a.first);
     c->allocs.clear();
+    if (c->h_flag) (void)hipHostFree(c->h_flag);
     for (Lane& L : c->ln) {
         if (L.h_read) (void)hipHostFree(L.h_read);
         if (L.h_stage) (void)hipHostFree(L.h_stage);
