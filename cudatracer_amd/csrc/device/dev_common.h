@@ -182,6 +182,18 @@ struct Queues {
     int max_stack = kMaxStack;  // traversal stack entries (LDS + spill); deeper trees report an overflow
 };
 
+// The rays of a ray-level launch, as the caller's arrays hold them (packed
+// triples, or the first three of four), and where the results go.
+struct RayArrays {
+    const float *o, *d;   // ray i at i * stride
+    uint32_t stride;      // floats per ray: 3 or 4
+    uint32_t hit_stride;  // words per hit: 1 (separate arrays) or 2 (t and id interleaved)
+    float* t;             // closest hit: ray i at i * hit_stride
+    int* prim;
+    const float* tmax;    // any hit
+    uint8_t* occluded;
+};
+
 // counters[] layout: for bounce b in [0, kMaxBounce]
 constexpr int kMaxBounce = 64;
 

@@ -112,24 +112,25 @@ __global__ void k_generate(const ViewDesc* __restrict__ views, const Segment* __
 }
 
 // --------------------------------------------------------------- extend --
-// Persistent closest-hit over a queue of rays (see trace_persistent): the
+// Persistent closest-hit over an array of rays (see trace_persistent): the
 // ray-level entry points.
+CT_DEV f3 load3(const float* p) { return mk3(p[0], p[1], p[2]); }
+
 template <int ACCEL>
-CT_DEV void extend_impl(const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n, LaneStack& st) {
-    const float4* __restrict__ ro = q.ray_o[0];
-    const float4* __restrict__ rd = q.ray_d[0];
-    float2* hit = q.hit;
+CT_DEV void extend_impl(const DevScene& sc, const TraceOpts& to, const Queues& q, const RayArrays& r, uint32_t n,
+                        LaneStack& st) {
     TravCount tc{0u, 0u, 0u, 0u};
     trace_persistent<ACCEL, kClosest, false>(
         sc, to.teps, n, 0u, cnt_fetch_ext(q.counters, 0), st, tc, q.err,
         [&](uint32_t i, bool, f3& o, f3& d, float& t) {
-            o = xyz(ro[i]);
-            d = xyz(rd[i]);
+            o = load3(r.o + (size_t)i * r.stride);
+            d = load3(r.d + (size_t)i * r.stride);
             t = 1e34f;
         },
         [&](uint32_t i, bool, float t, int prim) {
             if (prim == -2) { t = 1e34f; prim = -1; }
-            hit[i] = make_float2(t, __int_as_float(prim));
+            r.t[(size_t)i * r.hit_stride] = t;
+            r.prim[(size_t)i * r.hit_stride] = prim;
         });
 }
 
@@ -160,9 +161,9 @@ CT_DEV LaneStack make_stack(const Queues& q, int lds_depth) {
 // reaches it without spills (the counting copies spill a register).
 template <int TREE>
 __global__ void __attribute__((amdgpu_waves_per_eu(8)))
-k_extend(DevScene sc, TraceOpts to, Queues q, uint32_t n, int lds_depth) {
+k_extend(DevScene sc, TraceOpts to, Queues q, RayArrays r, uint32_t n, int lds_depth) {
     LaneStack st = make_stack(q, lds_depth);
-    extend_impl<TREE>(sc, to, q, n, st);
+    extend_impl<TREE>(sc, to, q, r, n, st);
 }
 
 // ---------------------------------------------------------------- trace --
@@ -823,25 +824,25 @@ __global__ void k_tonemap(const float4* __restrict__ accum, uint32_t n, float sa
     }
 }
 
-// Ray-level any-hit: occluded flag per ray (rays in sh_o / sh_d layout).
+// Ray-level any-hit: occluded flag per ray.
 template <int ACCEL>
-CT_DEV void flags_impl(const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n, LaneStack& st,
-                       uint8_t* out) {
+CT_DEV void flags_impl(const DevScene& sc, const TraceOpts& to, const Queues& q, const RayArrays& r, uint32_t n,
+                       LaneStack& st) {
     TravCount tc{0u, 0u, 0u, 0u};
     trace_persistent<ACCEL, kAny, false>(
         sc, to.teps, n, 0u, cnt_fetch_sh(q.counters, 0), st, tc, q.err,
         [&](uint32_t i, bool, f3& o, f3& d, float& t) {
-            o = xyz(q.sh_o[0][i]);
-            d = xyz(q.sh_d[0][i]);
-            t = q.sh_o[0][i].w;
+            o = load3(r.o + (size_t)i * r.stride);
+            d = load3(r.d + (size_t)i * r.stride);
+            t = r.tmax[i];
         },
-        [&](uint32_t i, bool, float, int prim) { out[i] = prim >= 0 ? 1 : 0; });
+        [&](uint32_t i, bool, float, int prim) { r.occluded[i] = prim >= 0 ? 1 : 0; });
 }
 
 template <int TREE>
-__global__ void k_shadow_flags(DevScene sc, TraceOpts to, Queues q, uint32_t n, int lds_depth, uint8_t* out) {
+__global__ void k_shadow_flags(DevScene sc, TraceOpts to, Queues q, RayArrays r, uint32_t n, int lds_depth) {
     LaneStack st = make_stack(q, lds_depth);
-    flags_impl<TREE>(sc, to, q, n, st, out);
+    flags_impl<TREE>(sc, to, q, r, n, st);
 }
 
 }  // namespace ctd
@@ -894,11 +895,11 @@ static hipError_t setup_rays(const LaunchShape& ls, int tree, const Queues& q, u
 }
 
 template <int TREE>
-void extend_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n,
-              hipStream_t s) {
+void extend_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, const RayArrays& r,
+              uint32_t n, hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
     const dim3 grid(ray_grid(ls, TREE, n)), block(ls.block);
-    hipLaunchKernelGGL((k_extend<TREE>), grid, block, lds, s, sc, to, q, n, ls.lds_depth);
+    hipLaunchKernelGGL((k_extend<TREE>), grid, block, lds, s, sc, to, q, r, n, ls.lds_depth);
 }
 template <int TREE>
 void trace_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, const ChunkHdr* hdr,
@@ -913,16 +914,16 @@ void trace_t(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, con
                            wstats);
 }
 
-hipError_t launch_extend(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q, uint32_t n,
-                         hipStream_t s) {
+hipError_t launch_extend(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q,
+                         const RayArrays& r, uint32_t n, hipStream_t s) {
     const int tree = tree_of(to);
     const hipError_t e = setup_rays(ls, tree, q, n, s);
     if (e != hipSuccess) return e;
     switch (tree) {
-        case 2: extend_t<2>(ls, sc, to, q, n, s); break;
-        case 4: extend_t<4>(ls, sc, to, q, n, s); break;
-        case kTreeCompact: extend_t<kTreeCompact>(ls, sc, to, q, n, s); break;
-        default: extend_t<8>(ls, sc, to, q, n, s); break;
+        case 2: extend_t<2>(ls, sc, to, q, r, n, s); break;
+        case 4: extend_t<4>(ls, sc, to, q, r, n, s); break;
+        case kTreeCompact: extend_t<kTreeCompact>(ls, sc, to, q, r, n, s); break;
+        default: extend_t<8>(ls, sc, to, q, r, n, s); break;
     }
     return hipGetLastError();
 }
@@ -1195,17 +1196,17 @@ hipError_t launch_tonemap(const float4* accum, uint32_t n, float samples, float4
     return hipGetLastError();
 }
 hipError_t launch_shadow_flags(const LaunchShape& ls, const DevScene& sc, const TraceOpts& to, const Queues& q,
-                               uint32_t n, uint8_t* out, hipStream_t s) {
+                               const RayArrays& r, uint32_t n, hipStream_t s) {
     const size_t lds = (size_t)ls.lds_depth * ls.block * 4;
     const int tree = tree_of(to);
     const hipError_t e = setup_rays(ls, tree, q, n, s);
     if (e != hipSuccess) return e;
     const dim3 grid(ray_grid(ls, tree, n)), block(ls.block);
-    if (tree == 2) hipLaunchKernelGGL(k_shadow_flags<2>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
-    else if (tree == 4) hipLaunchKernelGGL(k_shadow_flags<4>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
+    if (tree == 2) hipLaunchKernelGGL(k_shadow_flags<2>, grid, block, lds, s, sc, to, q, r, n, ls.lds_depth);
+    else if (tree == 4) hipLaunchKernelGGL(k_shadow_flags<4>, grid, block, lds, s, sc, to, q, r, n, ls.lds_depth);
     else if (tree == kTreeCompact)
-        hipLaunchKernelGGL(k_shadow_flags<kTreeCompact>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
-    else hipLaunchKernelGGL(k_shadow_flags<8>, grid, block, lds, s, sc, to, q, n, ls.lds_depth, out);
+        hipLaunchKernelGGL(k_shadow_flags<kTreeCompact>, grid, block, lds, s, sc, to, q, r, n, ls.lds_depth);
+    else hipLaunchKernelGGL(k_shadow_flags<8>, grid, block, lds, s, sc, to, q, r, n, ls.lds_depth);
     return hipGetLastError();
 }
 

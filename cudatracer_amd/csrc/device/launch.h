@@ -40,10 +40,10 @@ hipError_t launch_stage(const uint32_t* stage, uint32_t view_words, uint32_t seg
                         ctd::ViewDesc* views, ctd::Segment* segs, uint32_t* counters, hipStream_t s);
 hipError_t launch_generate(const LaunchShape& ls, const ctd::ViewDesc* views, const ctd::Segment* segs,
                            const ctd::ChunkHdr* hdr, uint32_t max_n, const ctd::Queues& q, hipStream_t s);
-// Closest hit for the n rays of q.ray_o/ray_d[0] into q.hit (the ray-level
-// entry points); clears the counters it needs.
+// Closest hit for the n rays of r (the ray-level entry points); clears the
+// counters it needs.
 hipError_t launch_extend(const LaunchShape& ls, const ctd::DevScene& sc, const ctd::TraceOpts& to,
-                         const ctd::Queues& q, uint32_t n, hipStream_t s);
+                         const ctd::Queues& q, const ctd::RayArrays& r, uint32_t n, hipStream_t s);
 // The frame loop's traversal of bounce b: closest hit for the extension rays
 // of bounce b and any hit for the shadow rays of bounce b - 1 in one launch
 // (bounce = max_depth: the last bounce's shadow rays).  wstats (may be null)
@@ -85,6 +85,6 @@ hipError_t launch_shading_records(const float* vert, const float* norm, const fl
 // The primitive ids of n triangle records from `first` on.
 hipError_t launch_prim_ids(const float4* tris, uint32_t first, uint32_t n, uint32_t* out, hipStream_t s);
 hipError_t launch_shadow_flags(const LaunchShape& ls, const ctd::DevScene& sc, const ctd::TraceOpts& to,
-                               const ctd::Queues& q, uint32_t n, uint8_t* out, hipStream_t s);
+                               const ctd::Queues& q, const ctd::RayArrays& r, uint32_t n, hipStream_t s);
 
 }  // namespace ctk

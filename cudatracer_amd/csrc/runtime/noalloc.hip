@@ -86,9 +86,6 @@ extern "C" int ct_trace_rays_device_noalloc(ct_ctx* c, const void* d_rays_o, con
     ls.fullc = std::min(ls.fullc, cap);
     uint8_t* base = static_cast<uint8_t*>(c->scratch);  // the device address, never the symbol itself
     ctd::Queues q{};
-    q.ray_o[0] = (float4*)d_rays_o;
-    q.ray_d[0] = (float4*)d_rays_d;
-    q.hit = (float2*)d_hits;
     q.counters = reinterpret_cast<uint32_t*>(base);
     q.err = c->h_flag_dev;
     q.spill = reinterpret_cast<uint32_t*>(base + kScratchCtl);
@@ -96,7 +93,7 @@ extern "C" int ct_trace_rays_device_noalloc(ct_ctx* c, const void* d_rays_o, con
     const ctd::TraceOpts to{o.accel, o.traversal, o.triangle_epsilon};
     hipStream_t s = c->ln[0].stream;
     if (kernel_ms) HIPCHK(hipEventRecord(c->ln[0].ev[0], s), "event");
-    HIPCHK(ctk::launch_extend(ls, c->sc, to, q, n, s), "extend");
+    HIPCHK(ctk::launch_extend(ls, c->sc, to, q, device_rays(d_rays_o, d_rays_d, d_hits), n, s), "extend");
     if (kernel_ms) HIPCHK(hipEventRecord(c->ln[0].ev[1], s), "event");
     HIPCHK(hipStreamSynchronize(s), "trace rays");
     if (kernel_ms) HIPCHK(hipEventElapsedTime(kernel_ms, c->ln[0].ev[0], c->ln[0].ev[1]), "elapsed");

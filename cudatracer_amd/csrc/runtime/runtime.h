@@ -145,6 +145,17 @@ bool camera_ok(const ct_camera* cam);
 // words (two), hit, shadow origin, direction and colour (two sets), path
 // radiance and the radiance terms (two sets each of shade's and connect's).
 constexpr size_t kPathSlotBytes = 6 * 16 + 2 * 4 + 8 + 6 * 16 + 16 + 4 * 16;
+// The arrays of the device-pointer entry points: float4 rays, (t, id) pairs.
+inline ctd::RayArrays device_rays(const void* o, const void* d, void* hits) {
+    ctd::RayArrays r{};
+    r.o = static_cast<const float*>(o);
+    r.d = static_cast<const float*>(d);
+    r.stride = 4;
+    r.hit_stride = 2;
+    r.t = static_cast<float*>(hits);
+    r.prim = static_cast<int*>(hits) + 1;
+    return r;
+}
 // Zeroed pinned words the device can access, and their device address.
 bool pinned_words(size_t words, uint32_t** host, uint32_t** dev);
 // Path buffers for chunks of up to cap paths on each lane.
