@@ -9,7 +9,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from conftest import ArrayView
+from conftest import ArrayView, ray_set
 from test_gpu_stack import chain_rays, chain_scene
 from test_gpu_traversal_edges import _edge_rays
 
@@ -60,6 +60,30 @@ def test_deep_stacks(ct, orc, gpu_ctx, n):
     osc.set_trees(arrays["bvh"], arrays["mbvh"], arrays["prim_indices"])
     o, d = chain_rays(n, 4)
     _same(gpu_ctx, osc, o, d, np.full(n, 40.0, np.float32), ct.default_opts(), 1)
+
+
+@pytest.mark.parametrize("axis", [1, 2])
+def test_wide_tree_axis_parallel(ct, orc, gpu_ctx, c1, axis):
+    """Rays without a y or z component have infinite slab terms in the wide
+    tree and take its general node test (which leaves that axis out, so a
+    superset of the exact boxes is entered); the others take the hardware
+    minimum and maximum.  Both find the oracle's distances, but for the few
+    rays of the exact tree's ulp-level culls (1 in 100,000, as for the rays of
+    test_fast_traversal_closest_hit)."""
+    scene, arrays, osc = c1
+    gpu_ctx.upload_build(scene, wide=True)
+    opts, _, _ = scene.frame_opts()
+    opts.accel, opts.traversal = ct.ACCEL_BVH4, ct.TRAV_FAST
+    n = 1 << 18
+    o, d = ray_set(scene, arrays, n, seed=60 + axis)
+    d[::2, axis] = 0.0
+    tmax = np.random.default_rng(axis).uniform(0.0, 60.0, n).astype(np.float32)
+    t, p = gpu_ctx.trace_rays(o, d, opts)
+    t_ref, p_ref = osc.trace(o, d, 1, 32, opts.triangle_epsilon, threads=16)
+    assert np.sum(_bits(t) != _bits(t_ref)) <= n // 100_000
+    assert np.sum((p >= 0) != (p_ref >= 0)) <= n // 100_000
+    occ = gpu_ctx.trace_shadow_rays(o, d, tmax, opts)
+    assert np.sum(occ != osc.trace_shadow(o, d, tmax, 1, 32, opts.triangle_epsilon, threads=16)) <= n // 100_000
 
 
 def _binary_tree(nodes):
