@@ -69,6 +69,8 @@ hipError_t launch_shade(const LaunchShape& ls, const ctd::DevScene& sc, const ct
 hipError_t launch_resolve(const LaunchShape& ls, const ctd::ViewDesc* views, const ctd::Segment* segs,
                           const ctd::ChunkHdr* hdr, uint32_t max_tasks, const ctd::Queues& q, float4* accum,
                           uint32_t* counts, hipStream_t s);
+// n bytes from device memory to `out`, the device address of pinned host memory.
+hipError_t launch_copy_out(const void* src, size_t n, void* out, hipStream_t s);
 hipError_t launch_tonemap(const float4* accum, uint32_t n, float samples, float4* out, hipStream_t s);
 hipError_t launch_tonemap8(const float4* accum, uint32_t n, float samples, uint32_t* out, hipStream_t s);
 // The fast node test's copy of a quad tree (8 float4 per node), its compact

@@ -747,8 +747,7 @@ int ct_read_accum(ct_ctx* c, float* rgba, size_t n_floats, int32_t* samples) {
     const size_t need = (size_t)c->width * c->height * 4;
     if (n_floats < need) return fail(c, CT_ERR_INVALID_ARG, "output buffer too small");
     (void)hipSetDevice(c->device);
-    HIPCHK(hipMemcpyAsync(rgba, c->accum, need * 4, hipMemcpyDeviceToHost, c->ln[0].stream), "read accumulator");
-    HIPCHK(hipStreamSynchronize(c->ln[0].stream), "read accumulator");
+    HIPCHK(c->read.copy(rgba, c->accum, need * 4, c->ln[0].stream), "read accumulator");
     if (samples) *samples = c->samples;
     return CT_OK;
 }
@@ -765,17 +764,6 @@ int ct_write_accum(ct_ctx* c, const float* rgba, size_t n_floats, int32_t sample
     return CT_OK;
 }
 
-// Device buffer for the tonemapped image, grown on demand and kept.
-static int image_buffer(ct_ctx* c, size_t bytes) {
-    if (c->image_bytes >= bytes) return CT_OK;
-    dfree(c, c->image);
-    c->image = nullptr;
-    c->image_bytes = 0;
-    const int r = dalloc(c, &c->image, bytes, "image");
-    if (r == CT_OK) c->image_bytes = bytes;
-    return r;
-}
-
 int ct_read_image(ct_ctx* c, float* rgba, size_t n_floats) {
     if (!c || !rgba) return CT_ERR_INVALID_ARG;
     if (!c->accum) return fail(c, CT_ERR_INVALID_ARG, "no frame buffer");
@@ -783,13 +771,14 @@ int ct_read_image(ct_ctx* c, float* rgba, size_t n_floats) {
     if (n_floats < npix * 4) return fail(c, CT_ERR_INVALID_ARG, "output buffer too small");
     (void)hipSetDevice(c->device);
     sync_lanes(c);
-    int r = image_buffer(c, npix * sizeof(float4));
-    if (r != CT_OK) return r;
-    hipError_t e = ctk::launch_tonemap(c->accum, (uint32_t)npix, (float)std::max(c->samples, 1), (float4*)c->image,
-                                       c->ln[0].stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(rgba, c->image, npix * sizeof(float4), hipMemcpyDeviceToHost, c->ln[0].stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->ln[0].stream);
-    if (e != hipSuccess) return hip_fail(c, e, "tonemap");
+    const hipStream_t s = c->ln[0].stream;
+    // the kernel writes to the pinned slots itself
+    HIPCHK(c->read.run(rgba, npix * sizeof(float4), s,
+                       [&](char* dev, size_t offset, size_t n) {
+                           return ctk::launch_tonemap(c->accum + offset / sizeof(float4), (uint32_t)(n / sizeof(float4)),
+                                                      (float)std::max(c->samples, 1), reinterpret_cast<float4*>(dev), s);
+                       }),
+           "tonemap");
     return CT_OK;
 }
 
@@ -800,13 +789,13 @@ int ct_read_image_rgba8(ct_ctx* c, uint8_t* rgba, size_t n_bytes) {
     if (n_bytes < npix * 4) return fail(c, CT_ERR_INVALID_ARG, "output buffer too small");
     (void)hipSetDevice(c->device);
     sync_lanes(c);
-    int r = image_buffer(c, npix * 4);
-    if (r != CT_OK) return r;
-    hipError_t e = ctk::launch_tonemap8(c->accum, (uint32_t)npix, (float)std::max(c->samples, 1), (uint32_t*)c->image,
-                                        c->ln[0].stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(rgba, c->image, npix * 4, hipMemcpyDeviceToHost, c->ln[0].stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->ln[0].stream);
-    if (e != hipSuccess) return hip_fail(c, e, "tonemap");
+    const hipStream_t s = c->ln[0].stream;
+    HIPCHK(c->read.run(rgba, npix * 4, s,
+                       [&](char* dev, size_t offset, size_t n) {
+                           return ctk::launch_tonemap8(c->accum + offset / 4, (uint32_t)(n / 4),
+                                                       (float)std::max(c->samples, 1), reinterpret_cast<uint32_t*>(dev), s);
+                       }),
+           "tonemap");
     return CT_OK;
 }
 
@@ -862,9 +851,8 @@ int ct_trace_rays(ct_ctx* c, const float* origins, const float* dirs, uint32_t n
         HIPCHK(ctk::launch_extend(c->shape, c->sc, to, q, ra, m, s), "extend");
         HIPCHK(hipStreamSynchronize(s), "trace rays");
         if (take_error(c)) return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded");
-        HIPCHK(hipMemcpyAsync(t_out + base, ra.t, 4 * (size_t)m, hipMemcpyDeviceToHost, s), "hits");
-        HIPCHK(hipMemcpyAsync(prim_out + base, ra.prim, 4 * (size_t)m, hipMemcpyDeviceToHost, s), "hits");
-        HIPCHK(hipStreamSynchronize(s), "hits");
+        HIPCHK(c->read.copy(t_out + base, ra.t, 4 * (size_t)m, s), "hits");
+        HIPCHK(c->read.copy(prim_out + base, ra.prim, 4 * (size_t)m, s), "hits");
     }
     return CT_OK;
 }
@@ -898,8 +886,7 @@ int ct_trace_shadow_rays(ct_ctx* c, const float* origins, const float* dirs, con
         HIPCHK(hipMemcpyAsync(d_d, dirs + 3 * (size_t)base, 12 * (size_t)m, hipMemcpyHostToDevice, s), "rays");
         HIPCHK(hipMemcpyAsync(d_t, tmax + base, 4 * (size_t)m, hipMemcpyHostToDevice, s), "rays");
         HIPCHK(ctk::launch_shadow_flags(c->shape, c->sc, to, q, ra, m, s), "shadow rays");
-        HIPCHK(hipMemcpyAsync(occluded_out + base, ra.occluded, m, hipMemcpyDeviceToHost, s), "occlusion flags");
-        HIPCHK(hipStreamSynchronize(s), "trace shadow rays");
+        HIPCHK(c->read.copy(occluded_out + base, ra.occluded, m, s), "occlusion flags");
         if (take_error(c)) return fail(c, CT_ERR_STACK_OVERFLOW, "traversal stack bound exceeded");
     }
     return CT_OK;
@@ -963,10 +950,8 @@ int ct_render_batch(ct_ctx* c, const ct_view* views, int32_t n_views, const ct_f
     r = run_paths(c, vd, runs, cap, arena, o, kRunGraph | (stats ? kRunClock : 0), &st);
     if (r == CT_OK) {
         for (int32_t i = 0; i < n_views && e == hipSuccess; ++i)
-            e = hipMemcpyAsync(views[i].accum_out, arena + vd[i].accum_offset,
-                               (size_t)views[i].width * views[i].height * sizeof(float4), hipMemcpyDeviceToHost,
-                               c->ln[0].stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->ln[0].stream);
+            e = c->read.copy(views[i].accum_out, arena + vd[i].accum_offset,
+                             (size_t)views[i].width * views[i].height * sizeof(float4), c->ln[0].stream);
         if (e != hipSuccess) r = hip_fail(c, e, "read batch accumulators");
     }
     dfree(c, arena);

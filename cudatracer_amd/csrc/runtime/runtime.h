@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -77,6 +79,63 @@ constexpr int kReadErr = ctd::kReadCounters;
 constexpr int kReadWork = ctd::kReadCounters + 2;  // 4 x uint64, 8-byte aligned
 constexpr int kReadWords = kReadWork + 8;
 
+namespace ctr {
+// Results to pageable host memory, through pinned slots: while the caller's
+// thread copies one slot to its place, the device fills the next ones.  The
+// runtime's own copy to pageable memory does the two in turn: 33 MB (a 1080p
+// float image, or a 4K byte image) 1.85 ms, pinned 0.59 ms, the thread's
+// memcpy 0.8-0.9 ms.  Textured 1080p frame with its float image 5.83 to 5.15
+// ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time; 2 or 8 MB, made at the first
+// use that needs as much (0.3 ms for 8 MB: results of up to 1 MB, where
+// there is little to overlap, are left to the runtime).
+class ReadBack {
+  public:
+    // bytes of results to dst, in parts; put(dev, offset, n) enqueues on
+    // stream s a kernel that writes the n bytes from `offset` on to a slot (its
+    // device address).  Offsets are multiples of 64 KiB.  s is idle when it
+    // returns.
+    template <class Put>
+    hipError_t run(void* dst, size_t bytes, hipStream_t s, Put put) {
+        hipError_t e = init(bytes <= kSlot ? kSlot : kSlots * kSlot);
+        // up to a slot in one part (a further part's launch and wait cost what
+        // the overlap gives); above, four at least
+        const size_t part = bytes <= kSlot ? kSlot : std::min(kSlot, (bytes / kSlots + kGrain - 1) / kGrain * kGrain);
+        const size_t n = (bytes + part - 1) / part;
+        auto size = [&](size_t k) { return std::min(part, bytes - k * part); };
+        for (size_t put_n = 0, k = 0; k < n && e == hipSuccess; ++k) {
+            for (; put_n < n && put_n < k + kSlots && e == hipSuccess; ++put_n) {
+                const size_t o = put_n % kSlots * kSlot;
+                e = put(dev_ + o, put_n * part, size(put_n));
+                if (e == hipSuccess) e = hipEventRecord(ev_[put_n % kSlots], s);
+            }
+            if (e == hipSuccess) e = hipEventSynchronize(ev_[k % kSlots]);
+            if (e == hipSuccess) std::memcpy(static_cast<char*>(dst) + k * part, host_ + k % kSlots * kSlot, size(k));
+        }
+        const hipError_t f = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : f;
+    }
+    // device memory
+    hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        if (bytes <= kDirect) {
+            const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+            const hipError_t f = hipStreamSynchronize(s);
+            return e != hipSuccess ? e : f;
+        }
+        return run(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
+            return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
+        });
+    }
+    void release();
+
+  private:
+    static constexpr size_t kSlots = 4, kSlot = 2u << 20, kGrain = 64u << 10, kDirect = 1u << 20;
+    hipError_t init(size_t bytes);
+    size_t bytes_ = 0;
+    char *host_ = nullptr, *dev_ = nullptr;
+    hipEvent_t ev_[kSlots] = {};
+};
+}  // namespace ctr
+
 struct ct_ctx {
     int device = 0;
     Lane ln[kLanes];
@@ -103,8 +162,7 @@ struct ct_ctx {
     int width = 0, height = 0;
     int32_t samples = 0;
     float4* accum = nullptr;
-    void* image = nullptr;  // tonemapped image of ct_read_image[_rgba8], kept between calls
-    size_t image_bytes = 0;
+    ctr::ReadBack read;  // results on their way to the caller's arrays
 
     // path state: buffers of kLanes * lane_cap slots, lane k uses [k * lane_cap, (k + 1) * lane_cap)
     uint32_t lane_cap = 0;

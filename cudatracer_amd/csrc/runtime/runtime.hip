@@ -155,6 +155,29 @@ bool pinned_words(size_t words, uint32_t** host, uint32_t** dev) {
     return true;
 }
 
+hipError_t ReadBack::init(size_t bytes) {
+    if (bytes_ >= bytes) return hipSuccess;
+    release();
+    hipError_t e = hipHostMalloc((void**)&host_, bytes, hipHostMallocMapped);
+    if (e != hipSuccess) host_ = nullptr;
+    else e = hipHostGetDevicePointer((void**)&dev_, host_, 0);
+    for (hipEvent_t& ev : ev_)
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) release();
+    else bytes_ = bytes;
+    return e;
+}
+
+void ReadBack::release() {
+    for (hipEvent_t& ev : ev_) {
+        if (ev) (void)hipEventDestroy(ev);
+        ev = nullptr;
+    }
+    if (host_) (void)hipHostFree(host_);
+    host_ = dev_ = nullptr;
+    bytes_ = 0;
+}
+
 int ensure_paths(ct_ctx* c, uint32_t cap) {
     cap = std::max<uint32_t>(cap, 64u);
     const uint32_t threads = (uint32_t)(c->shape.trace_blocks * c->shape.block);
@@ -863,6 +886,7 @@ void ct_ctx_destroy(ct_ctx* c) {
     for (auto& a : c->allocs) (void)hipFree(a.first);
     c->allocs.clear();
     if (c->h_flag) (void)hipHostFree(c->h_flag);
+    c->read.release();
     for (Lane& L : c->ln) {
         if (L.h_read) (void)hipHostFree(L.h_read);
         if (L.h_stage) (void)hipHostFree(L.h_stage);

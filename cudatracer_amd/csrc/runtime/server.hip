@@ -111,6 +111,7 @@ struct ct_server {
     bool stop = false, worker_done = false;
     std::deque<uint64_t> to_copy;  // finished requests awaiting copy-out
     hipStream_t copy_stream = nullptr;
+    ReadBack read;  // the copier's
     uint64_t next_id = 1;
     std::map<uint64_t, Req> reqs;
     std::deque<uint64_t> pending;
@@ -161,8 +162,7 @@ void ct_server::copy_loop() {
         float* dst = q.result.data();  // map nodes stay put while unlocked
         lk.unlock();
         // the chunk that finished this request was synchronised by the worker
-        hipError_t e = hipMemcpyAsync(dst, arena_ptr + off, n * sizeof(float), hipMemcpyDeviceToHost, copy_stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(copy_stream);
+        const hipError_t e = read.copy(dst, arena_ptr + off, n * sizeof(float), copy_stream);
         lk.lock();
         finish(q, e == hipSuccess ? CT_OK : CT_ERR_DEVICE);
     }
@@ -440,6 +440,7 @@ void ct_server_destroy(ct_server* s) {
     if (s->worker.joinable()) s->worker.join();
     if (s->copier.joinable()) s->copier.join();
     sync_lanes(s->ctx);
+    s->read.release();
     if (s->copy_stream) (void)hipStreamDestroy(s->copy_stream);
     dfree(s->ctx, s->arena_ptr);
     delete s;
