@@ -19,11 +19,11 @@ struct LaunchShape {
     // Eighths of the resident blocks that the frame loop's persistent
     // traversal grids (grid2 ... gridc) fill.  Below 8 the other lane's shade
     // kernel runs beside a traversal launch instead of waiting for its waves
-    // to retire: 5 gave the shortest frames both on the 259K-triangle atrium
-    // (cache-resident; +4% over 8) and on the 7.24M-triangle sphere (bound by
-    // memory latency; +1%).  The ray-level launches always fill every slot
-    // (full2 ...).
-    int trace_fill = 5;
+    // to retire.  3, 4, 5 and 6: the 259K-triangle atrium at 1080p 3.37, 3.31,
+    // 3.37 and 3.41 ms, the 7.24M-triangle sphere at 4K 7.25, 6.83, 6.93 and
+    // 6.87, 16 views of the small box 66.3, 63.0, 63.5 and 63.1.  The ray-level
+    // launches always fill every slot (full2 ...).
+    int trace_fill = 4;
     int full2 = 1024, full4 = 1024, full8 = 1024, fullc = 1024;
     int shade_blocks = 1024;  // grid-stride grid of shade
     int max_blocks = 65536;   // cap for the simple grid-stride kernels
