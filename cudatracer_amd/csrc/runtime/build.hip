@@ -51,6 +51,13 @@ constexpr int kBinWords = 3 * kBins * 7;  // per axis and bin: ordered min xyz, 
 constexpr uint32_t kMaxPrims = 4;  // BVHNode.cu:6
 constexpr int kMaxDepth = 64;      // BVHNode.cu:7; the root has depth 2
 constexpr uint32_t kRank = 0x7FFFFFFFu;
+constexpr int kTile = 1024;                // nodes (threads) per block of a level's finish
+constexpr uint32_t kOneBlock = 8 * kTile;  // levels up to this size are finished by one block
+
+// Words of the build's counters: error bits, slots on long chains and the
+// longest of their nodes.  And of what the host reads after a level.
+enum : uint32_t { kCntErr, kCntPending, kCntLongest, kCounts = 16 };
+enum : uint32_t { kHostSplit, kHostTiny, kHostSmall, kHostChunks, kHostErr, kHostPending, kHostLongest, kHostS, kHostSQ };
 
 // error bits
 constexpr uint32_t kErrNoPlane = 1;    // a split without a finite candidate (extent overflow)
@@ -97,7 +104,7 @@ __device__ __forceinline__ float area(const float* mn, const float* mx) {
     const float a = e0 * e1 + e0 * e2 + e1 * e2;
     return a > 0.0f ? a : 0.0f;
 }
-__device__ __forceinline__ bool active(uint32_t count, int level) {
+__host__ __device__ inline bool active(uint32_t count, int level) {
     return count >= kMaxPrims && level + 2 < kMaxDepth;
 }
 __device__ __forceinline__ float centroid(const float4& lo, const float4& hi, uint32_t axis) {
@@ -392,8 +399,39 @@ __global__ __launch_bounds__(kBlock) void k_init(Geo g, Slots b, uint32_t n, flo
     }
 }
 
+// Which of the three node kernels splits a node (tiny: one wave, small: one
+// workgroup, large: chunks), if it tries to split (count >= 4, depth < 64):
+// one tiny, one small, or its chunks.
+struct Class {
+    uint32_t tiny, small, chunks;
+};
+__host__ __device__ inline Class class_of(uint32_t count, int level) {
+    if (!active(count, level)) return {0u, 0u, 0u};
+    if (count <= kTiny) return {1u, 0u, 0u};
+    const uint32_t n = (count + kChunk - 1) / kChunk;
+    return n == 1 ? Class{0u, 1u, 0u} : Class{0u, 0u, n};
+}
+// A level's work lists, by node index within the level: the tiny and the small
+// nodes, the first chunk of every node, the nodes' split flags and flags of
+// long swap chains (two sets, for even and odd levels).
+struct Plan {
+    uint32_t *tiny, *small, *chunk, *split, *jflag;
+};
+// Node j's entries, given how many tiny and small nodes and chunks come before.
+__device__ void plan_node(const Plan& p, uint32_t j, uint32_t count, int level, uint32_t tiny, uint32_t small,
+                          uint32_t chunk) {
+    const Class c = class_of(count, level);
+    if (c.tiny) p.tiny[tiny] = j;
+    if (c.small) p.small[small] = j;
+    p.chunk[j] = chunk;
+    p.split[j] = 0;
+    p.jflag[j] = 0;
+}
+
 // Root record: CalculateBounds over all primitives (BVHNode.cu:25-38).
-__global__ __launch_bounds__(kBlock) void k_root(const float* part, uint32_t nparts, uint32_t n, NodeRec* root) {
+__global__ __launch_bounds__(kBlock) void k_root(const float* part, uint32_t nparts, uint32_t n, NodeRec* root,
+                                                 Plan first, uint32_t* cnt) {
+    if (threadIdx.x < kCounts) cnt[threadIdx.x] = 0;
     __shared__ float s_v[kBlock][6];
     float v[6] = {1e34f, 1e34f, 1e34f, -1e34f, -1e34f, -1e34f};
     for (uint32_t p = threadIdx.x; p < nparts; p += kBlock)
@@ -409,34 +447,9 @@ __global__ __launch_bounds__(kBlock) void k_root(const float* part, uint32_t npa
         if (k == 0) {
             root->first = 0;
             root->count = n;
+            plan_node(first, 0, n, 0, 0, 0, 0);
         }
     }
-}
-
-// Per level node: chunk counts of the nodes that try to split (count >= 4,
-// depth < 64); clears the split flag.
-// Per level node: which of the three node kernels splits it (tiny: one wave,
-// single: one workgroup, multi: chunks), for the nodes that try to split
-// (count >= 4, depth < 64); clears the split flag.
-__global__ void k_plan(const NodeRec* nodes, uint32_t n, int level, uint32_t* nt, uint32_t* ns, uint32_t* nm,
-                       uint32_t* split) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t count = nodes[j].count;
-    const bool act = active(count, level);
-    const uint32_t nch = (count + kChunk - 1) / kChunk;
-    nt[j] = act && count <= kTiny ? 1u : 0u;
-    ns[j] = act && count > kTiny && nch == 1 ? 1u : 0u;
-    nm[j] = act && nch > 1 ? nch : 0u;
-    split[j] = 0;
-}
-
-__global__ void k_lists(uint32_t n, const uint32_t* nt, const uint32_t* off_t, const uint32_t* ns,
-                        const uint32_t* off_s, uint32_t* tch, uint32_t* sch) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    if (nt[j]) tch[off_t[j]] = j;
-    if (ns[j]) sch[off_s[j]] = j;
 }
 
 // Chunk c of the large nodes: its node is the last with chunk offset <= c.
@@ -707,26 +720,117 @@ __global__ void k_pending(uint32_t n, const uint32_t* pend_dst, const uint32_t* 
     move_slot(b, level & 1, g, J[pend_q[i]], d & 0x3FFFFFFFu, (d >> 31) != 0, ((d >> 30) & 1u) != 0);
 }
 
-// Children of the split nodes, in level order, appended after the level.
-__global__ void k_children(uint32_t n, uint32_t g0, uint32_t next0, const uint32_t* split, const uint32_t* off,
-                           const NodeRec* kid, NodeRec* nodes, int32_t* child) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    if (split[j]) {
-        const uint32_t o = next0 + 2 * off[j];
-        nodes[o] = kid[2 * (size_t)j];
-        nodes[o + 1] = kid[2 * (size_t)j + 1];
-        child[g0 + j] = (int32_t)o;
-    } else {
-        child[g0 + j] = -1;
+// A level's end: the children of its split nodes, in level order, appended
+// after the level, and their plan.  A node counts for the scans with its
+// children: splits, tiny nodes, small nodes and chunks.
+struct Finish {
+    const uint32_t* split;
+    const NodeRec* kid;
+    NodeRec* nodes;
+    int32_t* child;
+    uint32_t g0, n, next0;     // the level's first node and size, the next level's first
+    uint32_t max_nodes, max_level;
+    int level;
+    Plan next;
+    uint32_t *sums, *cnt;      // [4][tiles]
+    volatile uint32_t* host;   // pinned
+};
+__device__ void finish_values(const Finish& f, uint32_t j, uint32_t (&v)[4]) {
+    v[0] = v[1] = v[2] = v[3] = 0;
+    if (j >= f.n || !f.split[j]) return;
+    const Class a = class_of(f.kid[2 * (size_t)j].count, f.level + 1), b = class_of(f.kid[2 * (size_t)j + 1].count, f.level + 1);
+    v[0] = 1;
+    v[1] = a.tiny + b.tiny;
+    v[2] = a.small + b.small;
+    v[3] = a.chunks + b.chunks;
+}
+// off: the sums of the values before node j.
+__device__ void finish_node(const Finish& f, uint32_t j, bool split, const uint32_t (&off)[4]) {
+    if (j >= f.n) return;
+    const uint32_t k = 2 * off[0], o = f.next0 + k;
+    // lists that would not fit are left to the host's check of the totals
+    if (!split || k + 2 > f.max_level || o + 2 > f.max_nodes) {
+        f.child[f.g0 + j] = -1;
+        return;
+    }
+    const NodeRec a = f.kid[2 * (size_t)j], b = f.kid[2 * (size_t)j + 1];
+    f.nodes[o] = a;
+    f.nodes[o + 1] = b;
+    f.child[f.g0 + j] = (int32_t)o;
+    const Class c = class_of(a.count, f.level + 1);
+    plan_node(f.next, k, a.count, f.level + 1, off[1], off[2], off[3]);
+    plan_node(f.next, k + 1, b.count, f.level + 1, off[1] + c.tiny, off[2] + c.small, off[3] + c.chunks);
+}
+// Totals to the host, by one thread; the chains' counters for the next level.
+__device__ void finish_totals(const Finish& f, const uint32_t (&total)[4]) {
+    for (int k = 0; k < 4; ++k) f.host[kHostSplit + k] = total[k];
+    f.host[kHostErr] = f.cnt[kCntErr];
+    f.host[kHostPending] = f.cnt[kCntPending];
+    f.host[kHostLongest] = f.cnt[kCntLongest];
+    f.cnt[kCntPending] = f.cnt[kCntLongest] = 0;
+}
+// A level of up to kOneBlock nodes in one launch.  Bound by launches and
+// read-backs, not by their work: a build of 1,000,003 triangles was 680
+// dependent launches of 4 to 5 us and two waits a level (plan, three scans of
+// three kernels, lists; then a scan of the splits and the children).  With the
+// next level's plan made along with its nodes, one wait a level and the ranks
+// of small levels in one launch, the upload of a changed scene of that size went from
+// 11.9 to 10.1 ms, and a new context's of 100,003 with its export from 4.84 to 3.45.
+__global__ __launch_bounds__(kTile) void k_finish(Finish f) {
+    __shared__ uint32_t s_w[kTile / 64];
+    uint32_t carry[4] = {0, 0, 0, 0};
+    for (uint32_t base = 0; base < f.n; base += kTile) {
+        const uint32_t j = base + threadIdx.x;
+        uint32_t v[4], off[4];
+        finish_values(f, j, v);
+        for (int k = 0; k < 4; ++k) {
+            uint32_t tot;
+            off[k] = carry[k] + block_scan<kTile>(v[k], s_w, tot);
+            carry[k] += tot;
+        }
+        finish_node(f, j, v[0] != 0, off);
+    }
+    if (threadIdx.x == 0) finish_totals(f, carry);
+}
+// A larger one in three: tile sums, their scan, the nodes.
+__global__ __launch_bounds__(kTile) void k_finish_sums(Finish f) {
+    __shared__ uint32_t s_w[kTile / 64];
+    uint32_t v[4], tot;
+    finish_values(f, blockIdx.x * kTile + threadIdx.x, v);
+    for (int k = 0; k < 4; ++k) {
+        (void)block_scan<kTile>(v[k], s_w, tot);
+        if (threadIdx.x == 0) f.sums[k * gridDim.x + blockIdx.x] = tot;
     }
 }
+__global__ __launch_bounds__(kTile) void k_finish_top(Finish f, uint32_t tiles) {
+    __shared__ uint32_t s_w[kTile / 64];
+    uint32_t carry[4] = {0, 0, 0, 0};
+    for (int k = 0; k < 4; ++k)
+        for (uint32_t base = 0; base < tiles; base += kTile) {
+            const uint32_t i = base + threadIdx.x;
+            uint32_t tot;
+            const uint32_t v = i < tiles ? f.sums[k * tiles + i] : 0u, ex = block_scan<kTile>(v, s_w, tot);
+            if (i < tiles) f.sums[k * tiles + i] = carry[k] + ex;
+            carry[k] += tot;
+        }
+    if (threadIdx.x == 0) finish_totals(f, carry);
+}
+__global__ __launch_bounds__(kTile) void k_finish_nodes(Finish f) {
+    __shared__ uint32_t s_w[kTile / 64];
+    const uint32_t j = blockIdx.x * kTile + threadIdx.x;
+    uint32_t v[4], off[4], tot;
+    finish_values(f, j, v);
+    for (int k = 0; k < 4; ++k) off[k] = f.sums[k * gridDim.x + blockIdx.x] + block_scan<kTile>(v[k], s_w, tot);
+    finish_node(f, j, v[0] != 0, off);
+}
+
+// Node ranges of the levels.
+struct Levels {
+    uint32_t n, first[kMaxDepth + 1];  // first[n]: the number of nodes
+};
 
 // Subtree counts: split nodes (S) and split nodes at even depth (SQ).
-__global__ void k_up(uint32_t g0, uint32_t n, int level, const int32_t* child, uint32_t* S, uint32_t* SQ) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t gi = g0 + j;
+__device__ void up_node(uint32_t gi, int level, const int32_t* child, uint32_t* S, uint32_t* SQ) {
     const int32_t c = child[gi];
     if (c < 0) {
         S[gi] = 0;
@@ -738,11 +842,8 @@ __global__ void k_up(uint32_t g0, uint32_t n, int level, const int32_t* child, u
 }
 
 // Preorder ranks: R among split nodes, Q among split nodes at even depth.
-__global__ void k_down(uint32_t g0, uint32_t n, int level, const int32_t* child, const uint32_t* S,
-                       const uint32_t* SQ, uint32_t* R, uint32_t* Q) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t gi = g0 + j;
+__device__ void down_node(uint32_t gi, int level, const int32_t* child, const uint32_t* S, const uint32_t* SQ,
+                          uint32_t* R, uint32_t* Q) {
     const int32_t c = child[gi];
     if (c < 0) return;
     R[c] = R[gi] + 1;
@@ -759,6 +860,31 @@ __global__ void k_down(uint32_t g0, uint32_t n, int level, const int32_t* child,
                 off += SQ[gc];
             }
         }
+    }
+}
+
+// Levels [a, b): one of any size by its blocks, or a run of small ones by one
+// block, from the last up (k_up) or the first down (k_down).  Level 0's k_up
+// also gives the host the tree's counts and starts the ranks.
+__global__ __launch_bounds__(kTile) void k_up(Levels lv, int a, int b, const int32_t* child, uint32_t* S, uint32_t* SQ,
+                                              uint32_t* R, uint32_t* Q, volatile uint32_t* host) {
+    for (int l = b - 1; l >= a; --l) {
+        for (uint32_t gi = lv.first[l] + blockIdx.x * kTile + threadIdx.x; gi < lv.first[l + 1]; gi += gridDim.x * kTile)
+            up_node(gi, l, child, S, SQ);
+        __syncthreads();
+    }
+    if (a == 0 && threadIdx.x == 0) {
+        host[kHostS] = S[0];
+        host[kHostSQ] = SQ[0];
+        R[0] = Q[0] = 0;
+    }
+}
+__global__ __launch_bounds__(kTile) void k_down(Levels lv, int a, int b, const int32_t* child, const uint32_t* S,
+                                                const uint32_t* SQ, uint32_t* R, uint32_t* Q) {
+    for (int l = a; l < b; ++l) {
+        for (uint32_t gi = lv.first[l] + blockIdx.x * kTile + threadIdx.x; gi < lv.first[l + 1]; gi += gridDim.x * kTile)
+            down_node(gi, l, child, S, SQ, R, Q);
+        __syncthreads();
     }
 }
 
@@ -779,11 +905,7 @@ __device__ ct_bvh_node out_rec(const NodeRec& r, const int32_t* child, const uin
 }
 
 // Binary nodes: the children pair of the split node of rank r at 2 + 2r.
-__global__ void k_emit2(uint32_t g0, uint32_t n, const NodeRec* nodes, const int32_t* child, const uint32_t* R,
-                        ct_bvh_node* out) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t gi = g0 + j;
+__device__ void emit2(uint32_t gi, const NodeRec* nodes, const int32_t* child, const uint32_t* R, ct_bvh_node* out) {
     const int32_t c = child[gi];
     if (gi == 0) {
         out[0] = out_rec(nodes[0], child, R, 0);
@@ -810,11 +932,7 @@ __device__ void set_slot(ct_mbvh_node& m, int s, const NodeRec& r) {
 
 // Quad nodes (GetBVHNodeInfo + MergeNodes): a split node at even depth takes
 // its leaf children and the children of its interior children, left first.
-__global__ void k_emit4(uint32_t g0, uint32_t n, const NodeRec* nodes, const int32_t* child, const uint32_t* Q,
-                        ct_mbvh_node* out) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t gi = g0 + j;
+__device__ void emit4(uint32_t gi, const NodeRec* nodes, const int32_t* child, const uint32_t* Q, ct_mbvh_node* out) {
     const int32_t c = child[gi];
     ct_mbvh_node m;
     for (int s = 0; s < 4; ++s) {
@@ -855,6 +973,17 @@ __global__ void k_emit4(uint32_t g0, uint32_t n, const NodeRec* nodes, const int
     out[Q[gi]] = m;
 }
 
+// Both trees' nodes, every level in one launch.
+__global__ void k_emit(Levels lv, const NodeRec* nodes, const int32_t* child, const uint32_t* R, const uint32_t* Q,
+                       ct_bvh_node* out2, ct_mbvh_node* out4) {
+    const uint32_t gi = blockIdx.x * blockDim.x + threadIdx.x;
+    if (gi >= lv.first[lv.n]) return;
+    emit2(gi, nodes, child, R, out2);
+    uint32_t l = 0;
+    while (gi >= lv.first[l + 1]) ++l;
+    if (!(l & 1)) emit4(gi, nodes, child, Q, out4);
+}
+
 // A leaf root (fewer than 4 primitives): records straight from slot order.
 __global__ void k_root_leaf(Geo g, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -875,8 +1004,8 @@ __global__ __launch_bounds__(kBlock) void k_scan_sums(const uint32_t* in, uint32
     if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// In-place exclusive scan of the tile sums (one block); total to *total.
-__global__ __launch_bounds__(kBlock) void k_scan_top(uint32_t* sums, uint32_t nt, uint32_t* total) {
+// In-place exclusive scan of the tile sums (one block).
+__global__ __launch_bounds__(kBlock) void k_scan_top(uint32_t* sums, uint32_t nt) {
     __shared__ uint32_t s_w[kBlock / 64];
     uint32_t carry = 0;
     for (uint32_t base = 0; base < nt; base += kBlock) {
@@ -887,7 +1016,6 @@ __global__ __launch_bounds__(kBlock) void k_scan_top(uint32_t* sums, uint32_t nt
         if (i < nt) sums[i] = carry + ex;
         carry += tot;
     }
-    if (threadIdx.x == 0) *total = carry;
 }
 
 __global__ __launch_bounds__(kBlock) void k_scan_out(const uint32_t* in, uint32_t n, const uint32_t* sums,
@@ -906,6 +1034,19 @@ __global__ __launch_bounds__(kBlock) void k_scan_out(const uint32_t* in, uint32_
             out[base + k] = run;
             run += v[k];
         }
+}
+
+// Exclusive scan by one block.
+__global__ __launch_bounds__(kTile) void k_scan_one(const uint32_t* in, uint32_t n, uint32_t* out) {
+    __shared__ uint32_t s_w[kTile / 64];
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < n; base += kTile) {
+        const uint32_t i = base + threadIdx.x;
+        uint32_t tot;
+        const uint32_t ex = block_scan<kTile>(i < n ? in[i] : 0u, s_w, tot);
+        if (i < n) out[i] = carry + ex;
+        carry += tot;
+    }
 }
 
 inline uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)std::max<uint64_t>(1, (n + per - 1) / per); }
@@ -961,9 +1102,8 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
     const uint64_t W = std::max<uint64_t>(4, (uint64_t)N / 2 + 2);  // nodes of one level
     const uint64_t Nn = 2 * (uint64_t)N + 2;                        // nodes of all levels
     const uint64_t Mc = 2 * (uint64_t)N / kChunk + 2;               // chunks of large nodes
-    uint32_t *ref0, *ref1, *rf, *nt, *ns, *nm, *off_t, *off_s, *off_m, *split, *coff, *tch, *sch, *mch_node,
-        *mch_k, *part, *J0, *J1, *pend_dst, *pend_q, *jflag,
-        *chunk_left, *chunk_pre, *S, *SQ, *R, *Q, *sums, *cnt;
+    uint32_t *ref0, *ref1, *rf, *split0, *split1, *jflag0, *jflag1, *tch, *sch, *off_m, *mch_node, *mch_k, *part, *J0,
+        *J1, *pend_dst, *pend_q, *chunk_left, *chunk_pre, *S, *SQ, *R, *Q, *sums, *cnt;
     float4 *box0, *box1;
     NodeRec *nodes, *kid;
     int32_t* child;
@@ -981,22 +1121,18 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
     GET(J1, N);
     GET(pend_dst, N);
     GET(pend_q, N);
-    GET(jflag, W);
+    GET(jflag0, W);
+    GET(jflag1, W);
+    GET(split0, W);
+    GET(split1, W);
     GET(nodes, Nn);
     GET(child, Nn);
     GET(S, Nn);
     GET(SQ, Nn);
     GET(R, Nn);
     GET(Q, Nn);
-    GET(nt, W);
-    GET(off_t, W);
     GET(tch, W);
-    GET(ns, W);
-    GET(nm, W);
-    GET(off_s, W);
     GET(off_m, W);
-    GET(split, W);
-    GET(coff, W);
     GET(sch, W);
     GET(kid, 2 * W);
     GET(dec, W);
@@ -1005,8 +1141,8 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
     GET(chunk_left, Mc);
     GET(chunk_pre, Mc);
     GET(part, Mc * kBinWords);
-    GET(sums, blocks_for(Nn, kScanTile) + 1);
-    GET(cnt, 16);
+    GET(sums, 4 * (uint64_t)blocks_for(std::max(W, Mc), kScanTile));
+    GET(cnt, kCounts);
     GET(rpart, (uint64_t)nblk_init * 6);
 #undef GET
     if ((r = sc.alloc("build: scratch")) != CT_OK) return r;
@@ -1018,100 +1154,93 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
         tris = static_cast<float4*>(p);
         out->tris = tris;
     }
-    uint32_t* h = nullptr;  // pinned read-back
-    BCHK(hipHostMalloc((void**)&h, 64, hipHostMallocDefault), "build: pinned read-back");
-    struct HostFree {
-        uint32_t* p;
-        ~HostFree() { (void)hipHostFree(p); }
-    } hf{h};
+    // pinned words that the kernels write, and the lane's first two events:
+    // nothing else runs on it
+    volatile uint32_t* h = c->h_flag + kHostWords;
+    volatile uint32_t* hd = c->h_flag_dev + kHostWords;
+    const hipEvent_t e0 = c->ln[0].ev[0], e1 = c->ln[0].ev[1];
 
-    hipEvent_t e0, e1;
-    BCHK(hipEventCreate(&e0), "build: event");
-    BCHK(hipEventCreate(&e1), "build: event");
-    struct EvFree {
-        hipEvent_t a, b;
-        ~EvFree() {
-            (void)hipEventDestroy(a);
-            (void)hipEventDestroy(b);
-        }
-    } ef{e0, e1};
-
-    BCHK(hipMemsetAsync(cnt, 0, 16 * sizeof(uint32_t), s), "build: counters");
     BCHK(hipEventRecord(e0, s), "build: event");
 
     const Slots slots{{box0, box1}, {ref0, ref1}};
     const Geo geo{d_vert, d_idx, tris};
     k_init<<<nblk_init, kBlock, 0, s>>>(geo, slots, N, rpart);
     BLAUNCH("build: init");
-    k_root<<<1, kBlock, 0, s>>>(rpart, nblk_init, N, nodes);
+    const Plan plans[2] = {{tch, sch, off_m, split0, jflag0}, {tch, sch, off_m, split1, jflag1}};
+    k_root<<<1, kBlock, 0, s>>>(rpart, nblk_init, N, nodes, plans[0], cnt);
     BLAUNCH("build: root");
 
-    // exclusive scan of n words into out; total into cnt[slot]
-    auto scan = [&](const uint32_t* in, uint32_t* outp, uint32_t n, int slot) -> int {
-        const uint32_t nt = blocks_for(n, kScanTile);
-        k_scan_sums<<<nt, kBlock, 0, s>>>(in, n, sums);
-        k_scan_top<<<1, kBlock, 0, s>>>(sums, nt, cnt + slot);
-        k_scan_out<<<nt, kBlock, 0, s>>>(in, n, sums, outp);
+    // exclusive scan of n words
+    auto scan = [&](const uint32_t* in, uint32_t* outp, uint32_t n) -> int {
+        if (n <= kOneBlock) {
+            k_scan_one<<<1, kTile, 0, s>>>(in, n, outp);
+        } else {
+            const uint32_t nt = blocks_for(n, kScanTile);
+            k_scan_sums<<<nt, kBlock, 0, s>>>(in, n, sums);
+            k_scan_top<<<1, kBlock, 0, s>>>(sums, nt);
+            k_scan_out<<<nt, kBlock, 0, s>>>(in, n, sums, outp);
+        }
         BLAUNCH("build: scan");
         return CT_OK;
     };
-    auto readback = [&](int words) -> int {
-        BCHK(hipMemcpyAsync(h, cnt, (size_t)words * 4, hipMemcpyDeviceToHost, s), "build: read-back");
-        BCHK(hipStreamSynchronize(s), "build: level");
-        return CT_OK;
-    };
 
-    std::vector<std::pair<uint32_t, uint32_t>> levels;  // [g0, n) per level
+    Levels levels{};
     uint32_t long_chains = 0, jump_rounds = 0;
     uint32_t g0 = 0, n = 1;
     const uint32_t tpb = 256;
+    Class todo = class_of(N, 0);  // the level's tiny and small nodes and its chunks
     for (int level = 0; n > 0; ++level) {
-        levels.emplace_back(g0, n);
+        levels.first[levels.n++] = g0;
         const NodeRec* lv = nodes + g0;
-        k_plan<<<blocks_for(n, tpb), tpb, 0, s>>>(lv, n, level, nt, ns, nm, split);
-        BLAUNCH("build: plan");
-        if ((r = scan(ns, off_s, n, 0)) || (r = scan(nm, off_m, n, 1)) || (r = scan(nt, off_t, n, 6)) ||
-            (r = readback(7)))
-            return r;
-        const uint32_t Ts = h[0], Tm = h[1], Tt = h[6];
+        const Plan& plan = plans[level & 1];
+        const uint32_t Tt = todo.tiny, Ts = todo.small, Tm = todo.chunks;
         if (Ts > W || Tt > W || Tm > Mc) return fail(c, CT_ERR_DEVICE, "build: chunk list overflow");
-        k_lists<<<blocks_for(n, tpb), tpb, 0, s>>>(n, nt, off_t, ns, off_s, tch, sch);
-        BLAUNCH("build: node lists");
         if (Tt) {
-            k_single<64, kTiny><<<Tt, 64, 0, s>>>(lv, level, tch, slots, geo, kid, split, cnt + 4);
+            k_single<64, kTiny><<<Tt, 64, 0, s>>>(lv, level, tch, slots, geo, kid, plan.split, cnt + kCntErr);
             BLAUNCH("build: tiny nodes");
         }
         if (Ts) {
-            k_single<kBlock, kChunk><<<Ts, kBlock, 0, s>>>(lv, level, sch, slots, geo, kid, split, cnt + 4);
+            k_single<kBlock, kChunk><<<Ts, kBlock, 0, s>>>(lv, level, sch, slots, geo, kid, plan.split, cnt + kCntErr);
             BLAUNCH("build: small nodes");
         }
         if (Tm) {
             k_mchunks<<<blocks_for(Tm, tpb), tpb, 0, s>>>(Tm, n, off_m, mch_node, mch_k);
             k_mbin<<<Tm, kBlock, 0, s>>>(lv, level, mch_node, mch_k, slots, part);
             k_mreduce<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, part);
-            k_mdecide<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, part, kid, split, dec, cnt + 4);
+            k_mdecide<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, part, kid, plan.split, dec, cnt + kCntErr);
             k_mrank<<<Tm, kBlock, 0, s>>>(lv, level, mch_node, mch_k, slots, dec, rf, chunk_left);
             BLAUNCH("build: large nodes");
-            if ((r = scan(chunk_left, chunk_pre, Tm, 3))) return r;
-            BCHK(hipMemsetAsync(cnt + 7, 0, 8, s), "build: counters");
-            BCHK(hipMemsetAsync(jflag, 0, (size_t)n * 4, s), "build: counters");
+            if ((r = scan(chunk_left, chunk_pre, Tm))) return r;
             k_mmove<<<Tm, kBlock, 0, s>>>(lv, level, mch_node, mch_k, slots, geo, dec, rf, chunk_pre, chunk_left,
-                                          cnt + 4, cnt + 7, pend_dst, pend_q, jflag, cnt + 8);
+                                          cnt + kCntErr, cnt + kCntPending, pend_dst, pend_q, plan.jflag,
+                                          cnt + kCntLongest);
             BLAUNCH("build: large nodes");
         }
-        if ((r = scan(split, coff, n, 2)) || (r = readback(9))) return r;
-        const uint32_t npend = Tm ? h[7] : 0;
+        const uint32_t next0 = g0 + n;
+        const Finish fin{plan.split, kid, nodes, child, g0, n, next0, (uint32_t)Nn, (uint32_t)W, level, plans[(level + 1) & 1],
+                         sums, cnt, hd};
+        if (n <= kOneBlock) {
+            k_finish<<<1, kTile, 0, s>>>(fin);
+        } else {
+            const uint32_t tiles = blocks_for(n, kTile);
+            k_finish_sums<<<tiles, kTile, 0, s>>>(fin);
+            k_finish_top<<<1, kTile, 0, s>>>(fin, tiles);
+            k_finish_nodes<<<tiles, kTile, 0, s>>>(fin);
+        }
+        BLAUNCH("build: children");
+        BCHK(hipStreamSynchronize(s), "build: level");
+        const uint32_t npend = h[kHostPending];
         if (npend) {
             // swap chains longer than the in-kernel chase: pointer jumping to
             // their ends in the nodes that have them; a chain is shorter than
             // its node, so ceil(log2(largest such node)) rounds reach every end
             long_chains += npend;
-            k_jinit<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, jflag, rf, chunk_pre, J0);
+            k_jinit<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, plan.jflag, rf, chunk_pre, J0);
             BLAUNCH("build: chain jumps");
             uint32_t* Jc = J0;
             uint32_t* Jn = J1;
-            for (uint32_t span = 1; span < h[8]; span *= 2) {
-                k_jump<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, jflag, Jc, Jn);
+            for (uint32_t span = 1; span < h[kHostLongest]; span *= 2) {
+                k_jump<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, plan.jflag, Jc, Jn);
                 BLAUNCH("build: chain jumps");
                 std::swap(Jc, Jn);
                 ++jump_rounds;
@@ -1119,13 +1248,11 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
             k_pending<<<blocks_for(npend, tpb), tpb, 0, s>>>(npend, pend_dst, pend_q, Jc, slots, level, geo);
             BLAUNCH("build: long chains");
         }
-        if (h[4]) return fail(c, CT_ERR_INVALID_SCENE, "device build: scene extent overflows the SAH cost");
-        const uint32_t nsplit = h[2];
-        const uint32_t next0 = g0 + n;
+        if (h[kHostErr]) return fail(c, CT_ERR_INVALID_SCENE, "device build: scene extent overflows the SAH cost");
+        const uint32_t nsplit = h[kHostSplit];
         if ((uint64_t)next0 + 2 * (uint64_t)nsplit > Nn || 2 * (uint64_t)nsplit > W)
             return fail(c, CT_ERR_DEVICE, "build: node list overflow");
-        k_children<<<blocks_for(n, tpb), tpb, 0, s>>>(n, g0, next0, split, coff, kid, nodes, child);
-        BLAUNCH("build: children");
+        todo = {h[kHostTiny], h[kHostSmall], h[kHostChunks]};
         if (level == 0 && nsplit == 0) {
             k_root_leaf<<<blocks_for(N, tpb), tpb, 0, s>>>(geo, N);
             BLAUNCH("build: leaf root");
@@ -1134,38 +1261,35 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
         n = 2 * nsplit;
         if (level + 1 >= kMaxDepth) return fail(c, CT_ERR_DEVICE, "build: level limit");
     }
-    const uint32_t n_levels = (uint32_t)levels.size();
-    // bottom-up subtree counts, top-down ranks
-    for (uint32_t L = n_levels; L-- > 0;) {
-        k_up<<<blocks_for(levels[L].second, tpb), tpb, 0, s>>>(levels[L].first, levels[L].second, (int)L, child, S, SQ);
+    const uint32_t n_levels = levels.n;
+    levels.first[n_levels] = g0;
+    // bottom-up subtree counts, top-down ranks: a launch for every large level
+    // and for every run of small ones
+    auto small = [&](int l) { return levels.first[l + 1] - levels.first[l] <= kOneBlock; };
+    auto grid = [&](int l) { return small(l) ? 1u : blocks_for(levels.first[l + 1] - levels.first[l], kTile); };
+    for (int b = (int)n_levels, a; b > 0; b = a) {
+        a = b - 1;
+        while (a > 0 && small(b - 1) && small(a - 1)) --a;
+        k_up<<<grid(a), kTile, 0, s>>>(levels, a, b, child, S, SQ, R, Q, hd);
         BLAUNCH("build: subtree counts");
     }
-    BCHK(hipMemsetAsync(R, 0, 4, s), "build: ranks");
-    BCHK(hipMemsetAsync(Q, 0, 4, s), "build: ranks");
-    for (uint32_t L = 0; L < n_levels; ++L) {
-        k_down<<<blocks_for(levels[L].second, tpb), tpb, 0, s>>>(levels[L].first, levels[L].second, (int)L, child, S,
-                                                                  SQ, R, Q);
+    for (int a = 0, b; a < (int)n_levels; a = b) {
+        b = a + 1;
+        while (b < (int)n_levels && small(a) && small(b)) ++b;
+        k_down<<<grid(a), kTile, 0, s>>>(levels, a, b, child, S, SQ, R, Q);
         BLAUNCH("build: ranks");
     }
-    BCHK(hipMemcpyAsync(cnt + 8, S, 4, hipMemcpyDeviceToDevice, s), "build: sizes");
-    BCHK(hipMemcpyAsync(cnt + 9, SQ, 4, hipMemcpyDeviceToDevice, s), "build: sizes");
-    if ((r = readback(10))) return r;
-    if (h[4] & kErrCount) return fail(c, CT_ERR_DEVICE, "device build: partition count mismatch");
-    const uint32_t n2 = 2 + 2 * h[8];
-    const uint32_t n4 = h[8] ? h[9] : 1;
+    BCHK(hipStreamSynchronize(s), "build: sizes");
+    if (h[kHostErr] & kErrCount) return fail(c, CT_ERR_DEVICE, "device build: partition count mismatch");
+    const uint32_t n2 = 2 + 2 * h[kHostS];
+    const uint32_t n4 = h[kHostS] ? h[kHostSQ] : 1;
     void *p2 = nullptr, *p4 = nullptr;
     if ((r = dalloc(c, &p2, (size_t)n2 * sizeof(ct_bvh_node), "binary nodes"))) return r;
     out->nodes2 = static_cast<ct_bvh_node*>(p2);
     if ((r = dalloc(c, &p4, (size_t)n4 * sizeof(ct_mbvh_node), "quad nodes"))) return r;
     out->nodes4 = static_cast<ct_mbvh_node*>(p4);
-    for (uint32_t L = 0; L < n_levels; ++L) {
-        k_emit2<<<blocks_for(levels[L].second, tpb), tpb, 0, s>>>(levels[L].first, levels[L].second, nodes, child, R,
-                                                                   out->nodes2);
-        if (!(L & 1))
-            k_emit4<<<blocks_for(levels[L].second, tpb), tpb, 0, s>>>(levels[L].first, levels[L].second, nodes, child,
-                                                                       Q, out->nodes4);
-        BLAUNCH("build: emit");
-    }
+    k_emit<<<blocks_for(g0, tpb), tpb, 0, s>>>(levels, nodes, child, R, Q, out->nodes2, out->nodes4);
+    BLAUNCH("build: emit");
     BCHK(hipEventRecord(e1, s), "build: event");
     BCHK(hipStreamSynchronize(s), "build: finish");
     float ms = 0.0f;

@@ -74,6 +74,7 @@ struct Lane {
     int tail = -1;     // the chunk's k_paths bounce, or -1
     bool paths = false;  // the chunk runs as whole paths (k_paths)
 };
+constexpr int kHostWords = 16;  // in ct_ctx::h_flag: the words of a tree build
 // h_read layout (uint32 words)
 constexpr int kReadErr = ctd::kReadCounters;
 constexpr int kReadWork = ctd::kReadCounters + 2;  // 4 x uint64, 8-byte aligned
@@ -169,7 +170,8 @@ struct ct_ctx {
     std::vector<void*> path_bufs;
     uint32_t spill_threads = 0;
 
-    // error flag of the allocation-free entry point (pinned; its device address)
+    // error flag of the allocation-free entry point (pinned; its device
+    // address), and from kHostWords on the words a tree build writes for the host
     uint32_t* h_flag = nullptr;
     uint32_t* h_flag_dev = nullptr;
     // this device's copy of the allocation-free entry point's scratch array

@@ -868,7 +868,7 @@ int ct_ctx_create(const ct_device_opts* opts, ct_ctx** out) {
             return CT_ERR_DEVICE;
         }
     }
-    if (!pinned_words(16, &c->h_flag, &c->h_flag_dev) || scratch_init(c) != CT_OK) {
+    if (!pinned_words(2 * kHostWords, &c->h_flag, &c->h_flag_dev) || scratch_init(c) != CT_OK) {
         ct_ctx_destroy(c);
         return CT_ERR_DEVICE;
     }

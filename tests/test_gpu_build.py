@@ -207,3 +207,18 @@ def test_shading_records_without_room_for_the_arrays(ct):
         frames.append(ctx.read_accum()[0])
         ctx.close()
     assert np.array_equal(_bits(frames[0]), _bits(frames[1]))
+
+
+@pytest.mark.parametrize("cells", [1024, 8192, 8193, 32_768, 33_000])
+def test_device_build_level_sizes(ct, gpu_ctx, cells):
+    """Levels of up to 8,192 nodes are finished by one block of 1,024 threads,
+    larger ones by one block a 1,024 nodes.  Separate cells of four small
+    triangles on a grid split in halves, so a level's size passes through the
+    powers of two up to `cells`: exactly at the tile and the one-block bound,
+    and a few nodes past them."""
+    i = np.arange(cells)
+    at = 10.0 * np.stack([i % 256, i // 256, np.zeros(cells)], 1)[:, None, None, :]
+    rng = np.random.default_rng(cells)
+    s = _soup(ct, (at + rng.uniform(0.0, 1.0, (cells, 4, 3, 3))).reshape(-1, 3, 3))
+    gpu_ctx.upload_build(s)
+    _assert_same_trees(gpu_ctx, s.arrays())
