@@ -27,9 +27,12 @@
 // A request's result does not depend on what it was batched with: the RNG is
 // keyed by (pixel, frame_base + sample, bounce) and samples are summed in
 // sample order.
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
+#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <map>
@@ -50,6 +53,28 @@ constexpr uint32_t kServerChunk = 1u << 23;
 
 enum ReqState { PENDING = 0, ACTIVE = 1, COPYING = 2, DONE = 3 };
 
+// A finished request's accumulator.  Not a vector: its zeroes, page by page
+// into fresh memory, took 6 of the 12 ms that the last 1080p request's way out
+// did.  Large pages from 4 MB on.
+struct Result {
+    float* data = nullptr;
+    size_t size = 0;  // floats
+    Result() = default;
+    Result(Result&& o) noexcept : data(o.data), size(o.size) { o.data = nullptr; }
+    ~Result() { std::free(data); }
+    bool alloc(size_t n) {
+        constexpr size_t kLarge = 2u << 20;
+        const size_t bytes = n * sizeof(float);
+        const bool large = bytes >= 2 * kLarge;
+        data = static_cast<float*>(large ? std::aligned_alloc(kLarge, (bytes + kLarge - 1) / kLarge * kLarge)
+                                         : std::malloc(bytes));
+        if (!data) return false;
+        if (large) (void)madvise(data, bytes, MADV_HUGEPAGE);
+        size = n;
+        return true;
+    }
+};
+
 struct Req {
     uint64_t id = 0;
     ct_request r{};
@@ -62,7 +87,7 @@ struct Req {
     double submit_ms = 0, admit_ms = 0, done_ms = 0;
     uint64_t rays = 0;
     bool cancel = false;
-    std::vector<float> result;
+    Result result;
 };
 
 // First-fit allocator over the accumulator arena (units: float4).
@@ -157,9 +182,12 @@ void ct_server::copy_loop() {
         Req& q = reqs[to_copy.front()];
         to_copy.pop_front();
         const size_t n = (size_t)q.r.width * q.r.height * 4;
-        q.result.resize(n);
+        if (!q.result.alloc(n)) {
+            finish(q, CT_ERR_OUT_OF_MEMORY);
+            continue;
+        }
         const uint64_t off = q.acc_off;
-        float* dst = q.result.data();  // map nodes stay put while unlocked
+        float* dst = q.result.data;  // map nodes stay put while unlocked
         lk.unlock();
         // the chunk that finished this request was synchronised by the worker
         const hipError_t e = read.copy(dst, arena_ptr + off, n * sizeof(float), copy_stream);
@@ -363,9 +391,9 @@ int ct_server_submit(ct_server* s, const ct_request* req, uint64_t* id) {
     q.total = total;
     q.footprint = fp;
     q.submit_ms = s->now();
-    s->reqs[q.id] = q;
-    s->pending.push_back(q.id);
     *id = q.id;
+    s->pending.push_back(*id);
+    s->reqs.emplace(*id, std::move(q));
     s->cv.notify_all();
     return CT_OK;
 }
@@ -392,8 +420,8 @@ int ct_server_poll(ct_server* s, uint64_t id, int32_t* done, ct_result* res, flo
     if (q.state != DONE) return CT_OK;
     fill_result(q, res);
     if (accum_out && q.status == CT_OK) {
-        if (n_floats < q.result.size()) return CT_ERR_INVALID_ARG;
-        std::memcpy(accum_out, q.result.data(), q.result.size() * sizeof(float));
+        if (n_floats < q.result.size) return CT_ERR_INVALID_ARG;
+        std::memcpy(accum_out, q.result.data, q.result.size * sizeof(float));
     }
     return CT_OK;
 }
