@@ -119,3 +119,37 @@ def test_odd_binary_trees(ct, orc, gpu_ctx, tree):
     o, d = chain_rays(1000, 9)
     d[::5] = [1.0, 0.0, 0.0]
     _same(gpu_ctx, osc, o, d, np.full(1000, 40.0, np.float32), opts, 0)
+
+
+@pytest.mark.parametrize("n", [5, 140_001])
+@pytest.mark.parametrize("levels", [14, 15, 16, 17, 40, 127])
+def test_deep_binary_stacks(ct, orc, gpu_ctx, levels, n):
+    """Every box around the scene, so each level leaves its right leaf on the
+    stack under the left child: up to the LDS part's 16 entries and past it, up
+    to 127 and the entry kept in a register, which is the bound."""
+    _binary_chain(ct, orc, gpu_ctx, levels, n)
+
+
+@pytest.mark.parametrize("n", [5, 140_001])
+def test_binary_stack_bound(ct, orc, gpu_ctx, n):
+    with pytest.raises(ct.CTError) as e:
+        _binary_chain(ct, orc, gpu_ctx, 128, n)
+    assert e.value.code == ct.CT_ERR_STACK_OVERFLOW
+
+
+def _binary_chain(ct, orc, gpu_ctx, levels, n):
+    arrays = chain_scene(ct, 64, seed=8)
+    assert len(arrays["prim_indices"]) > levels
+    nodes = [(2, -1), (0, 0)]
+    for k in range(levels):
+        left = (4 + 2 * k, -1) if k + 1 < levels else (levels, len(arrays["prim_indices"]) - levels)
+        nodes += [left, (k, 1)]
+    arrays["bvh"] = _binary_tree(nodes)
+    arrays["mbvh"] = np.zeros(0, np.uint8)
+    gpu_ctx.upload_view(ArrayView(ct, arrays).view)
+    osc = orc.Scene(arrays, build=False)
+    osc.set_trees(arrays["bvh"], arrays["mbvh"], arrays["prim_indices"])
+    opts = ct.default_opts()
+    opts.accel = ct.ACCEL_BVH2
+    o, d = chain_rays(n, 4)
+    _same(gpu_ctx, osc, o, d, np.full(n, 40.0, np.float32), opts, 0)
