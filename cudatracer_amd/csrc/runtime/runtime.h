@@ -86,21 +86,22 @@ namespace ctr {
 // runtime's own copy to pageable memory does the two in turn: 33 MB (a 1080p
 // float image, or a 4K byte image) 1.85 ms, pinned 0.59 ms, the thread's
 // memcpy 0.8-0.9 ms.  Textured 1080p frame with its float image 5.83 to 5.15
-// ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time; 2 or 8 MB, made at the first
-// use that needs as much (0.3 ms for 8 MB: results of up to 1 MB, where
-// there is little to overlap, are left to the runtime).
+// ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time.
+// 2 MB in all, made at the first use: a slot of 2 MB each served no better, and
+// pinning the 8 MB took 3 ms of a context's first image.  Results of up to 1 MB,
+// where there is little to overlap, are left to the runtime.
 class ReadBack {
   public:
     // bytes of results to dst, in parts; put(dev, offset, n) enqueues on
     // stream s a kernel that writes the n bytes from `offset` on to a slot (its
-    // device address).  Offsets are multiples of 64 KiB.  s is idle when it
+    // device address).  Offsets are multiples of 512 KiB.  s is idle when it
     // returns.
     template <class Put>
     hipError_t run(void* dst, size_t bytes, hipStream_t s, Put put) {
-        hipError_t e = init(bytes <= kSlot ? kSlot : kSlots * kSlot);
-        // up to a slot in one part (a further part's launch and wait cost what
-        // the overlap gives); above, four at least
-        const size_t part = bytes <= kSlot ? kSlot : std::min(kSlot, (bytes / kSlots + kGrain - 1) / kGrain * kGrain);
+        hipError_t e = init();
+        // what all slots hold in one part: a further part's launch and wait
+        // cost what the overlap would give
+        const size_t part = bytes <= kSlots * kSlot ? kSlots * kSlot : kSlot;
         const size_t n = (bytes + part - 1) / part;
         auto size = [&](size_t k) { return std::min(part, bytes - k * part); };
         for (size_t put_n = 0, k = 0; k < n && e == hipSuccess; ++k) {
@@ -129,9 +130,8 @@ class ReadBack {
     void release();
 
   private:
-    static constexpr size_t kSlots = 4, kSlot = 2u << 20, kGrain = 64u << 10, kDirect = 1u << 20;
-    hipError_t init(size_t bytes);
-    size_t bytes_ = 0;
+    static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
+    hipError_t init();
     char *host_ = nullptr, *dev_ = nullptr;
     hipEvent_t ev_[kSlots] = {};
 };

@@ -155,16 +155,14 @@ bool pinned_words(size_t words, uint32_t** host, uint32_t** dev) {
     return true;
 }
 
-hipError_t ReadBack::init(size_t bytes) {
-    if (bytes_ >= bytes) return hipSuccess;
-    release();
-    hipError_t e = hipHostMalloc((void**)&host_, bytes, hipHostMallocMapped);
+hipError_t ReadBack::init() {
+    if (host_) return hipSuccess;
+    hipError_t e = hipHostMalloc((void**)&host_, kSlots * kSlot, hipHostMallocMapped);
     if (e != hipSuccess) host_ = nullptr;
     else e = hipHostGetDevicePointer((void**)&dev_, host_, 0);
     for (hipEvent_t& ev : ev_)
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     if (e != hipSuccess) release();
-    else bytes_ = bytes;
     return e;
 }
 
@@ -175,7 +173,6 @@ void ReadBack::release() {
     }
     if (host_) (void)hipHostFree(host_);
     host_ = dev_ = nullptr;
-    bytes_ = 0;
 }
 
 int ensure_paths(ct_ctx* c, uint32_t cap) {
