@@ -87,9 +87,10 @@ namespace ctr {
 // float image, or a 4K byte image) 1.85 ms, pinned 0.59 ms, the thread's
 // memcpy 0.8-0.9 ms.  Textured 1080p frame with its float image 5.83 to 5.15
 // ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time.
-// 2 MB in all, made at the first use: a slot of 2 MB each served no better, and
-// pinning the 8 MB took 3 ms of a context's first image.  Results of up to 1 MB,
-// where there is little to overlap, are left to the runtime.
+// 2 MB in all (0.5 MB for smaller results), made while the first frame is on the
+// device or at the first use: a slot of 2 MB each served no better, and pinning
+// the 8 MB took 3 ms of a context's first image.  Results of up to 1 MB in device
+// memory, where there is little to overlap, are left to the runtime.
 class ReadBack {
   public:
     // bytes of results to dst, in parts; put(dev, offset, n) enqueues on
@@ -98,7 +99,7 @@ class ReadBack {
     // returns.
     template <class Put>
     hipError_t run(void* dst, size_t bytes, hipStream_t s, Put put) {
-        hipError_t e = init();
+        hipError_t e = init(bytes);
         // what all slots hold in one part: a further part's launch and wait
         // cost what the overlap would give
         const size_t part = bytes <= kSlots * kSlot ? kSlots * kSlot : kSlot;
@@ -127,11 +128,17 @@ class ReadBack {
             return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
         });
     }
+    // Makes the slots for results of this size, while the device has something
+    // else to do; a failure is left to the next run().
+    void prepare(size_t bytes) {
+        if (bytes > kDirect) (void)init(bytes);
+    }
     void release();
 
   private:
     static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
-    hipError_t init();
+    hipError_t init(size_t bytes);
+    size_t bytes_ = 0;
     char *host_ = nullptr, *dev_ = nullptr;
     hipEvent_t ev_[kSlots] = {};
 };
@@ -242,8 +249,9 @@ struct Run {
 // tests, kRunGraph replays each lane's captured bounce loop, kRunSerial
 // runs one chunk at a time (nothing overlaps: per-kernel times are the
 // kernels' own, for measurement), kRunClock measures the chunks' device time
-// (ChunkStats::total_ms; kRunTimed does too).
-enum RunFlags { kRunTimed = 1, kRunCount = 2, kRunGraph = 4, kRunSerial = 8, kRunClock = 16 };
+// (ChunkStats::total_ms; kRunTimed does too), kRunRead prepares the context's
+// read-back while the chunks run.
+enum RunFlags { kRunTimed = 1, kRunCount = 2, kRunGraph = 4, kRunSerial = 8, kRunClock = 16, kRunRead = 32 };
 int run_paths(ct_ctx* c, const std::vector<ctd::ViewDesc>& views, const std::vector<Run>& runs, uint32_t cap,
               float4* accum, const ct_frame_opts& o, int flags, ChunkStats* st);
 
