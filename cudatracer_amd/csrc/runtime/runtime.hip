@@ -661,8 +661,13 @@ static void abort_lanes(ct_ctx* c) {
         if (L.h_read) L.h_read[kReadErr] = 0;
 }
 
-// Paths of a workload below which it is not split over the lanes.
-static constexpr uint64_t kSplitMin = 1u << 18;
+// Paths of a workload below which it is not split over the lanes: halves of it
+// have launches as long, which the other half's only fill from here on.  One
+// chunk / two, us: 132,000 paths of the box 824 / 844, the atrium 897 / 909, the
+// 7.24M triangles 1,522 / 1,509; 200,000 of the box 939 / 938, the textured
+// atrium 1,337 / 1,218; 232,683 of the box 1,018 / 992, the atrium 1,086 / 1,051,
+// the 7.24M triangles 1,698 / 1,661.
+static constexpr uint64_t kSplitMin = 3u << 16;
 
 int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<Run>& runs, uint32_t cap,
               float4* accum, const ct_frame_opts& o, int flags, ChunkStats* st) {
