@@ -680,7 +680,7 @@ int ct_trace_frame(ct_ctx* c, const ct_camera* cam, const ct_frame_opts* opts, c
     std::vector<Run> runs{{0u, 0u, (uint32_t)total}};
     const uint32_t cap = (uint32_t)std::min<uint64_t>(total, c->chunk_default);
     ChunkStats st;
-    r = run_paths(c, views, runs, cap, c->accum, o, kRunRead | (stats ? kRunTimed : 0), &st);
+    r = run_paths(c, views, runs, cap, c->accum, o, stats ? kRunTimed : 0, &st);
     if (r != CT_OK) return r;
     c->samples += o.spp;
     fill_stats(st, stats);

@@ -87,10 +87,9 @@ namespace ctr {
 // float image, or a 4K byte image) 1.85 ms, pinned 0.59 ms, the thread's
 // memcpy 0.8-0.9 ms.  Textured 1080p frame with its float image 5.83 to 5.15
 // ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time.
-// 2 MB in all (0.5 MB for smaller results), made while the first frame is on the
-// device or at the first use: a slot of 2 MB each served no better, and pinning
-// the 8 MB took 3 ms of a context's first image.  Results of up to 1 MB in device
-// memory, where there is little to overlap, are left to the runtime.
+// Pinning takes 0.4 ms a MB, so the slots are small (four of 2 MB served no better)
+// and made at the second result: a context's first goes by the runtime's copy,
+// as do results of up to 1 MB in device memory, where there is little to overlap.
 class ReadBack {
   public:
     // bytes of results to dst, in parts; put(dev, offset, n) enqueues on
@@ -99,7 +98,19 @@ class ReadBack {
     // returns.
     template <class Put>
     hipError_t run(void* dst, size_t bytes, hipStream_t s, Put put) {
-        hipError_t e = init(bytes);
+        if (!host_ && !used_) {
+            used_ = true;
+            void* d = nullptr;
+            if (hipMalloc(&d, std::max<size_t>(bytes, 16)) == hipSuccess) {
+                hipError_t e = put(static_cast<char*>(d), 0, bytes);
+                if (e == hipSuccess) e = direct(dst, d, bytes, s);
+                else (void)hipStreamSynchronize(s);
+                (void)hipFree(d);
+                return e;
+            }
+            (void)hipGetLastError();  // no room: through the slots
+        }
+        hipError_t e = init();
         // what all slots hold in one part: a further part's launch and wait
         // cost what the overlap would give
         const size_t part = bytes <= kSlots * kSlot ? kSlots * kSlot : kSlot;
@@ -119,26 +130,25 @@ class ReadBack {
     }
     // device memory
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        if (bytes <= kDirect) {
-            const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-            const hipError_t f = hipStreamSynchronize(s);
-            return e != hipSuccess ? e : f;
+        if (bytes <= kDirect || (!host_ && !used_)) {
+            used_ = used_ || bytes > kDirect;
+            return direct(dst, src, bytes, s);
         }
         return run(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
             return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
         });
     }
-    // Makes the slots for results of this size, while the device has something
-    // else to do; a failure is left to the next run().
-    void prepare(size_t bytes) {
-        if (bytes > kDirect) (void)init(bytes);
-    }
     void release();
 
   private:
     static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
-    hipError_t init(size_t bytes);
-    size_t bytes_ = 0;
+    hipError_t init();
+    static hipError_t direct(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        const hipError_t f = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : f;
+    }
+    bool used_ = false;
     char *host_ = nullptr, *dev_ = nullptr;
     hipEvent_t ev_[kSlots] = {};
 };
@@ -249,9 +259,8 @@ struct Run {
 // tests, kRunGraph replays each lane's captured bounce loop, kRunSerial
 // runs one chunk at a time (nothing overlaps: per-kernel times are the
 // kernels' own, for measurement), kRunClock measures the chunks' device time
-// (ChunkStats::total_ms; kRunTimed does too), kRunRead prepares the context's
-// read-back while the chunks run.
-enum RunFlags { kRunTimed = 1, kRunCount = 2, kRunGraph = 4, kRunSerial = 8, kRunClock = 16, kRunRead = 32 };
+// (ChunkStats::total_ms; kRunTimed does too).
+enum RunFlags { kRunTimed = 1, kRunCount = 2, kRunGraph = 4, kRunSerial = 8, kRunClock = 16 };
 int run_paths(ct_ctx* c, const std::vector<ctd::ViewDesc>& views, const std::vector<Run>& runs, uint32_t cap,
               float4* accum, const ct_frame_opts& o, int flags, ChunkStats* st);
 

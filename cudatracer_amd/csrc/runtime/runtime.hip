@@ -155,17 +155,14 @@ bool pinned_words(size_t words, uint32_t** host, uint32_t** dev) {
     return true;
 }
 
-hipError_t ReadBack::init(size_t bytes) {
-    if (bytes_ >= std::min(bytes, kSlots * kSlot)) return hipSuccess;
-    release();
-    bytes = bytes <= kSlot ? kSlot : kSlots * kSlot;
-    hipError_t e = hipHostMalloc((void**)&host_, bytes, hipHostMallocMapped);
+hipError_t ReadBack::init() {
+    if (host_) return hipSuccess;
+    hipError_t e = hipHostMalloc((void**)&host_, kSlots * kSlot, hipHostMallocMapped);
     if (e != hipSuccess) host_ = nullptr;
     else e = hipHostGetDevicePointer((void**)&dev_, host_, 0);
     for (hipEvent_t& ev : ev_)
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     if (e != hipSuccess) release();
-    else bytes_ = bytes;
     return e;
 }
 
@@ -176,7 +173,6 @@ void ReadBack::release() {
     }
     if (host_) (void)hipHostFree(host_);
     host_ = dev_ = nullptr;
-    bytes_ = 0;
 }
 
 int ensure_paths(ct_ctx* c, uint32_t cap) {
@@ -779,7 +775,6 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
         if (r != CT_OK) { abort_lanes(c); return r; }
     }
     if (!group.empty() && (r = launch_group()) != CT_OK) { abort_lanes(c); return r; }
-    if (flags & kRunRead) c->read.prepare((size_t)c->width * c->height * sizeof(float4));
     for (int k = 0; k < kLanes; ++k) {
         r = finish_chunk(c, c->ln[lane], st);
         lane = (lane + 1) % kLanes;
