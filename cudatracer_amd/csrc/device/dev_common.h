@@ -66,6 +66,7 @@ struct DevScene {
     int sky_enabled;
     int sky_tex;            // -1: the constant sky colour
     float sky_r, sky_g, sky_b;
+    float wide_extent;      // largest coordinate of the wide tree's boxes (ray_inv in device/traverse.h)
     uint32_t root2;         // the binary root's traversal item (item2 in device/traverse.h)
     uint32_t plane_flags;   // kPlaneNegZero | kPlaneNaN | kCompactBad over the quad tree, kPlaneInf2
 };

@@ -406,11 +406,14 @@ CT_DEV bool cnode4_step(const float4 (&n)[7], f3 o, f3 inv, float t, LaneStack& 
 // finite slab terms (then no slab value is NaN) the tests use the hardware
 // minimum and maximum, 8 instructions a child where compare-and-select takes
 // 20, with the same comparisons' results (they do not see a zero's sign).  The
-// general test, for the axis-parallel rays, is a loop, since a second unrolled
+// general test, for terms that are not finite, is a loop, since a second unrolled
 // copy would cost the registers again; the seven entries below the nearest are
 // stored in sequence, without 19 registers spilled for values and flags.
 // Atrium 1080p 6.57 to 4.82 ms, 7.24M triangles at 4K 13.1 to 9.0 ms, 1,048,576
 // rays 1.01 to 0.71 ms.
+//
+// A ray parallel to an axis has no 1 / d there (its terms would be infinity minus
+// infinity, and a NaN in x culls every child): ray_inv.
 CT_DEV bool fnode8_step(bool sort, const float4 (&n)[7], f3 o, f3 inv, float t, LaneStack& st, uint32_t& next) {
     const uint4 h = ubits4(n[0]), qx = ubits4(n[1]), qy = ubits4(n[2]), qz = ubits4(n[3]), ca = ubits4(n[4]),
                 cb = ubits4(n[5]);
@@ -788,6 +791,26 @@ CT_DEV bool ray_is_fast(const DevScene& sc, f3 o, f3 inv) {
     else return false;
 }
 
+// 1 / d as the tree's node test takes it.  The wide tree's gets a large finite K
+// for an infinite one: a plane is a grid step s or more outside the box it was
+// encoded from, so within the box t runs from below -s * K to above s * K, and
+// outside the grid's box the range is empty.  K is a power of two, 2^120 over the
+// largest coordinate in play (2^100 at most): every term stays finite, and s * K
+// is further than any hit (5e23 for boxes 1e-4 wide at coordinates of 1e6).
+// Decided per ray; per node it cost every launch ten spilled registers (1080p
+// atrium 4.72 to 5.56 ms).
+template <int ACCEL>
+CT_DEV f3 ray_inv(const DevScene& sc, f3 o, f3 d) {
+    f3 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    if constexpr (ACCEL == 8) {
+        const float m = fmaxf(fmaxf(sc.wide_extent, fabsf(o.x)), fmaxf(fabsf(o.y), fabsf(o.z)));
+        const float k = __uint_as_float(min(374u - (fbits(m) >> 23), 227u) << 23);
+        auto finite = [&](float v) { return fabsf(v) > 3.40282347e38f ? copysignf(k, v) : v; };
+        inv = mk3(finite(inv.x), finite(inv.y), finite(inv.z));
+    }
+    return inv;
+}
+
 // The item a ray starts at.
 template <int ACCEL>
 CT_DEV uint32_t root_item(const DevScene& sc) {
@@ -1038,7 +1061,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
                 if (MODE == kDual) any = v >= fe.nfirst;
                 ray = (MODE == kDual && any) ? fe.lo2 + (v - fe.nfirst) : fe.lo + v;
                 src(ray, any, o, d, t);
-                inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+                inv = ray_inv<ACCEL>(sc, o, d);
                 fast = ray_is_fast<ACCEL>(sc, o, inv);
                 st.top = 4u * (threadIdx.x & ~3u);
                 cur = root_item<ACCEL>(sc);
@@ -1073,7 +1096,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
         if (isnew) {
             // the ray loaded in the previous step
             prim = -1;
-            inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+            inv = ray_inv<ACCEL>(sc, o, d);
             fast = ray_is_fast<ACCEL>(sc, o, inv);
             st.reset();
             isnew = 0u;
@@ -1142,7 +1165,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
 template <int ACCEL>
 CT_DEV int trace_single(const DevScene& sc, float eps, f3 o, f3 d, float& t, bool any, LaneStack& st,
                         uint32_t* err) {
-    const f3 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    const f3 inv = ray_inv<ACCEL>(sc, o, d);
     const bool fast = ray_is_fast<ACCEL>(sc, o, inv);
     int prim = -1;
     uint32_t cur = root_item<ACCEL>(sc);

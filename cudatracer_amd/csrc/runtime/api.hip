@@ -338,6 +338,18 @@ int upload_shading(ct_ctx* c, const Shading& sh, ctd::DevScene& sc) {
     return r;
 }
 
+// The largest coordinate of the wide root's grid, which holds every box.
+float wide_extent(const std::vector<uint32_t>& fn) {
+    float m = 0.0f;
+    for (int a = 0; a < 3 && !fn.empty(); ++a) {
+        float p;
+        std::memcpy(&p, &fn[a], 4);
+        const float s = std::ldexp(1.0f, (int)((fn[3] >> (8 * a)) & 0xFFu) - 127);
+        m = std::max(m, std::max(std::fabs(p), std::fabs(std::fmaf(255.0f, s, p))));
+    }
+    return m;
+}
+
 // What the traversals need of the uploaded trees: the fast node test's copy
 // of the quad tree (sc.nodes4f), its compact layout (sc.cnodes, 64 bytes per
 // node), the trees' flags (sc.plane_flags: the fast tests need planes that
@@ -486,6 +498,7 @@ int ct_scene_upload(ct_ctx* c, const ct_scene_view* v) {
         const float4* fp = nullptr;
         r = upload_vec(c, fn, &fp, "wide nodes");
         sc.fnodes = reinterpret_cast<const uint4*>(fp);
+        sc.wide_extent = wide_extent(fn);
     }
     if (r == CT_OK && !n2.empty()) r = upload_vec(c, n2, &sc.nodes2, "binary nodes");
     if (r != CT_OK) { free_scene(c); return r; }
@@ -545,6 +558,7 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
         const float4* fp = nullptr;
         if (r == CT_OK) r = upload_vec(c, fn, &fp, "wide nodes");
         sc.fnodes = reinterpret_cast<const uint4*>(fp);
+        sc.wide_extent = wide_extent(fn);
         sc.n_fnodes = (uint32_t)(fn.size() / ct::kWideNodeWords);
     }
     if (r != CT_OK) { free_scene(c); return r; }
