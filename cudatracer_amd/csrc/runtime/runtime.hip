@@ -25,7 +25,11 @@ int fail(ct_ctx* c, int code, const std::string& msg) {
     return code;
 }
 
+// An error that has been reported is taken from the runtime, which would hand it
+// to the next launch's check as well: a refused allocation failed the next
+// call, or the host path taken in its place.
 int hip_fail(ct_ctx* c, hipError_t e, const char* what) {
+    (void)hipGetLastError();
     std::ostringstream os;
     os << what << ": " << hipGetErrorString(e);
     return fail(c, CT_ERR_DEVICE, os.str());
@@ -42,6 +46,7 @@ int dalloc(ct_ctx* c, void** p, size_t bytes, const char* what) {
     }
     const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         *p = nullptr;
         std::ostringstream os;
         os << "hipMalloc " << what << " (" << bytes << " bytes): " << hipGetErrorString(e);
@@ -143,11 +148,13 @@ static void free_paths(ct_ctx* c) {
 // it after the stream without a copy), and its device address.
 bool pinned_words(size_t words, uint32_t** host, uint32_t** dev) {
     if (hipHostMalloc((void**)host, words * 4, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) {
+        (void)hipGetLastError();
         *host = nullptr;
         return false;
     }
     std::memset(*host, 0, words * 4);
     if (hipHostGetDevicePointer((void**)dev, *host, 0) != hipSuccess) {
+        (void)hipGetLastError();
         (void)hipHostFree(*host);
         *host = nullptr;
         return false;

@@ -1,0 +1,98 @@
+"""What the library asks of the HIP runtime, counted on the CPU: the library runs
+in a process of its own over a stand-in for the runtime (hip_calls/standin.cpp:
+device memory is host memory, kernels do nothing)."""
+from __future__ import annotations
+
+import ctypes as C
+import subprocess
+import sys
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+HERE = Path(__file__).resolve().parent
+MB = 1 << 20
+CASES = {}
+
+
+def case(f):
+    CASES[f.__name__] = f
+    return f
+
+
+@pytest.fixture(scope="module")
+def standin(tmp_path_factory):
+    so = tmp_path_factory.mktemp("hip") / "standin.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-o", str(so), str(HERE / "hip_calls" / "standin.cpp")], check=True)
+    return so
+
+
+class Hip:
+    """The stand-in's records."""
+
+    def __init__(self, so):
+        self.lib = C.CDLL(so, mode=C.RTLD_GLOBAL)
+        for f in ("standin_used", "standin_peak", "standin_copied"):
+            getattr(self.lib, f).restype = C.c_size_t
+
+    def calls(self, name):
+        return self.lib.standin_calls(name.encode())
+
+    def fail(self, name, times):
+        self.lib.standin_fail(name.encode(), times)
+
+    def capacity(self, n):
+        self.lib.standin_capacity(C.c_size_t(n))
+
+    def used(self):
+        return self.lib.standin_used()
+
+    def peak(self):
+        """The largest use since the last call."""
+        p = self.lib.standin_peak(0)
+        self.lib.standin_peak(1)
+        return p
+
+    def copied(self, a):
+        """Bytes copied to the array by the runtime."""
+        return self.lib.standin_copied(C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes))
+
+    def pinned(self, shape, dtype=np.float32):
+        n = int(np.prod(shape)) * np.dtype(dtype).itemsize
+        p = C.c_void_p()
+        assert self.lib.hipHostMalloc(C.byref(p), C.c_size_t(n), 0) == 0
+        return np.frombuffer((C.c_char * n).from_address(p.value), dtype).reshape(shape)
+
+
+@case
+def refused_allocation(hip, ct):
+    """An allocation the runtime refuses is reported by the call that asked for
+    it, and not again by the next call's launch."""
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    ctx = ct.Context(0, mem_budget=1 << 40)
+    ctx.upload(scene)
+    hip.capacity(hip.used() + 512 * MB)
+    try:
+        ctx.resize(8192, 8192)
+        raise AssertionError("1 GiB fitted")
+    except ct.CTError as e:
+        assert e.code == ct.CT_ERR_OUT_OF_MEMORY
+    ctx.resize(64, 64)
+    ctx.trace_frame(scene.camera(64, 64), scene.frame_opts()[0], stats=False)
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_hip_calls(standin, name):
+    r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, str(HERE.parent))
+    hip_ = Hip(sys.argv[1])  # before the library
+    import cudatracer_amd
+
+    CASES[sys.argv[2]](hip_, cudatracer_amd)
+    assert hip_.calls("hipSetDevice") > 0, "the library did not reach the stand-in"
