@@ -540,6 +540,10 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     sc.n_nodes2 = t.n2;
     sc.n_nodes4 = t.n4;
     r = upload_prim_records(c, v, tmp, d_vert, d_idx, sc);
+    // the arrays make room before the textures and the wide nodes
+    if (r == CT_OK && hipStreamSynchronize(c->ln[0].stream) != hipSuccess)
+        r = fail(c, CT_ERR_DEVICE, "shading records");
+    tmp.release();
     if (r == CT_OK) r = upload_shading(c, sh, sc);
     uint32_t wide_bound = 0;
     if (r == CT_OK && (flags & CT_BUILD_WIDE)) {
@@ -563,7 +567,6 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
     }
     if (r != CT_OK) { free_scene(c); return r; }
     HIPCHK(hipStreamSynchronize(c->ln[0].stream), "scene upload");
-    tmp.release();
     if ((r = prepare_trees(c, sc)) != CT_OK) { free_scene(c); return r; }
     install_scene(c, v, sc, sh, wide_bound);
     bs.total_ms = (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

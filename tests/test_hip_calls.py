@@ -83,6 +83,35 @@ def refused_allocation(hip, ct):
     ctx.trace_frame(scene.camera(64, 64), scene.frame_opts()[0], stats=False)
 
 
+def _textured(ct, n, side):
+    """A view of n separate triangles with one float texture of side^2 texels."""
+    from conftest import ArrayView
+    rng = np.random.default_rng(5)
+    v = rng.uniform(-8, 8, (n, 1, 3)) + rng.uniform(-0.5, 0.5, (n, 3, 3))
+    cn = np.cross(v[:, 1] - v[:, 0], v[:, 2] - v[:, 0])
+    none = np.zeros(0, np.uint8)
+    arrays = dict(vertices=v.reshape(-1, 3), normals=np.repeat(cn, 3, axis=0), center_normals=cn,
+                  texcoords=rng.uniform(0, 1, (3 * n, 2)), indices=np.arange(3 * n).reshape(-1, 3),
+                  material_idx=np.zeros(n), light_indices=np.zeros(0), prim_indices=np.arange(n), bvh=none, mbvh=none,
+                  sky_enabled=0, sky=(0.0, 0.0, 0.0))
+    return ArrayView(ct, arrays, textures=[rng.uniform(0, 1, (side, side, 4))], mats=[ct.Material()])
+
+
+@case
+def build_beside_textures(hip, ct):
+    """upload_build needs the finished scene's memory for its textures, and not
+    that of the arrays its kernels read as well: 124 bytes a triangle here."""
+    n = 5_000
+    scene = _textured(ct, n, 1024)
+    budget = 1 << 40
+    for _ in range(2):
+        ctx = ct.Context(0, mem_budget=budget)
+        before = hip.used()
+        ctx.upload_build(scene.view)
+        budget = hip.used() - before + 16 * n
+        ctx.close()
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
