@@ -550,8 +550,16 @@ int ct_scene_upload_build(ct_ctx* c, const ct_scene_view* v, uint32_t flags, ct_
         // wide nodes are collapsed on the host from the device-built trees
         std::vector<ct_bvh_node> n2(t.n2);
         std::vector<ct_mbvh_node> n4(t.n4);
-        HIPCHK(hipMemcpy(n2.data(), t.nodes2, n2.size() * sizeof(ct_bvh_node), hipMemcpyDeviceToHost), "read trees");
-        HIPCHK(hipMemcpy(n4.data(), t.nodes4, n4.size() * sizeof(ct_mbvh_node), hipMemcpyDeviceToHost), "read trees");
+        // on the lane's stream, see prepare_trees
+        const hipStream_t s = c->ln[0].stream;
+        hipError_t e = hipMemcpyAsync(n2.data(), t.nodes2, n2.size() * sizeof(ct_bvh_node), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(n4.data(), t.nodes4, n4.size() * sizeof(ct_mbvh_node), hipMemcpyDeviceToHost, s);
+        const hipError_t w = hipStreamSynchronize(s);
+        if (e != hipSuccess || w != hipSuccess) {
+            free_scene(c);
+            return hip_fail(c, e != hipSuccess ? e : w, "read trees");
+        }
         ct_scene_view tv = *v;
         tv.n_bvh_nodes = t.n2;
         tv.bvh_nodes = n2.data();

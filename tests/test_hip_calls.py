@@ -112,6 +112,21 @@ def build_beside_textures(hip, ct):
         ctx.close()
 
 
+@case
+def no_copies_on_the_null_stream(hip, ct):
+    """The null stream takes a hardware queue for the rest of the process, and
+    a later context's two lanes then share one."""
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    ctx = ct.Context(0)
+    ctx.upload_build(scene, wide=True)
+    ctx.read_trees()
+    ctx.upload(scene)
+    ctx.resize(64, 64)
+    ctx.trace_frame(scene.camera(64, 64), scene.frame_opts()[0])
+    ctx.read_image()
+    assert hip.calls("hipMemcpyAsync") > 0 and hip.calls("hipMemcpy") == 0
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
