@@ -975,8 +975,10 @@ int ct_render_batch(ct_ctx* c, const ct_view* views, int32_t n_views, const ct_f
     r = run_paths(c, vd, runs, cap, arena, o, kRunGraph | (stats ? kRunClock : 0), &st);
     if (r == CT_OK) {
         for (int32_t i = 0; i < n_views && e == hipSuccess; ++i)
-            e = c->read.copy(views[i].accum_out, arena + vd[i].accum_offset,
-                             (size_t)views[i].width * views[i].height * sizeof(float4), c->ln[0].stream);
+            e = c->read.queue(views[i].accum_out, arena + vd[i].accum_offset,
+                              (size_t)views[i].width * views[i].height * sizeof(float4), c->ln[0].stream);
+        const hipError_t w = hipStreamSynchronize(c->ln[0].stream);
+        if (e == hipSuccess) e = w;
         if (e != hipSuccess) r = hip_fail(c, e, "read batch accumulators");
     }
     dfree(c, arena);

@@ -128,15 +128,22 @@ class ReadBack {
         const hipError_t f = hipStreamSynchronize(s);
         return e != hipSuccess ? e : f;
     }
-    // device memory
-    hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    // device memory; queue() leaves a result that needs no slots to be waited
+    // for with s, so that many small ones cost one wait (each on its own: 12 us
+    // against 3)
+    hipError_t queue(void* dst, const void* src, size_t bytes, hipStream_t s) {
         if (bytes <= kDirect || (!host_ && !used_)) {
             used_ = used_ || bytes > kDirect;
-            return direct(dst, src, bytes, s);
+            return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         }
         return run(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
             return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
         });
+    }
+    hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        const hipError_t e = queue(dst, src, bytes, s);
+        const hipError_t f = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : f;
     }
     void release();
 

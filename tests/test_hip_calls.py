@@ -127,6 +127,22 @@ def no_copies_on_the_null_stream(hip, ct):
     assert hip.calls("hipMemcpyAsync") > 0 and hip.calls("hipMemcpy") == 0
 
 
+@case
+def batch_waits_once(hip, ct):
+    """A batch's results are waited for together, not view by view."""
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    opts, _, _ = scene.frame_opts()
+    ctx = ct.Context(0)
+    ctx.upload(scene)
+    cam = scene.camera(8, 8)
+    waits = []
+    for n in (400, 4, 400):  # the first makes the path buffers
+        before = hip.calls("hipStreamSynchronize")
+        ctx.render_batch([(cam, 8, 8, 1, i) for i in range(n)], opts)
+        waits.append(hip.calls("hipStreamSynchronize") - before)
+    assert waits[1] == waits[2], waits
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
