@@ -80,7 +80,13 @@ constexpr int kReadErr = ctd::kReadCounters;
 constexpr int kReadWork = ctd::kReadCounters + 2;  // 4 x uint64, 8-byte aligned
 constexpr int kReadWords = kReadWork + 8;
 
+struct ct_ctx;
+
 namespace ctr {
+// Device memory, counted against the context's budget.
+int dalloc(ct_ctx* c, void** p, size_t bytes, const char* what);
+void dfree(ct_ctx* c, void* p);
+
 // Results to pageable host memory, through pinned slots: while the caller's
 // thread copies one slot to its place, the device fills the next ones.  The
 // runtime's own copy to pageable memory does the two in turn: 33 MB (a 1080p
@@ -97,19 +103,46 @@ class ReadBack {
     // device address).  Offsets are multiples of 512 KiB.  s is idle when it
     // returns.
     template <class Put>
-    hipError_t run(void* dst, size_t bytes, hipStream_t s, Put put) {
+    hipError_t run(ct_ctx* c, void* dst, size_t bytes, hipStream_t s, Put put) {
         if (!host_ && !used_) {
             used_ = true;
             void* d = nullptr;
-            if (hipMalloc(&d, std::max<size_t>(bytes, 16)) == hipSuccess) {
+            if (dalloc(c, &d, bytes, "image") == CT_OK) {
                 hipError_t e = put(static_cast<char*>(d), 0, bytes);
                 if (e == hipSuccess) e = direct(dst, d, bytes, s);
                 else (void)hipStreamSynchronize(s);
-                (void)hipFree(d);
+                dfree(c, d);
                 return e;
             }
-            (void)hipGetLastError();  // no room: through the slots
+            // no room: through the slots
         }
+        return parts(dst, bytes, s, put);
+    }
+    // device memory; queue() leaves a result that needs no slots to be waited
+    // for with s, so that many small ones cost one wait (each on its own: 12 us
+    // against 3)
+    hipError_t queue(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        if (bytes <= kDirect || (!host_ && !used_)) {
+            used_ = used_ || bytes > kDirect;
+            return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        }
+        return parts(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
+            return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
+        });
+    }
+    hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        const hipError_t e = queue(dst, src, bytes, s);
+        const hipError_t f = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : f;
+    }
+    void release();
+
+  private:
+    static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
+    hipError_t init();
+    // through the slots
+    template <class Put>
+    hipError_t parts(void* dst, size_t bytes, hipStream_t s, Put put) {
         hipError_t e = init();
         // what all slots hold in one part: a further part's launch and wait
         // cost what the overlap would give
@@ -128,28 +161,6 @@ class ReadBack {
         const hipError_t f = hipStreamSynchronize(s);
         return e != hipSuccess ? e : f;
     }
-    // device memory; queue() leaves a result that needs no slots to be waited
-    // for with s, so that many small ones cost one wait (each on its own: 12 us
-    // against 3)
-    hipError_t queue(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        if (bytes <= kDirect || (!host_ && !used_)) {
-            used_ = used_ || bytes > kDirect;
-            return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        }
-        return run(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
-            return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
-        });
-    }
-    hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        const hipError_t e = queue(dst, src, bytes, s);
-        const hipError_t f = hipStreamSynchronize(s);
-        return e != hipSuccess ? e : f;
-    }
-    void release();
-
-  private:
-    static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
-    hipError_t init();
     static hipError_t direct(void* dst, const void* src, size_t bytes, hipStream_t s) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         const hipError_t f = hipStreamSynchronize(s);
@@ -214,8 +225,6 @@ namespace ctr {
 
 int fail(ct_ctx* c, int code, const std::string& msg);
 int hip_fail(ct_ctx* c, hipError_t e, const char* what);
-int dalloc(ct_ctx* c, void** p, size_t bytes, const char* what);
-void dfree(ct_ctx* c, void* p);
 
 int validate_opts(ct_ctx* c, const ct_frame_opts& o);
 // Option checks of validate_opts without touching the context's error string

@@ -143,6 +143,17 @@ def batch_waits_once(hip, ct):
     assert waits[1] == waits[2], waits
 
 
+@case
+def image_within_the_budget(hip, ct):
+    """mem_budget holds for the buffer of a context's first image too: without
+    room for it the image comes through the pinned slots."""
+    ctx = ct.Context(0, mem_budget=20 * MB)
+    ctx.resize(1024, 1024)  # 16 MB
+    for read in (ctx.read_image, ctx.read_image, ctx.read_image_rgba8):
+        read()
+    assert hip.peak() <= 20 * MB
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
