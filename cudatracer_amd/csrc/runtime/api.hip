@@ -608,18 +608,27 @@ int ct_scene_read_trees(ct_ctx* c, ct_bvh_node* bvh, uint32_t cap_bvh, ct_mbvh_n
     HIPCHK(hipStreamSynchronize(s), "read trees");
     if (prim_indices) {
         // gathered on the device, a part of at most 4M ids at a time (a
-        // strided copy of the records' id words cost 7 us a row)
+        // strided copy of the records' id words costs 7 us a row), if the
+        // budget has room for them
         const uint32_t part = std::min<uint32_t>(N, 1u << 22);
-        uint32_t* ids = nullptr;
-        HIPCHK(hipMalloc(&ids, (size_t)part * 4), "read trees");
+        void* ids = nullptr;
         hipError_t e = hipSuccess;
-        for (uint32_t k = 0; k < N && e == hipSuccess; k += part) {
-            const uint32_t m = std::min(part, N - k);
-            e = ctk::launch_prim_ids(c->sc.tris, k, m, ids, s);
-            if (e == hipSuccess) e = hipMemcpyAsync(prim_indices + k, ids, (size_t)m * 4, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (dalloc(c, &ids, (size_t)part * 4, "primitive ids") == CT_OK) {
+            for (uint32_t k = 0; k < N && e == hipSuccess; k += part) {
+                const uint32_t m = std::min(part, N - k);
+                e = ctk::launch_prim_ids(c->sc.tris, k, m, static_cast<uint32_t*>(ids), s);
+                if (e == hipSuccess) e = hipMemcpyAsync(prim_indices + k, ids, (size_t)m * 4, hipMemcpyDeviceToHost, s);
+                if (e == hipSuccess) e = hipStreamSynchronize(s);
+            }
+            dfree(c, ids);
+        } else {
+            // the w word of each slot's first record, without the last-in-leaf bit
+            e = hipMemcpy2DAsync(prim_indices, 4, reinterpret_cast<const char*>(c->sc.tris) + 12, 3 * sizeof(float4), 4,
+                                 N, hipMemcpyDeviceToHost, s);
+            const hipError_t w = hipStreamSynchronize(s);
+            if (e == hipSuccess) e = w;
+            for (uint32_t k = 0; k < N && e == hipSuccess; ++k) prim_indices[k] &= 0x7FFFFFFFu;
         }
-        (void)hipFree(ids);
         if (e != hipSuccess) return hip_fail(c, e, "read trees");
     }
     return CT_OK;

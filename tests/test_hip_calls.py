@@ -154,6 +154,25 @@ def image_within_the_budget(hip, ct):
     assert hip.peak() <= 20 * MB
 
 
+@case
+def primitive_order_within_the_budget(hip, ct):
+    """So it does for read_trees; without room for the ids' buffer they come by
+    a strided copy."""
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    budget = 1 << 40
+    for _ in range(2):
+        ctx = ct.Context(0, mem_budget=budget)
+        before = hip.used()
+        ctx.upload(scene)
+        budget = hip.used() - before + 1024
+        hip.peak()
+        ids = ctx.read_trees()["prim_indices"]
+        peak = hip.peak() - before
+        ctx.close()
+    assert peak <= budget
+    assert np.array_equal(ids, scene.arrays()["prim_indices"])
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
