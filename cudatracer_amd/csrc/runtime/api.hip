@@ -807,13 +807,10 @@ int ct_read_image(ct_ctx* c, float* rgba, size_t n_floats) {
     sync_lanes(c);
     const hipStream_t s = c->ln[0].stream;
     // the kernel writes to the pinned slots itself
-    HIPCHK(c->read.run(c, rgba, npix * sizeof(float4), s,
-                       [&](char* dev, size_t offset, size_t n) {
-                           return ctk::launch_tonemap(c->accum + offset / sizeof(float4), (uint32_t)(n / sizeof(float4)),
-                                                      (float)std::max(c->samples, 1), reinterpret_cast<float4*>(dev), s);
-                       }),
-           "tonemap");
-    return CT_OK;
+    return c->read.run(c, rgba, npix * sizeof(float4), s, "image", [&](char* dev, size_t offset, size_t n) {
+        return ctk::launch_tonemap(c->accum + offset / sizeof(float4), (uint32_t)(n / sizeof(float4)),
+                                   (float)std::max(c->samples, 1), reinterpret_cast<float4*>(dev), s);
+    });
 }
 
 int ct_read_image_rgba8(ct_ctx* c, uint8_t* rgba, size_t n_bytes) {
@@ -824,13 +821,10 @@ int ct_read_image_rgba8(ct_ctx* c, uint8_t* rgba, size_t n_bytes) {
     (void)hipSetDevice(c->device);
     sync_lanes(c);
     const hipStream_t s = c->ln[0].stream;
-    HIPCHK(c->read.run(c, rgba, npix * 4, s,
-                       [&](char* dev, size_t offset, size_t n) {
-                           return ctk::launch_tonemap8(c->accum + offset / 4, (uint32_t)(n / 4),
-                                                       (float)std::max(c->samples, 1), reinterpret_cast<uint32_t*>(dev), s);
-                       }),
-           "tonemap");
-    return CT_OK;
+    return c->read.run(c, rgba, npix * 4, s, "image", [&](char* dev, size_t offset, size_t n) {
+        return ctk::launch_tonemap8(c->accum + offset / 4, (uint32_t)(n / 4), (float)std::max(c->samples, 1),
+                                    reinterpret_cast<uint32_t*>(dev), s);
+    });
 }
 
 // The error flag of lane 0's finished launch, cleared for the next call.

@@ -86,6 +86,7 @@ namespace ctr {
 // Device memory, counted against the context's budget.
 int dalloc(ct_ctx* c, void** p, size_t bytes, const char* what);
 void dfree(ct_ctx* c, void* p);
+int hip_fail(ct_ctx* c, hipError_t e, const char* what);
 
 // Results to pageable host memory, through pinned slots: while the caller's
 // thread copies one slot to its place, the device fills the next ones.  The
@@ -95,37 +96,44 @@ void dfree(ct_ctx* c, void* p);
 // ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time.
 // Pinning takes 0.4 ms a MB, so the slots are small (four of 2 MB served no better)
 // and made at the second result: a context's first goes by the runtime's copy,
-// as do results of up to 1 MB in device memory, where there is little to overlap.
+// as do results of up to 1 MB in device memory, where there is little to overlap,
+// and all of them where no slots can be had.
 class ReadBack {
   public:
     // bytes of results to dst, in parts; put(dev, offset, n) enqueues on
     // stream s a kernel that writes the n bytes from `offset` on to a slot (its
     // device address).  Offsets are multiples of 512 KiB.  s is idle when it
-    // returns.
+    // returns a CT_ code.
     template <class Put>
-    hipError_t run(ct_ctx* c, void* dst, size_t bytes, hipStream_t s, Put put) {
-        if (!host_ && !used_) {
-            used_ = true;
+    int run(ct_ctx* c, void* dst, size_t bytes, hipStream_t s, const char* what, Put put) {
+        const bool first = !host_ && !used_;
+        used_ = true;
+        hipError_t e;
+        if (first || init() != hipSuccess) {
+            // by the runtime's copy, from a buffer in device memory
             void* d = nullptr;
-            if (dalloc(c, &d, bytes, "image") == CT_OK) {
-                hipError_t e = put(static_cast<char*>(d), 0, bytes);
-                if (e == hipSuccess) e = direct(dst, d, bytes, s);
-                else (void)hipStreamSynchronize(s);
+            const int r = dalloc(c, &d, bytes, what);
+            if (r == CT_OK) {
+                e = put(static_cast<char*>(d), 0, bytes);
+                if (e == hipSuccess) e = hipMemcpyAsync(dst, d, bytes, hipMemcpyDeviceToHost, s);
+                const hipError_t f = hipStreamSynchronize(s);
                 dfree(c, d);
-                return e;
+                if (e == hipSuccess) e = f;
+                return e == hipSuccess ? CT_OK : hip_fail(c, e, what);
             }
-            // no room: through the slots
+            if (init() != hipSuccess) return r;
         }
-        return parts(dst, bytes, s, put);
+        e = parts(dst, bytes, s, put);
+        return e == hipSuccess ? CT_OK : hip_fail(c, e, what);
     }
     // device memory; queue() leaves a result that needs no slots to be waited
     // for with s, so that many small ones cost one wait (each on its own: 12 us
     // against 3)
     hipError_t queue(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        if (bytes <= kDirect || (!host_ && !used_)) {
-            used_ = used_ || bytes > kDirect;
+        const bool first = !host_ && !used_;
+        used_ = used_ || bytes > kDirect;
+        if (bytes <= kDirect || first || init() != hipSuccess)
             return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        }
         return parts(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
             return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
         });
@@ -140,10 +148,10 @@ class ReadBack {
   private:
     static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
     hipError_t init();
-    // through the slots
+    // through the slots, which are there
     template <class Put>
     hipError_t parts(void* dst, size_t bytes, hipStream_t s, Put put) {
-        hipError_t e = init();
+        hipError_t e = hipSuccess;
         // what all slots hold in one part: a further part's launch and wait
         // cost what the overlap would give
         const size_t part = bytes <= kSlots * kSlot ? kSlots * kSlot : kSlot;
@@ -158,11 +166,6 @@ class ReadBack {
             if (e == hipSuccess) e = hipEventSynchronize(ev_[k % kSlots]);
             if (e == hipSuccess) std::memcpy(static_cast<char*>(dst) + k * part, host_ + k % kSlots * kSlot, size(k));
         }
-        const hipError_t f = hipStreamSynchronize(s);
-        return e != hipSuccess ? e : f;
-    }
-    static hipError_t direct(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         const hipError_t f = hipStreamSynchronize(s);
         return e != hipSuccess ? e : f;
     }
@@ -224,7 +227,6 @@ struct ct_ctx {
 namespace ctr {
 
 int fail(ct_ctx* c, int code, const std::string& msg);
-int hip_fail(ct_ctx* c, hipError_t e, const char* what);
 
 int validate_opts(ct_ctx* c, const ct_frame_opts& o);
 // Option checks of validate_opts without touching the context's error string

@@ -169,7 +169,10 @@ hipError_t ReadBack::init() {
     else e = hipHostGetDevicePointer((void**)&dev_, host_, 0);
     for (hipEvent_t& ev : ev_)
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (e != hipSuccess) release();
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        release();
+    }
     return e;
 }
 

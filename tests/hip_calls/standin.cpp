@@ -71,11 +71,12 @@ size_t standin_peak(int reset) {
     if (reset) peak = used;
     return peak;
 }
-// Bytes that copies have written to [p, p + n).
+// Bytes that copies have written to [p, p + n) since the last call.
 size_t standin_copied(const char* p, size_t n) {
     size_t sum = 0;
     for (const auto& c : copies)
         if (c.first >= p && c.first < p + n) sum += c.second;
+    copies.clear();
     return sum;
 }
 

@@ -56,7 +56,7 @@ class Hip:
         return p
 
     def copied(self, a):
-        """Bytes copied to the array by the runtime."""
+        """Bytes the runtime has copied to the array since the last call."""
         return self.lib.standin_copied(C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes))
 
     def pinned(self, shape, dtype=np.float32):
@@ -171,6 +171,25 @@ def primitive_order_within_the_budget(hip, ct):
         ctx.close()
     assert peak <= budget
     assert np.array_equal(ids, scene.arrays()["prim_indices"])
+
+
+@case
+def results_without_pinned_memory(hip, ct):
+    """Results need no pinned memory: where the slots cannot be had they come
+    by the runtime's copy."""
+    ctx = ct.Context(0)
+    ctx.resize(512, 512)  # 4 MB
+    acc = np.random.default_rng(1).uniform(0, 4, (512, 512, 4)).astype(np.float32)
+    ctx.write_accum(acc, 1)
+    for failing in ("hipHostMalloc", "hipHostGetDevicePointer", "hipEventCreateWithFlags"):
+        hip.fail(failing, 1000)
+        for _ in range(3):
+            assert np.array_equal(ctx.read_accum()[0], acc)
+            for read in (ctx.read_image, ctx.read_image_rgba8):
+                hip.copied(acc)
+                image = read()
+                assert hip.copied(image) == image.nbytes
+        hip.fail(failing, 0)
 
 
 @pytest.mark.parametrize("name", list(CASES))
