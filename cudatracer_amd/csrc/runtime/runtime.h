@@ -88,11 +88,11 @@ int dalloc(ct_ctx* c, void** p, size_t bytes, const char* what);
 void dfree(ct_ctx* c, void* p);
 int hip_fail(ct_ctx* c, hipError_t e, const char* what);
 
-// Results to pageable host memory, through pinned slots: while the caller's
-// thread copies one slot to its place, the device fills the next ones.  The
-// runtime's own copy to pageable memory does the two in turn: 33 MB (a 1080p
-// float image, or a 4K byte image) 1.85 ms, pinned 0.59 ms, the thread's
-// memcpy 0.8-0.9 ms.  Textured 1080p frame with its float image 5.83 to 5.15
+// Results to the caller's memory.  To memory the runtime knows (pinned by the
+// caller) by its copy: 33 MB (a 1080p float image, or a 4K byte image) 0.59 ms.
+// To pageable memory through pinned slots: while the caller's thread copies one
+// slot to its place, the device fills the next ones.  The runtime's own copy
+// does the two in turn: 33 MB 1.85 ms, the thread's memcpy 0.8-0.9 ms of it.  Textured 1080p frame with its float image 5.83 to 5.15
 // ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time.
 // Pinning takes 0.4 ms a MB, so the slots are small (four of 2 MB served no better)
 // and made at the second result: a context's first goes by the runtime's copy,
@@ -106,22 +106,23 @@ class ReadBack {
     // returns a CT_ code.
     template <class Put>
     int run(ct_ctx* c, void* dst, size_t bytes, hipStream_t s, const char* what, Put put) {
-        const bool first = !host_ && !used_;
-        used_ = true;
+        const hipMemoryType type = type_of(dst);
+        const bool to_known = type != hipMemoryTypeUnregistered, first = !host_ && !used_;
+        used_ = used_ || !to_known;
         hipError_t e;
-        if (first || init() != hipSuccess) {
-            // by the runtime's copy, from a buffer in device memory
-            void* d = nullptr;
-            const int r = dalloc(c, &d, bytes, what);
+        if (to_known || first || init() != hipSuccess) {
+            // by the runtime's copy, from a buffer in device memory (kept for
+            // the next known destination)
+            const int r = buffer(c, bytes, what);
             if (r == CT_OK) {
-                e = put(static_cast<char*>(d), 0, bytes);
-                if (e == hipSuccess) e = hipMemcpyAsync(dst, d, bytes, hipMemcpyDeviceToHost, s);
+                e = put(buf_, 0, bytes);
+                if (e == hipSuccess) e = hipMemcpyAsync(dst, buf_, bytes, hipMemcpyDeviceToHost, s);
                 const hipError_t f = hipStreamSynchronize(s);
-                dfree(c, d);
+                if (!to_known) drop(c);
                 if (e == hipSuccess) e = f;
                 return e == hipSuccess ? CT_OK : hip_fail(c, e, what);
             }
-            if (init() != hipSuccess) return r;
+            if (type == hipMemoryTypeDevice || init() != hipSuccess) return r;
         }
         e = parts(dst, bytes, s, put);
         return e == hipSuccess ? CT_OK : hip_fail(c, e, what);
@@ -130,9 +131,9 @@ class ReadBack {
     // for with s, so that many small ones cost one wait (each on its own: 12 us
     // against 3)
     hipError_t queue(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        const bool first = !host_ && !used_;
-        used_ = used_ || bytes > kDirect;
-        if (bytes <= kDirect || first || init() != hipSuccess)
+        const bool direct = bytes <= kDirect || type_of(dst) != hipMemoryTypeUnregistered, first = !host_ && !used_;
+        used_ = used_ || !direct;
+        if (direct || first || init() != hipSuccess)
             return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         return parts(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
             return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
@@ -148,6 +149,24 @@ class ReadBack {
   private:
     static constexpr size_t kSlots = 4, kSlot = 512u << 10, kDirect = 1u << 20;
     hipError_t init();
+    static hipMemoryType type_of(const void* p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type;
+        (void)hipGetLastError();
+        return hipMemoryTypeUnregistered;
+    }
+    int buffer(ct_ctx* c, size_t bytes, const char* what) {
+        if (buf_bytes_ >= bytes) return CT_OK;
+        drop(c);
+        const int r = dalloc(c, reinterpret_cast<void**>(&buf_), bytes, what);
+        if (r == CT_OK) buf_bytes_ = bytes;
+        return r;
+    }
+    void drop(ct_ctx* c) {
+        dfree(c, buf_);
+        buf_ = nullptr;
+        buf_bytes_ = 0;
+    }
     // through the slots, which are there
     template <class Put>
     hipError_t parts(void* dst, size_t bytes, hipStream_t s, Put put) {
@@ -170,7 +189,8 @@ class ReadBack {
         return e != hipSuccess ? e : f;
     }
     bool used_ = false;
-    char *host_ = nullptr, *dev_ = nullptr;
+    char *host_ = nullptr, *dev_ = nullptr, *buf_ = nullptr;
+    size_t buf_bytes_ = 0;
     hipEvent_t ev_[kSlots] = {};
 };
 }  // namespace ctr

@@ -192,6 +192,32 @@ def results_without_pinned_memory(hip, ct):
         hip.fail(failing, 0)
 
 
+@case
+def pinned_destinations(hip, ct):
+    """Results go straight to an array the caller has pinned."""
+    ctx = ct.Context(0)
+    ctx.resize(512, 512)  # 4 MB
+    acc = np.random.default_rng(1).uniform(0, 4, (512, 512, 4)).astype(np.float32)
+    ctx.write_accum(acc, 1)
+    f, b = hip.pinned((512, 512, 4)), hip.pinned((512, 512, 4), np.uint8)
+    fp = f.ctypes.data_as(C.POINTER(C.c_float))
+    bp = b.ctypes.data_as(C.POINTER(C.c_uint8))
+    n = C.c_int32()
+    for read, out in ((lambda: ct.lib.ct_read_accum(ctx.handle, fp, f.size, C.byref(n)), f),
+                      (lambda: ct.lib.ct_read_image(ctx.handle, fp, f.size), f),
+                      (lambda: ct.lib.ct_read_image_rgba8(ctx.handle, bp, b.size), b)):
+        for k in range(3):
+            hip.copied(acc)
+            allocated = hip.calls("hipMalloc")
+            assert read() == 0
+            assert hip.copied(out) == out.nbytes
+            assert k == 0 or hip.calls("hipMalloc") == allocated  # the image's buffer is kept
+    ctx.read_accum(), ctx.read_image()  # pageable ones in between
+    hip.copied(acc)
+    assert ct.lib.ct_read_accum(ctx.handle, fp, f.size, C.byref(n)) == 0
+    assert hip.copied(f) == f.nbytes and np.array_equal(f, acc)
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
