@@ -171,9 +171,10 @@ class ReadBack {
     template <class Put>
     hipError_t parts(void* dst, size_t bytes, hipStream_t s, Put put) {
         hipError_t e = hipSuccess;
-        // what all slots hold in one part: a further part's launch and wait
-        // cost what the overlap would give
-        const size_t part = bytes <= kSlots * kSlot ? kSlots * kSlot : kSlot;
+        // up to 1.5 MB in one part: a further part's launch and wait cost what
+        // the overlap would give (at 2 MB one part took 118 us, four 106, and
+        // the runtime's copy 113)
+        const size_t part = bytes <= 3 * kSlot ? 3 * kSlot : kSlot;
         const size_t n = (bytes + part - 1) / part;
         auto size = [&](size_t k) { return std::min(part, bytes - k * part); };
         for (size_t put_n = 0, k = 0; k < n && e == hipSuccess; ++k) {

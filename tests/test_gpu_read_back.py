@@ -1,5 +1,5 @@
 """Results on their way to the caller's arrays: by the runtime's copy up to 1
-MB, through one pinned slot up to 2 MB, in parts through four above.  The sizes
+MB, through the pinned slots in one part up to 1.5 MB, in parts above.  The sizes
 are the edges of those, part sizes that do not divide the result, and enough
 parts to reuse every slot; each must bring every byte to its place."""
 from __future__ import annotations
@@ -70,3 +70,9 @@ def test_first_image_of_a_context(ct, gpu_ctx, w, h):
     assert np.array_equal(second.view(np.uint32), ref.view(np.uint32))
     assert np.array_equal(bytes8, gpu_ctx.read_image_rgba8())
     gpu_ctx.reset()
+
+
+@pytest.mark.parametrize("w,h", [(384, 256), (385, 256), (448, 256), (449, 256)])
+def test_read_back_up_to_four_parts(ct, gpu_ctx, w, h):
+    """One part up to 1.5 MB, then three and a bit, and four."""
+    test_read_back(ct, gpu_ctx, w, h)

@@ -218,6 +218,18 @@ def pinned_destinations(hip, ct):
     assert hip.copied(f) == f.nbytes and np.array_equal(f, acc)
 
 
+@case
+def parts_of_a_result(hip, ct):
+    """One part up to 1.5 MB, parts of 512 KB above: at 2 MB one part took longer
+    than the runtime's copy."""
+    ctx = ct.Context(0)
+    for rows, parts in ((1024, 0), (257, 1), (384, 1), (385, 4), (512, 4), (513, 5)):
+        ctx.resize(256, rows)  # 4 KB a row; the first makes the slots due
+        before = hip.calls("hipLaunchKernel")
+        ctx.read_accum()
+        assert hip.calls("hipLaunchKernel") - before == parts, rows
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
