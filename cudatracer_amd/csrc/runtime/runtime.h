@@ -72,7 +72,6 @@ struct Lane {
     bool timed = false, count = false, clock = false;
     bool nee = false;  // the chunk ends with a launch for the last bounce's shadow rays
     int tail = -1;     // the chunk's k_paths bounce, or -1
-    bool paths = false;  // the chunk runs as whole paths (k_paths)
 };
 constexpr int kHostWords = 16;  // in ct_ctx::h_flag: the words of a tree build
 // h_read layout (uint32 words)

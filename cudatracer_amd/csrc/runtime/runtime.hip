@@ -398,9 +398,10 @@ int tail_bounce(const ct_frame_opts& o, bool count) {
 // (k_paths) instead of the queue pipeline: while the GPU holds all of them at
 // once, two lanes each (131,072 paths on 256 CUs; above, the pipeline is
 // faster: 262,144 paths in two chunks 0.90 against 1.04 ms).  Not for a
-// counting frame: k_paths does not count node and triangle tests.
-static bool whole_paths(const ct_ctx* c, uint64_t total, bool count) {
-    return !count && total <= (uint64_t)c->shape.tail_blocks * (uint64_t)c->shape.block / 2u;
+// counting frame: k_paths does not count node and triangle tests; nor for a
+// timed one, whose stages k_paths does not tell apart.
+static bool whole_paths(const ct_ctx* c, uint64_t total, bool count, bool timed) {
+    return !count && !timed && total <= (uint64_t)c->shape.tail_blocks * (uint64_t)c->shape.block / 2u;
 }
 
 struct BounceSeq {
@@ -426,12 +427,11 @@ struct BounceSeq {
     hipError_t step(int k) {
         hipStream_t s = L->stream;
         hipError_t r;
+        if (paths)
+            return k == 0 ? hipSuccess
+                          : ctk::launch_paths(c->shape, c->sc, to, so, L->d_views, L->d_segs, L->d_hdr, L->q, paths, s);
         if (k == 0) {
             rec();
-            if (paths) {
-                rec();
-                return hipSuccess;
-            }
             if ((r = ctk::launch_generate(c->shape, L->d_views, L->d_segs, L->d_hdr, c->lane_cap, L->q, s)) !=
                 hipSuccess)
                 return r;
@@ -444,14 +444,6 @@ struct BounceSeq {
         // rays and bounce b's shadow rays, or, at the tail bounce, k_paths
         // runs every remaining bounce
         const int b = k - 1;
-        if (paths) {
-            rec();
-            if ((r = ctk::launch_paths(c->shape, c->sc, to, so, L->d_views, L->d_segs, L->d_hdr, L->q, paths, s)) !=
-                hipSuccess)
-                return r;
-            rec();
-            return hipSuccess;
-        }
         rec();
         if ((r = ctk::launch_trace(c->shape, c->sc, to, L->q, L->d_hdr, sel, b, ws, s)) != hipSuccess) return r;
         rec();
@@ -470,10 +462,7 @@ struct BounceSeq {
     // traces its own)
     hipError_t finish() {
         hipError_t r;
-        if (paths) {
-            L->n_events = e;
-            return hipSuccess;
-        }
+        if (paths) return hipSuccess;
         rec();
         if (nee && tail < 0 &&
             (r = ctk::launch_trace(c->shape, c->sc, to, L->q, L->d_hdr, sel, o.max_depth, ws, L->stream)) !=
@@ -579,7 +568,7 @@ static int graph_chunk(ct_ctx* c, Lane& L, const ct_frame_opts& o) {
 }
 
 static int close_chunk(ct_ctx* c, Lane& L, uint32_t n, float4* accum, const ct_frame_opts& o, bool timed,
-                       bool count, bool clock, bool whole, bool alone, hipEvent_t prev_resolved) {
+                       bool count, bool clock, bool alone, hipEvent_t prev_resolved) {
     hipStream_t s = L.stream;
     // accumulator updates in chunk order
     if (prev_resolved) HIPCHK(hipStreamWaitEvent(s, prev_resolved, 0), "order resolves");
@@ -596,7 +585,6 @@ static int close_chunk(ct_ctx* c, Lane& L, uint32_t n, float4* accum, const ct_f
     L.max_depth = o.max_depth;
     L.nee = o.shadow && c->sc.n_lights > 0;
     L.tail = tail_bounce(o, count);
-    L.paths = whole;
     L.timed = timed;
     L.count = count;
     L.clock = clock;
@@ -635,8 +623,7 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
         };
         st->other_ms += pair(e);
         e += 2;
-        if (L.paths) st->tail_ms += pair(e);
-        const int nb = L.paths ? 0 : (L.tail >= 0 ? L.tail + 1 : L.max_depth);
+        const int nb = L.tail >= 0 ? L.tail + 1 : L.max_depth;
         for (int b = 0; b < nb; ++b) {
             st->extend_ms += pair(e);
             st->extend_launches += 1;
@@ -644,7 +631,7 @@ static int finish_chunk(ct_ctx* c, Lane& L, ChunkStats* st) {
             else st->shade_ms += pair(e + 2);
             e += 4;
         }
-        if (L.nee && L.tail < 0 && !L.paths) {
+        if (L.nee && L.tail < 0) {
             st->connect_ms += pair(e);
             st->extend_launches += 1;
         }
@@ -690,7 +677,7 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
     int r = ensure_paths(c, cap);
     if (r != CT_OK) return r;
     cap = std::min(cap, c->lane_cap);
-    const bool whole = whole_paths(c, total, count);
+    const bool whole = whole_paths(c, total, count, timed);
     // work queued on lane 0 by the caller (accumulator clears) comes first
     const bool alone = total <= cap;  // one chunk, on lane 0
     if (!alone) HIPCHK(hipEventRecord(c->ln[0].resolved, c->ln[0].stream), "event");
@@ -738,7 +725,7 @@ int run_paths(ct_ctx* c, const std::vector<ViewDesc>& views, const std::vector<R
             if (here[i]) HIPCHK(seq[i].finish(), "launch chunk");
         for (int i = 0; i < g; ++i) {
             Lane& L = c->ln[(lane + i) % kLanes];
-            if ((rr = close_chunk(c, L, group[i].fill, accum, o, timed, count, clock, whole, alone, prev)) !=
+            if ((rr = close_chunk(c, L, group[i].fill, accum, o, timed, count, clock, alone, prev)) !=
                 CT_OK)
                 return rr;
             prev = L.resolved;

@@ -203,13 +203,10 @@ typedef struct ct_frame_stats {
                                  plus one per chunk for the last shadow rays
                                  when NEE is on; with roulette, the bounces
                                  up to the tail's first)                      */
-    double tail_ms;           /* the device time of the launches that run whole paths:
-                                 with roulette (rr_start >= 0) each chunk's
-                                 remaining bounces once roulette has thinned its
-                                 paths; for a small frame (while the GPU holds all
-                                 its paths at once: 131,072 on 256 CUs) all of it,
-                                 extend_ms, shade_ms, connect_ms and
-                                 extend_launches then being 0                   */
+    double tail_ms;           /* with roulette (rr_start >= 0): the device time of
+                                 the launches that run each chunk's remaining
+                                 bounces once roulette has thinned its paths
+                                 (whole paths, two lanes each)                 */
 } ct_frame_stats;
 
 /* Fill with the reference defaults (depth 5, 1 spp, no RR, BVH4, reference BSDF,
@@ -271,7 +268,9 @@ int ct_reset(ct_ctx* ctx);
 
 /* launchKernels (Kernel.cu:355-372): trace opts->spp samples per pixel from
  * the camera, add them to the persistent accumulator and advance the sample
- * counter.  opts may be NULL (reference defaults).  stats may be NULL. */
+ * counter.  opts may be NULL (reference defaults).  stats may be NULL: a small
+ * frame (131,072 paths on 256 CUs) then runs as whole paths in one launch,
+ * which has no stages to time. */
 int ct_trace_frame(ct_ctx* ctx, const ct_camera* cam, const ct_frame_opts* opts,
                    ct_frame_stats* stats);
 

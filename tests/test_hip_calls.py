@@ -230,6 +230,22 @@ def parts_of_a_result(hip, ct):
         assert hip.calls("hipLaunchKernel") - before == parts, rows
 
 
+@case
+def stages_of_a_small_frame(hip, ct):
+    """A frame with statistics has its stages' device times, however small."""
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    opts, _, _ = scene.frame_opts()
+    opts.rr_start, opts.max_depth = -1, 4
+    ctx = ct.Context(0)
+    ctx.upload(scene)
+    ctx.resize(64, 64)
+    for trace in (ctx.trace_frame, ctx.trace_frame_serial):
+        st = trace(scene.camera(64, 64), opts)
+        # one launch a bounce and one for the last shadow rays
+        assert st.chunks == 1 and st.extend_launches == 5
+        assert min(st.extend_ms, st.shade_ms, st.connect_ms, st.other_ms) > 0.0 and st.tail_ms == 0.0
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
