@@ -991,52 +991,7 @@ __global__ void k_root_leaf(Geo g, uint32_t n) {
 }
 
 // ------------------------------------------------------------- device scan
-constexpr uint32_t kScanTile = 1024;  // 256 threads x 4
-
-__global__ __launch_bounds__(kBlock) void k_scan_sums(const uint32_t* in, uint32_t n, uint32_t* sums) {
-    __shared__ uint32_t s_w[kBlock / 64];
-    const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * 4;
-    uint32_t v = 0;
-    for (int k = 0; k < 4; ++k)
-        if (base + k < n) v += in[base + k];
-    uint32_t tot;
-    (void)block_scan(v, s_w, tot);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-
-// In-place exclusive scan of the tile sums (one block).
-__global__ __launch_bounds__(kBlock) void k_scan_top(uint32_t* sums, uint32_t nt) {
-    __shared__ uint32_t s_w[kBlock / 64];
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < nt; base += kBlock) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < nt ? sums[i] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_scan(v, s_w, tot);
-        if (i < nt) sums[i] = carry + ex;
-        carry += tot;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_scan_out(const uint32_t* in, uint32_t n, const uint32_t* sums,
-                                                     uint32_t* out) {
-    __shared__ uint32_t s_w[kBlock / 64];
-    const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * 4;
-    uint32_t v[4], t = 0;
-    for (int k = 0; k < 4; ++k) {
-        v[k] = base + k < n ? in[base + k] : 0u;
-        t += v[k];
-    }
-    uint32_t tot;
-    uint32_t run = sums[blockIdx.x] + block_scan(t, s_w, tot);
-    for (int k = 0; k < 4; ++k)
-        if (base + k < n) {
-            out[base + k] = run;
-            run += v[k];
-        }
-}
-
-// Exclusive scan by one block.
+// Exclusive scan by one block: of a level's chunks, one word for 2,048 slots.
 __global__ __launch_bounds__(kTile) void k_scan_one(const uint32_t* in, uint32_t n, uint32_t* out) {
     __shared__ uint32_t s_w[kTile / 64];
     uint32_t carry = 0;
@@ -1141,7 +1096,7 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
     GET(chunk_left, Mc);
     GET(chunk_pre, Mc);
     GET(part, Mc * kBinWords);
-    GET(sums, 4 * (uint64_t)blocks_for(std::max(W, Mc), kScanTile));
+    GET(sums, 4 * (uint64_t)blocks_for(W, kTile));
     GET(cnt, kCounts);
     GET(rpart, (uint64_t)nblk_init * 6);
 #undef GET
@@ -1170,20 +1125,6 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
     k_root<<<1, kBlock, 0, s>>>(rpart, nblk_init, N, nodes, plans[0], cnt);
     BLAUNCH("build: root");
 
-    // exclusive scan of n words
-    auto scan = [&](const uint32_t* in, uint32_t* outp, uint32_t n) -> int {
-        if (n <= kOneBlock) {
-            k_scan_one<<<1, kTile, 0, s>>>(in, n, outp);
-        } else {
-            const uint32_t nt = blocks_for(n, kScanTile);
-            k_scan_sums<<<nt, kBlock, 0, s>>>(in, n, sums);
-            k_scan_top<<<1, kBlock, 0, s>>>(sums, nt);
-            k_scan_out<<<nt, kBlock, 0, s>>>(in, n, sums, outp);
-        }
-        BLAUNCH("build: scan");
-        return CT_OK;
-    };
-
     Levels levels{};
     uint32_t long_chains = 0, jump_rounds = 0;
     uint32_t g0 = 0, n = 1;
@@ -1210,7 +1151,8 @@ int device_build(ct_ctx* c, const ct_scene_view* v, const float* d_vert, const u
             k_mdecide<<<Tm, kBlock, 0, s>>>(lv, mch_node, mch_k, part, kid, plan.split, dec, cnt + kCntErr);
             k_mrank<<<Tm, kBlock, 0, s>>>(lv, level, mch_node, mch_k, slots, dec, rf, chunk_left);
             BLAUNCH("build: large nodes");
-            if ((r = scan(chunk_left, chunk_pre, Tm))) return r;
+            k_scan_one<<<1, kTile, 0, s>>>(chunk_left, Tm, chunk_pre);
+            BLAUNCH("build: scan");
             k_mmove<<<Tm, kBlock, 0, s>>>(lv, level, mch_node, mch_k, slots, geo, dec, rf, chunk_pre, chunk_left,
                                           cnt + kCntErr, cnt + kCntPending, pend_dst, pend_q, plan.jflag,
                                           cnt + kCntLongest);
