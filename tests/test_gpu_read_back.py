@@ -76,3 +76,8 @@ def test_first_image_of_a_context(ct, gpu_ctx, w, h):
 def test_read_back_up_to_four_parts(ct, gpu_ctx, w, h):
     """One part up to 1.5 MB, then three and a bit, and four."""
     test_read_back(ct, gpu_ctx, w, h)
+
+
+def test_host_hits_in_two_parts(ct, gpu_ctx, c1):
+    """Host rays go to the device 4,194,304 at a time: a second part of one ray."""
+    test_host_hits(ct, gpu_ctx, c1, (1 << 22) + 1)
