@@ -214,8 +214,8 @@ CT_DEV void add_term(float4& L, float4 t) {
 }
 CT_DEV uint32_t* cnt_active(uint32_t* c, int b) { return c + b; }
 CT_DEV uint32_t* cnt_shadow(uint32_t* c, int b) { return c + (kMaxBounce + 1) + b; }
-// Extension and shadow rays traced by k_paths (a chunk's roulette tail), over
-// all the bounces it runs.
+// Extension and shadow rays traced by k_paths (whole paths, or a chunk's
+// roulette tail), over all the bounces it runs.
 CT_DEV uint32_t* cnt_tail_ext(uint32_t* c) { return c + 2 * (kMaxBounce + 1); }
 CT_DEV uint32_t* cnt_tail_shadow(uint32_t* c) { return c + 2 * (kMaxBounce + 1) + 1; }
 // Work-fetch counters, [queue][range][bounce]: each queue range owns a

@@ -625,14 +625,16 @@ k_shade(DevScene sc, ShadeOpts so, const ViewDesc* __restrict__ views, const Seg
 // its own needs the sum of its own rays.  Used for
 //  - small workloads, with eight lanes while each path can have them at once,
 //    and with two while each path can (launch_paths); five waves per SIMD for
-//    eight lanes (four and six were up to 8% slower at 49,284 paths);
+//    eight lanes (atrium: at 32,761 paths four, five and six waves 354, 355 and
+//    381 us; at 40,960, which four do not hold at once, 475, 396 and 417);
 //  - a chunk's bounces from rr_start on, once roulette has thinned its paths,
 //    with two (the 4K displaced frame is 0.5% slower with eight).
 // Frame times in us of the pipeline / two / eight lanes:
-//   paths                    3,072          32,761         65,536          131,044
-//   box, binary tree, 4   442 565 342    585 498 410    664 515 670     781 607 1093
-//   box, quad tree, 8     489 584 328    694 561 417    802 564 624     953 706 1172
-//   atrium, quad tree, 8  488 540 333    658 551 407    692 536 687     810 678 1095
+//   paths                             3,072         32,761        40,960        65,536        131,044
+//   box, binary tree, depth 4      365 470 287   506 421 362   546 427 389   582 432 576   678 509 1064
+//   atrium, quad tree, 8           426 502 287   548 462 357   570 476 396   618 462 604   742 578 1042
+//   textured atrium, quad tree, 8  452 539 308   643 503 385   674 518 427   792 534 680  1036 647 1138
+//   7.24M triangles, 16, roulette  665 546 362  1070 704 466  1040 722 478  1207 753 658  1367 819 1010
 template <int ACCEL, int G, bool FIRST>
 __global__ void __attribute__((amdgpu_waves_per_eu(G == 8 ? 5 : 4)))
 k_paths(DevScene sc, TraceOpts to, ShadeOpts so, const ViewDesc* __restrict__ views, const Segment* __restrict__ segs,

@@ -1135,7 +1135,7 @@ CT_DEV void trace_persistent(const DevScene& sc, float eps, uint32_t n, uint32_t
         const uint64_t alive = __ballot(cur != kDead);
         if (alive == 0) return;
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(alive >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)alive, 0u));
-        // idle lanes send to the quads past the last ray, where nothing reads
+        // idle lanes send to lane 1, which no quad reads
         const uint32_t n_alive = (uint32_t)__popcll(alive);
         const uint32_t dst = 4u * (cur != kDead ? rank : 0u);
         const uint32_t from = quad_dpp<0x00>((uint32_t)__builtin_amdgcn_ds_permute((int)(4u * (cur != kDead ? dst : dst + 1u)), (int)lane_id()));
