@@ -130,16 +130,12 @@ class ReadBack {
     // for with s, so that many small ones cost one wait (each on its own: 12 us
     // against 3)
     hipError_t queue(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        const bool direct = bytes <= kDirect || type_of(dst) != hipMemoryTypeUnregistered, first = !host_ && !used_;
-        used_ = used_ || !direct;
-        if (direct || first || init() != hipSuccess)
-            return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        return parts(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
-            return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
-        });
+        return through_slots(dst, bytes) ? copy_parts(dst, src, bytes, s)
+                                         : hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
     }
     hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
-        const hipError_t e = queue(dst, src, bytes, s);
+        if (through_slots(dst, bytes)) return copy_parts(dst, src, bytes, s);
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         const hipError_t f = hipStreamSynchronize(s);
         return e != hipSuccess ? e : f;
     }
@@ -153,6 +149,12 @@ class ReadBack {
         if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type;
         (void)hipGetLastError();
         return hipMemoryTypeUnregistered;
+    }
+    bool through_slots(const void* dst, size_t bytes) {
+        if (bytes <= kDirect || type_of(dst) != hipMemoryTypeUnregistered) return false;
+        const bool first = !host_ && !used_;
+        used_ = true;
+        return !first && init() == hipSuccess;
     }
     int buffer(ct_ctx* c, size_t bytes, const char* what) {
         if (buf_bytes_ >= bytes) return CT_OK;
@@ -187,6 +189,11 @@ class ReadBack {
         }
         const hipError_t f = hipStreamSynchronize(s);
         return e != hipSuccess ? e : f;
+    }
+    hipError_t copy_parts(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        return parts(dst, bytes, s, [&](char* dev, size_t offset, size_t n) {
+            return ctk::launch_copy_out(static_cast<const char*>(src) + offset, n, dev, s);
+        });
     }
     bool used_ = false;
     char *host_ = nullptr, *dev_ = nullptr, *buf_ = nullptr;

@@ -246,6 +246,18 @@ def stages_of_a_small_frame(hip, ct):
         assert min(st.extend_ms, st.shade_ms, st.connect_ms, st.other_ms) > 0.0 and st.tail_ms == 0.0
 
 
+@case
+def one_wait_a_result(hip, ct):
+    """A result is waited for once, by the runtime's copy (the first) or through
+    the slots."""
+    ctx = ct.Context(0)
+    ctx.resize(512, 512)  # 4 MB
+    for _ in range(3):
+        before = hip.calls("hipStreamSynchronize")
+        ctx.read_accum()
+        assert hip.calls("hipStreamSynchronize") - before == 1
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
