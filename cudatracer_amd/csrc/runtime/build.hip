@@ -775,7 +775,7 @@ __device__ void finish_totals(const Finish& f, const uint32_t (&total)[4]) {
 // three kernels, lists; then a scan of the splits and the children).  With the
 // next level's plan made along with its nodes, one wait a level and the ranks
 // of small levels in one launch, the upload of a changed scene of that size went from
-// 11.9 to 10.1 ms, and a new context's of 100,003 with its export from 4.84 to 3.45.
+// 11.9 to 10.1 ms, and one of 100,003 with its export from 4.84 to 3.45.
 __global__ __launch_bounds__(kTile) void k_finish(Finish f) {
     __shared__ uint32_t s_w[kTile / 64];
     uint32_t carry[4] = {0, 0, 0, 0};
