@@ -1238,18 +1238,20 @@ hipError_t launch_shadow_flags(const LaunchShape& ls, const DevScene& sc, const 
 }  // namespace ctk
 
 namespace ctk {
-// Resident blocks per CU of the persistent traversal kernels of one tree
-// (extend and trace, the smaller of the two) for a block size and LDS depth.
+// Resident blocks of a kernel per CU; 0, and no error kept for the next launch,
+// if there is no telling.
+static int resident_blocks(const void* kernel, int block, size_t lds) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, block, lds) == hipSuccess) return n;
+    (void)hipGetLastError();
+    return 0;
+}
+// Of the persistent traversal kernels of one tree (extend and trace, the
+// smaller of the two) for a block size and LDS depth.
 template <int TREE>
 static int per_cu(int block, size_t lds) {
-    int nb = 0, nc = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(&ctd::k_extend<TREE>),
-                                                     block, lds) != hipSuccess)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nc, reinterpret_cast<const void*>(&ctd::k_trace<TREE, false>),
-                                                     block, lds) != hipSuccess)
-        return 0;
-    return nb < nc ? nb : nc;
+    return std::min(resident_blocks(reinterpret_cast<const void*>(&ctd::k_extend<TREE>), block, lds),
+                    resident_blocks(reinterpret_cast<const void*>(&ctd::k_trace<TREE, false>), block, lds));
 }
 
 bool set_trace_grids(LaunchShape& ls, int num_cus) {
@@ -1273,11 +1275,8 @@ bool set_trace_grids(LaunchShape& ls, int num_cus) {
     // k_paths: the blocks of its most register-hungry tree that fit at once
     auto resident = [&](std::initializer_list<const void*> kernels, int& blocks) {
         int least = 1 << 30;
-        for (const void* f : kernels) {
-            int nb = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, ls.block, lds) != hipSuccess || nb <= 0) return false;
-            least = std::min(least, nb);
-        }
+        for (const void* f : kernels) least = std::min(least, resident_blocks(f, ls.block, lds));
+        if (least <= 0) return false;
         blocks = std::min(ls.trace_blocks, std::max(1, num_cus * least));
         return true;
     };

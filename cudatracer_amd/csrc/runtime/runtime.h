@@ -90,13 +90,14 @@ int hip_fail(ct_ctx* c, hipError_t e, const char* what);
 // Results to the caller's memory.  To memory the runtime knows (pinned by the
 // caller) by its copy: 33 MB (a 1080p float image, or a 4K byte image) 0.59 ms.
 // To pageable memory through pinned slots: while the caller's thread copies one
-// slot to its place, the device fills the next ones.  The runtime's own copy
-// does the two in turn: 33 MB 1.85 ms, the thread's memcpy 0.8-0.9 ms of it.  Textured 1080p frame with its float image 5.83 to 5.15
-// ms, 4K frame with its byte image 7.61 to 6.95 ms.  For one thread at a time.
-// Pinning takes 0.4 ms a MB, so the slots are small (four of 2 MB served no better)
-// and made at the second result: a context's first goes by the runtime's copy,
-// as do results of up to 1 MB in device memory, where there is little to overlap,
-// and all of them where no slots can be had.
+// slot to its place, the device fills the next ones.  The runtime's own copy does
+// the two in turn: 33 MB 1.85 ms, the thread's memcpy 0.8-0.9 ms of it.  Textured
+// 1080p frame with its float image 5.83 to 5.15 ms, 4K frame with its byte image
+// 7.61 to 6.95 ms.  For one thread at a time.  Pinning takes 0.4 ms a MB, so the
+// slots are small (four of 2 MB served no better) and made at the second result: a
+// context's first goes by the runtime's copy, as do results of up to 1 MB in
+// device memory, where there is little to overlap, and all of them where no
+// slots can be had.
 class ReadBack {
   public:
     // bytes of results to dst, in parts; put(dev, offset, n) enqueues on

@@ -20,16 +20,16 @@ using ctd::ViewDesc;
 
 namespace ctr {
 
+// A device error that has been reported is taken from the runtime, which would
+// hand it to the next launch's check as well: a refused allocation failed the
+// next call, or the host path taken in its place.
 int fail(ct_ctx* c, int code, const std::string& msg) {
+    if (code == CT_ERR_DEVICE) (void)hipGetLastError();
     if (c) c->err = msg;
     return code;
 }
 
-// An error that has been reported is taken from the runtime, which would hand it
-// to the next launch's check as well: a refused allocation failed the next
-// call, or the host path taken in its place.
 int hip_fail(ct_ctx* c, hipError_t e, const char* what) {
-    (void)hipGetLastError();
     std::ostringstream os;
     os << what << ": " << hipGetErrorString(e);
     return fail(c, CT_ERR_DEVICE, os.str());

@@ -83,6 +83,25 @@ def refused_allocation(hip, ct):
     ctx.trace_frame(scene.camera(64, 64), scene.frame_opts()[0], stats=False)
 
 
+@case
+def failures_reported_once(hip, ct):
+    """So it is with other calls that fail: in a frame's first buffers, and where
+    a launch shape is looked for (a fixed one is taken then)."""
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    frame = scene.camera(64, 64), scene.frame_opts()[0]
+    hip.fail("hipOccupancyMaxActiveBlocksPerMultiprocessor", 1)
+    ctx = ct.Context(0)
+    ctx.upload(scene)
+    ctx.resize(64, 64)
+    hip.fail("hipMemsetAsync", 1)
+    try:
+        ctx.trace_frame(*frame, stats=False)
+        raise AssertionError("the path buffers were not cleared")
+    except ct.CTError as e:
+        assert e.code == ct.CT_ERR_DEVICE
+    ctx.trace_frame(*frame, stats=False)
+
+
 def _textured(ct, n, side):
     """A view of n separate triangles with one float texture of side^2 texels."""
     from conftest import ArrayView
