@@ -153,3 +153,13 @@ def _binary_chain(ct, orc, gpu_ctx, levels, n):
     opts.accel = ct.ACCEL_BVH2
     o, d = chain_rays(n, 4)
     _same(gpu_ctx, osc, o, d, np.full(n, 40.0, np.float32), opts, 0)
+
+
+@pytest.mark.parametrize("n", [2, 4095, 4096, 4097])
+def test_hits_in_one_copy(ct, orc, gpu_ctx, c1, n):
+    """Up to 4,096 host rays' distances and ids come in one copy."""
+    scene, arrays, osc = c1
+    gpu_ctx.upload(scene)
+    opts, _, _ = scene.frame_opts()
+    o, d = ray_set(scene, arrays, n, 21)
+    _same(gpu_ctx, osc, o, d, np.full(n, 20.0, np.float32), opts, int(opts.accel == ct.ACCEL_BVH4))

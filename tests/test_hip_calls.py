@@ -277,6 +277,21 @@ def one_wait_a_result(hip, ct):
         assert hip.calls("hipStreamSynchronize") - before == 1
 
 
+@case
+def one_wait_for_a_few_rays(hip, ct):
+    scene = ct.HostScene.generate(ct.SCENE_C1, 7)
+    ctx = ct.Context(0)
+    ctx.upload(scene)
+    opts, _, _ = scene.frame_opts()
+    waits = []
+    for n in (4096, 1, 64, 4096):  # the first makes the path buffers
+        o, d = np.zeros((n, 3), np.float32), np.ones((n, 3), np.float32)
+        before = hip.calls("hipStreamSynchronize")
+        ctx.trace_rays(o, d, opts)
+        waits.append(hip.calls("hipStreamSynchronize") - before)
+    assert waits[1:] == [1, 1, 1], waits
+
+
 @pytest.mark.parametrize("name", list(CASES))
 def test_hip_calls(standin, name):
     r = subprocess.run([sys.executable, __file__, str(standin), name], capture_output=True, text=True, timeout=120)
