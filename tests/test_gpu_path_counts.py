@@ -1,6 +1,8 @@
 """Frames at the path counts where the frame loop changes: whole paths in one
 launch with eight lanes each (up to 40,960 paths on 256 CUs) or two (up to
-131,072), the queue pipeline above.  Each must equal the FP32 oracle bit for
+131,072), the queue pipeline above.  These frames ask for statistics, so they
+take the pipeline at every count (test_gpu_whole_paths.py holds the whole paths
+against them).  Each must equal the FP32 oracle bit for
 bit, ray counts included, on the trees whose traversal is exact; on the
 compact and the wide tree 99.9% of the pixels must equal the exact frame (t is
 equal there, ids on exact ties of t may differ)."""
